@@ -32,8 +32,10 @@ NODATA = 0.0      # cells outside the study area, in the mask and in the raster 
 TWO_PI_F = float(np.float32(6.2831853071795862))   # the estimator's constant is a float
 EPS_DEN = float(np.float32(1e-14))
 
-# candidate bandwidths of a search span these multiples of the rule of thumb
-SEARCH_LO, SEARCH_HI = 0.1, 10.0
+# candidate bandwidths of a whole search span these multiples of the rule of
+# thumb h; a golden-section step starts with two probes inside [h / 20, 2 h]
+WIDE = (0.1, 10.0)
+STEP = (0.6526, 1.3974)
 
 
 # ------------------------------------------------------------------ inputs --
@@ -116,9 +118,9 @@ def _rule(x, y, w):
     return np.sqrt(np.float32(float(np.sqrt(np.float32(2.0) / np.float32(3 * len(x)))) * d2))
 
 
-def _candidates(h0, k):
+def _candidates(h0, k, lo=WIDE[0], hi=WIDE[1]):
     t = np.arange(k) / max(k - 1, 1)
-    return (float(h0) * SEARCH_LO * (SEARCH_HI / SEARCH_LO) ** t).astype(np.float32)
+    return (float(h0) * lo * (hi / lo) ** t).astype(np.float32)
 
 
 def _bandwidths(case, x, y, w, seed):
@@ -177,10 +179,11 @@ def listed():
         _case("points", name="points_1m", n=1000000, ncols=8192, nrows=8192, points="thomas", parents=200,
               weights=True, mask="disk", holes=20),
         # the batched bandwidth search: 64 candidates
-        _case("search", name="search_64", n=200000, ncols=4096, nrows=4096, k=64, points="mixture"),
+        _case("search", name="search_64", n=200000, ncols=4096, nrows=4096, k=64, points="mixture", lo=WIDE[0],
+              hi=WIDE[1]),
         # one step of the golden-section optimiser: two candidates, called again and again
         _case("search", name="search_2", n=100000, ncols=2048, nrows=2048, k=2, points="thomas", parents=100,
-              mask="disk", holes=6),
+              mask="disk", holes=6, lo=STEP[0], hi=STEP[1]),
         # one probe of the (h, alpha) optimiser
         _case("adaptive", name="adaptive_2", n=100000, ncols=2048, nrows=2048, k=2, points="thomas", parents=100,
               weights=True, mask="disk", holes=6),
@@ -218,8 +221,10 @@ def draw(rng):
         side = _log_int(rng, 500, 8000)
         kw.update(n=_log_int(rng, 2000, 800000), ncols=side, nrows=max(200, int(side * rng.uniform(0.6, 1.0))))
     elif kind == "search":
-        k = rng.randrange(1, 49)
-        kw.update(n=_log_int(rng, 2000, 100000), ncols=_log_int(rng, 300, 3000), nrows=_log_int(rng, 300, 3000), k=k)
+        lo, hi = rng.choice([WIDE, STEP])
+        k = rng.randrange(1, 49) if hi > 2.0 else rng.randrange(1, 9)
+        kw.update(n=_log_int(rng, 2000, 100000), ncols=_log_int(rng, 300, 3000), nrows=_log_int(rng, 300, 3000), k=k,
+                  lo=lo, hi=hi)
     elif kind == "adaptive":
         kw.update(n=_log_int(rng, 2000, 150000), ncols=_log_int(rng, 300, 3000), nrows=_log_int(rng, 300, 3000),
                   k=rng.randrange(1, 5))
@@ -266,7 +271,7 @@ def prepare(case, seed):
         elif kind == "points":
             st["h0"] = float(_rule(x, y, w))
         elif kind == "search":
-            st["h"] = _candidates(_rule(x, y, w), case["k"])
+            st["h"] = _candidates(_rule(x, y, w), case["k"], case["lo"], case["hi"])
         elif kind == "adaptive":
             st["h"], st["alpha"] = _pairs(case, float(_rule(x, y, w)))
     return st
@@ -372,7 +377,7 @@ def work(case):
     if kind == "adaptive":
         return {"bytes": case["k"] * 12.0 * n + cells, "flops": case["k"] * (2.0 * pair + 2.0 * n * 40.0 * cols)}
     f = 0.0
-    for hk in _candidates(h, case["k"]).astype(float):
+    for hk in _candidates(h, case["k"], case["lo"], case["hi"]).astype(float):
         share = min(1.0, math.pi * (3.0 * hk) ** 2 / (cells * cs * cs))
         f += 10.0 * n * n * share + n * 40.0 * min(6.0 * hk / cs, case["ncols"])
     return {"bytes": 12.0 * n + cells + 8.0 * case["k"], "flops": float(f)}
@@ -663,7 +668,7 @@ def exact(case, seed):
     cx, cy = (_t(v) for v in _centres(case["ncols"], case["nrows"], 0.0, 0.0, cs))
     dist = _boundary_dist(x, y, m, cx, cy)
     if kind == "search":
-        return _loglik(x, y, wt, _candidates(h0, case["k"]), m, cx, cy, cs, dist, bud)
+        return _loglik(x, y, wt, _candidates(h0, case["k"], case["lo"], case["hi"]), m, cx, cy, cs, dist, bud)
     pairs = [(float(h0), -0.5)] if kind == "points" else list(zip(*(v.tolist() for v in _pairs(case, float(h0)))))
     lls = []
     for hp, alpha in pairs:
@@ -683,7 +688,8 @@ def _too_large(case):
     """Whether the pairs of the whole case are plainly beyond EXACT_PAIRS."""
     n, k = float(case["n"]), case.get("k", 1)
     if case["kind"] == "search":
-        h, wide = _candidates(_typical_h(case, case["n"]), k).astype(float), min(case["ncols"], case["nrows"])
+        h = _candidates(_typical_h(case, case["n"]), k, case["lo"], case["hi"]).astype(float)
+        wide = min(case["ncols"], case["nrows"])
         cells = np.minimum(6.0 * h / case["cs"], wide) ** 2
         share = np.minimum(1.0, math.pi * (3.0 * h) ** 2 / (case["ncols"] * case["nrows"] * case["cs"] ** 2))
         return bool((0.5 * n * cells + 2.0 * n * n * share).sum() > EXACT_PAIRS)
