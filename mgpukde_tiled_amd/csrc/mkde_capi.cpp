@@ -26,6 +26,7 @@
 #include <vector>
 
 #include "mkde.h"
+#include "mkde_copy.h"
 #include "mkde_device.h"
 
 namespace mkde_dev {
@@ -163,6 +164,7 @@ struct RunsHost {
 
 struct mkde_ctx {
     int device = 0;
+    bool shared_device = false;          // other contexts' kernels run beside this one's (job server)
     std::atomic<int64_t> dev_bytes{0};   // device memory held by the buffers below
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
@@ -319,8 +321,15 @@ extern "C" int mkde_ctx_create(int device, mkde_ctx **out)
         delete c;
         return fail(MKDE_E_HIP, "context set-up failed: %s", hipGetErrorString(e));
     }
+    mkde_copy::retain();
     *out = c;
     return MKDE_OK;
+}
+
+// The job server's contexts run side by side on one device (mkde_serve.cpp).
+extern "C" __attribute__((visibility("hidden"))) void mkde_internal_share_device(mkde_ctx *c)
+{
+    c->shared_device = true;
 }
 
 extern "C" int mkde_ctx_destroy(mkde_ctx *c)
@@ -335,6 +344,7 @@ extern "C" int mkde_ctx_destroy(mkde_ctx *c)
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
     t_acct = nullptr;
+    mkde_copy::release();
     return MKDE_OK;
 }
 
@@ -357,6 +367,7 @@ extern "C" int mkde_ctx_release(mkde_ctx *c)
     unsigned char *scr = c->scratch;
     std::vector<hipEvent_t> pool;
     pool.swap(c->ev_pool);
+    const bool shared = c->shared_device;
     const bool order_on = c->dt_order_on, graph_on = c->search_graph_on;
     const Tuning tune = c->tune;
     const int ppb = c->pts_per_bin;
@@ -370,6 +381,7 @@ extern "C" int mkde_ctx_release(mkde_ctx *c)
     c->ev1 = e1;
     c->scratch = scr;
     c->ev_pool.swap(pool);
+    c->shared_device = shared;
     c->dt_order_on = order_on;
     c->search_graph_on = graph_on;
     c->tune = tune;
@@ -386,20 +398,29 @@ extern "C" int mkde_synchronize(mkde_ctx *c)
     return MKDE_OK;
 }
 
-static int copy_h2d(mkde_ctx *c, void *dst, const void *src, size_t bytes)
+// Large copies take several lanes (mkde_copy.cpp), the others the stream.
+static int copy_host(mkde_ctx *c, void *dst, const void *src, size_t bytes, bool to_host)
 {
     if (bytes == 0) return MKDE_OK;
-    HIPCHK(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, c->stream));
+    bool done = false;
+    if (bytes >= (c->shared_device ? mkde_copy::SHARED_MIN_BYTES : mkde_copy::MIN_BYTES)) {
+        HIPCHK(hipStreamSynchronize(c->stream));
+        HIPCHK(mkde_copy::run(c->device, c->shared_device ? c->stream : nullptr, dst, src, bytes, to_host, &done));
+    }
+    if (done) return MKDE_OK;
+    HIPCHK(hipMemcpyAsync(dst, src, bytes, to_host ? hipMemcpyDeviceToHost : hipMemcpyHostToDevice, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
     return MKDE_OK;
 }
 
+static int copy_h2d(mkde_ctx *c, void *dst, const void *src, size_t bytes)
+{
+    return copy_host(c, dst, src, bytes, false);
+}
+
 static int copy_d2h(mkde_ctx *c, void *dst, const void *src, size_t bytes)
 {
-    if (bytes == 0) return MKDE_OK;
-    HIPCHK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
-    return MKDE_OK;
+    return copy_host(c, dst, src, bytes, true);
 }
 
 // ---------------------------------------------------------- point index --

@@ -40,6 +40,7 @@
 #include "mkde_device.h"
 
 extern "C" int mkde_internal_fail(int code, const char *msg);
+extern "C" void mkde_internal_share_device(mkde_ctx *c);
 namespace mkde_dev {
 Tuning default_tuning();
 }
@@ -219,6 +220,7 @@ static void worker(mkde_server *s, int i)
     Slot &me = s->slots[i];
     mkde_ctx *c = nullptr;
     const int st = mkde_ctx_create(s->device, &c);
+    if (st == MKDE_OK && s->slots.size() > 1) mkde_internal_share_device(c);
     {
         std::lock_guard<std::mutex> lk(s->mu);
         if (st != MKDE_OK && s->init_status == MKDE_OK) {
