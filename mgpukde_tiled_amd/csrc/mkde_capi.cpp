@@ -35,17 +35,18 @@ hipError_t prep_points(hipStream_t, int64_t, const int *, const float *, const f
 hipError_t bin_stats(hipStream_t, int, const int *, const PtRec *, BinInfo *, double *);
 int64_t raster_blocks(const GridDesc &, const Tiling &);
 hipError_t density_plan(hipStream_t, const GridDesc &, const float *, const PointIndex &, const Tiling &,
-                        const DensityWork &, const Tuning &);
-hipError_t density_items(hipStream_t, int, const DensityWork &, int, int4 *, int4 *, int *, const unsigned *);
+                        const WorkList &, const Tuning &, unsigned *);
+hipError_t work_items(hipStream_t, int, const WorkList &, int4 *, int4 *, int *);
 hipError_t density_tile(hipStream_t, const GridDesc &, const float *, float *, const PointIndex &,
                         unsigned long long *, const int *, const int4 *, const unsigned *, double *, int,
                         const Tiling &);
 hipError_t density_merge(hipStream_t, const GridDesc &, const Tiling &, const float *, int, const int4 *,
                          const double *, float *);
-hipError_t point_plan(hipStream_t, const PointIndex &, int, float, const double *, int, const DensityWork &,
-                      const Tuning &);
+SplitRule point_rule(int, const Tuning &, bool);
+hipError_t point_plan(hipStream_t, const PointIndex &, float, const double *, int, const SplitRule &,
+                      const WorkList &, unsigned *);
 hipError_t point_density(hipStream_t, const PointIndex &, int, float *, float, const int *, const int4 *,
-                         const unsigned *, double *, int);
+                         const unsigned *, double *, int, const unsigned *);
 hipError_t loo_multi(hipStream_t, const PointIndex &, const float *, const double *, const double *, int, float *,
                      const int *, const int4 *, const unsigned *, double *, int, const unsigned *);
 hipError_t point_merge(hipStream_t, int64_t, int, int, int, const int4 *, const double *, float *, const unsigned *);
@@ -170,6 +171,8 @@ struct mkde_ctx {
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     // the device's static scratch array (allocation-free entry point)
     unsigned char *scratch = nullptr;
+    // pinned words that kernels leave a work list's counts in
+    unsigned *host_words = nullptr;
     // events of a job's phase timers, created once and reused by every job
     std::vector<hipEvent_t> ev_pool;
     size_t ev_next = 0;
@@ -253,8 +256,7 @@ struct mkde_ctx {
     hipGraphExec_t s_exec = nullptr;
     std::vector<uint64_t> s_key;
     // work list of the point kernels (64-query waves, heavy ones split)
-    DevBuf<unsigned> pw_cost, pw_parts, pw_item0, pw_slot0, pw_sidx, pw_sidx2, pw_chunks, pw_counts, pw_hist;
-    DevBuf<unsigned long long> pw_total;
+    DevBuf<unsigned> pw_cost, pw_item0, pw_slot0, pw_sidx, pw_counts, pw_hist;
     DevBuf<int4> pw_items, pw_splits;
     DevBuf<int> pw_order;
     DevBuf<double> pw_partials;
@@ -265,9 +267,7 @@ struct mkde_ctx {
     // items visited heaviest first
     bool dt_order_on = true;
     int pts_per_bin = 64;   // target points per bin of the point index
-    DevBuf<unsigned> blk_cost, blk_parts, blk_item0, blk_slot0, blk_sidx, blk_sidx2, blk_chunks, blk_counts,
-        blk_hist;
-    DevBuf<unsigned long long> blk_total;
+    DevBuf<unsigned> blk_cost, blk_item0, blk_slot0, blk_sidx, blk_counts, blk_hist;
     DevBuf<int4> dt_items, dt_splits;
     DevBuf<int> dt_order;
     DevBuf<double> dt_partials;
@@ -317,6 +317,7 @@ extern "C" int mkde_ctx_create(int device, mkde_ctx **out)
     if (e == hipSuccess) e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking);
     if (e == hipSuccess) e = hipEventCreate(&c->ev0);
     if (e == hipSuccess) e = hipEventCreate(&c->ev1);
+    if (e == hipSuccess) e = hipHostMalloc((void **)&c->host_words, 64, hipHostMallocDefault);
     if (e != hipSuccess) {
         delete c;
         return fail(MKDE_E_HIP, "context set-up failed: %s", hipGetErrorString(e));
@@ -341,6 +342,7 @@ extern "C" int mkde_ctx_destroy(mkde_ctx *c)
     if (c->ev1) (void)hipEventDestroy(c->ev1);
     if (c->s_exec) (void)hipGraphExecDestroy(c->s_exec);
     for (hipEvent_t e : c->ev_pool) (void)hipEventDestroy(e);
+    if (c->host_words) (void)hipHostFree(c->host_words);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
     t_acct = nullptr;
@@ -365,6 +367,7 @@ extern "C" int mkde_ctx_release(mkde_ctx *c)
     hipStream_t s = c->stream;
     hipEvent_t e0 = c->ev0, e1 = c->ev1;
     unsigned char *scr = c->scratch;
+    unsigned *words = c->host_words;
     std::vector<hipEvent_t> pool;
     pool.swap(c->ev_pool);
     const bool shared = c->shared_device;
@@ -380,6 +383,7 @@ extern "C" int mkde_ctx_release(mkde_ctx *c)
     c->ev0 = e0;
     c->ev1 = e1;
     c->scratch = scr;
+    c->host_words = words;
     c->ev_pool.swap(pool);
     c->shared_device = shared;
     c->dt_order_on = order_on;
@@ -1016,41 +1020,59 @@ extern "C" int mkde_range_candidates(mkde_ctx *c, int64_t *offsets, int32_t *idx
 
 // ------------------------------------------------- densities at points --
 
-// Work list of the point kernels: plan on the device, read the three counts,
-// then items, heaviest-first order and partial slots (m values per query).
+// Work list of the point kernels.  Where the partial sums of the largest list
+// are small, every buffer is sized for it and the counts stay on the device
+// (n_items and n_split are grid bounds then); else the counts are read back.
 struct PointWork {
     const int *order = nullptr;
     const int4 *items = nullptr;
     int n_items = 0, n_split = 0;
+    const unsigned *n_items_dev = nullptr, *n_split_dev = nullptr;
 };
 
-static int plan_points(mkde_ctx *c, const PointIndex &I, int kind, float h_fixed, const double *thr_k, int K, int m,
+static const int64_t MKDE_POINT_DEV_PARTIALS = (int64_t)64 << 20;   // bytes of split-part sums
+
+static int point_list(mkde_ctx *c, int64_t nw, WorkList &W)
+{
+    CHK(c->pw_cost.ensure(nw));
+    CHK(c->pw_item0.ensure(nw));
+    CHK(c->pw_slot0.ensure(nw));
+    CHK(c->pw_sidx.ensure(nw));
+    CHK(c->pw_counts.ensure(4));
+    CHK(c->pw_hist.ensure(32));
+    W = WorkList{c->pw_cost.p, c->pw_item0.p, c->pw_slot0.p, c->pw_sidx.p, c->pw_counts.p, c->pw_hist.p};
+    return MKDE_OK;
+}
+
+// m values per query; thr_k non-null: the batched leave-one-out pass.
+static int plan_points(mkde_ctx *c, const PointIndex &I, int loo, float h_fixed, const double *thr_k, int K, int m,
                        PointWork &P)
 {
     const int64_t nw = (c->n + 63) / 64;
     if (nw == 0) return MKDE_OK;
-    CHK(c->pw_cost.ensure(nw));
-    CHK(c->pw_parts.ensure(nw));
-    CHK(c->pw_item0.ensure(nw));
-    CHK(c->pw_slot0.ensure(nw));
-    CHK(c->pw_sidx.ensure(nw));
-    CHK(c->pw_sidx2.ensure(nw));
-    CHK(c->pw_chunks.ensure((nw + 1023) / 1024));
-    CHK(c->pw_counts.ensure(3));
-    CHK(c->pw_hist.ensure(32));
-    CHK(c->pw_total.ensure(1));
-    DensityWork W{c->pw_cost.p,  c->pw_parts.p,  c->pw_item0.p, c->pw_slot0.p, c->pw_sidx.p,
-                  c->pw_sidx2.p, c->pw_chunks.p, c->pw_total.p, c->pw_counts.p, c->pw_hist.p};
-    HIPCHK(mkde_dev::point_plan(c->stream, I, kind, h_fixed, thr_k, K, W, c->tune));
-    unsigned cnt[3];
-    CHK(copy_d2h(c, cnt, c->pw_counts.p, sizeof cnt));
-    P.n_items = (int)cnt[0];
-    P.n_split = (int)cnt[2];
+    WorkList W;
+    CHK(point_list(c, nw, W));
+    const SplitRule rule = mkde_dev::point_rule(loo, c->tune, thr_k != nullptr);
+    int64_t items_max = 0, slots_max = 0;
+    point_work_bounds(c->n, rule, &items_max, &slots_max);
+    const bool dev = slots_max * 64 * m * (int64_t)sizeof(double) <= MKDE_POINT_DEV_PARTIALS;
+    HIPCHK(mkde_dev::point_plan(c->stream, I, h_fixed, thr_k, K, rule, W, dev ? nullptr : c->host_words));
+    if (dev) {
+        P.n_items = (int)items_max;
+        P.n_split = (int)std::min(slots_max / 2, nw);   // a split unit has two parts or more
+        P.n_items_dev = c->pw_counts.p;
+        P.n_split_dev = c->pw_counts.p + 2;
+    } else {
+        HIPCHK(hipStreamSynchronize(c->stream));
+        P.n_items = (int)c->host_words[0];
+        slots_max = c->host_words[1];
+        P.n_split = (int)c->host_words[2];
+    }
     CHK(c->pw_items.ensure(P.n_items));
     CHK(c->pw_order.ensure(P.n_items));
     CHK(c->pw_splits.ensure(P.n_split));
-    CHK(c->pw_partials.ensure((size_t)cnt[1] * 64 * m));
-    HIPCHK(mkde_dev::density_items(c->stream, (int)nw, W, P.n_items, c->pw_items.p, c->pw_splits.p, c->pw_order.p, nullptr));
+    CHK(c->pw_partials.ensure((size_t)slots_max * 64 * m));
+    HIPCHK(mkde_dev::work_items(c->stream, (int)nw, W, c->pw_items.p, c->pw_splits.p, c->pw_order.p));
     P.order = c->pw_order.p;
     P.items = c->pw_items.p;
     return MKDE_OK;
@@ -1062,10 +1084,11 @@ static int density_points_sorted(mkde_ctx *c, int loo, float *den_sorted)
     PointIndex I = index_of(c);
     HIPCHK(hipEventRecord(c->ev0, c->stream));
     PointWork P;
-    CHK(plan_points(c, I, 0, c->h_fixed, nullptr, 0, 1, P));
+    CHK(plan_points(c, I, loo, c->h_fixed, nullptr, 0, 1, P));
     HIPCHK(mkde_dev::point_density(c->stream, I, loo, den_sorted, c->h_fixed, P.order, P.items, c->pw_cost.p,
-                                   c->pw_partials.p, P.n_items));
-    HIPCHK(mkde_dev::point_merge(c->stream, c->n, 1, 1, P.n_split, c->pw_splits.p, c->pw_partials.p, den_sorted, nullptr));
+                                   c->pw_partials.p, P.n_items, P.n_items_dev));
+    HIPCHK(mkde_dev::point_merge(c->stream, c->n, 1, 1, P.n_split, c->pw_splits.p, c->pw_partials.p, den_sorted,
+                                 P.n_split_dev));
     HIPCHK(hipEventRecord(c->ev1, c->stream));
     return MKDE_OK;
 }
@@ -1120,20 +1143,26 @@ extern "C" int mkde_density_at_points_noalloc(mkde_ctx *c, int loo, float *den_d
     const int64_t n = c->n, nw = (n + 63) / 64;
     Carve cv(c->scratch, MKDE_SCRATCH_BYTES);
     float *den_s = cv.take<float>((size_t)n);
-    unsigned *cost = cv.take<unsigned>(nw), *parts = cv.take<unsigned>(nw), *item0 = cv.take<unsigned>(nw);
-    unsigned *slot0 = cv.take<unsigned>(nw), *sidx = cv.take<unsigned>(nw), *sidx2 = cv.take<unsigned>(nw);
-    unsigned *chunks = cv.take<unsigned>((nw + 1023) / 1024), *counts = cv.take<unsigned>(3);
+    unsigned *cost = cv.take<unsigned>(nw), *item0 = cv.take<unsigned>(nw), *slot0 = cv.take<unsigned>(nw);
+    unsigned *sidx = cv.take<unsigned>(nw);
+    // two words a wave and one per 1024 waves in reserve: the sizes that fit do
+    // not depend on how many scans the work list takes
+    (void)cv.take<unsigned>(nw);
+    (void)cv.take<unsigned>(nw);
+    (void)cv.take<unsigned>((nw + 1023) / 1024);
+    unsigned *counts = cv.take<unsigned>(4);
     unsigned *hist = cv.take<unsigned>(32);
-    unsigned long long *total = cv.take<unsigned long long>(1);
+    (void)cv.take<unsigned long long>(1);
     if (!cv.ok)
         return fail(MKDE_E_RANGE, "%lld points need %zu bytes of scratch, more than the %u available", (long long)n,
                     cv.used, MKDE_SCRATCH_BYTES);
     CHK(prep(c));
     PointIndex I = index_of(c);
-    DensityWork W{cost, parts, item0, slot0, sidx, sidx2, chunks, total, counts, hist};
-    HIPCHK(mkde_dev::point_plan(c->stream, I, 0, c->h_fixed, nullptr, 0, W, c->tune));
-    unsigned cnt[3];   // items, split slots, split waves
-    CHK(copy_d2h(c, cnt, counts, sizeof cnt));
+    const WorkList W{cost, item0, slot0, sidx, counts, hist};
+    HIPCHK(mkde_dev::point_plan(c->stream, I, c->h_fixed, nullptr, 0, mkde_dev::point_rule(loo ? 1 : 0, c->tune, false),
+                                W, c->host_words));
+    HIPCHK(hipStreamSynchronize(c->stream));
+    const unsigned cnt[3] = {c->host_words[0], c->host_words[1], c->host_words[2]};   // items, slots, split waves
     int4 *items = cv.take<int4>(cnt[0]);
     int *order = cv.take<int>(cnt[0]);
     int4 *splits = cv.take<int4>(cnt[2]);
@@ -1143,9 +1172,9 @@ extern "C" int mkde_density_at_points_noalloc(mkde_ctx *c, int loo, float *den_d
                     "the work list of %lld points (%u items, %u split parts) needs %zu bytes of scratch, more than "
                     "the %u available",
                     (long long)n, cnt[0], cnt[1], cv.used, MKDE_SCRATCH_BYTES);
-    HIPCHK(mkde_dev::density_items(c->stream, (int)nw, W, (int)cnt[0], items, splits, order, nullptr));
+    HIPCHK(mkde_dev::work_items(c->stream, (int)nw, W, items, splits, order));
     HIPCHK(mkde_dev::point_density(c->stream, I, loo ? 1 : 0, den_s, c->h_fixed, order, items, cost, partials,
-                                   (int)cnt[0]));
+                                   (int)cnt[0], nullptr));
     HIPCHK(mkde_dev::point_merge(c->stream, n, 1, 1, (int)cnt[2], splits, partials, den_s, nullptr));
     HIPCHK(mkde_dev::unsort_f32(c->stream, n, c->perm.p, den_s, den_dev));
     HIPCHK(hipStreamSynchronize(c->stream));
@@ -1204,12 +1233,11 @@ struct BandwidthGuard {
 static const int64_t MKDE_SEARCH_GRAPH_MAX_PARTIALS = (int64_t)1 << 30;   // bytes of split-part sums
 
 static int search_enqueue(mkde_ctx *c, int K, int ec_on, const PointIndex &I, int64_t items_max, int64_t nw,
-                          const std::vector<int> &wcols)
+                          const WorkList &W, const std::vector<int> &wcols)
 {
     const int64_t n = c->n;
     MaskRuns R{c->run_ptr.p, c->run_se.p};
-    DensityWork W{c->pw_cost.p,  c->pw_parts.p,  c->pw_item0.p, c->pw_slot0.p, c->pw_sidx.p,
-                  c->pw_sidx2.p, c->pw_chunks.p, c->pw_total.p, c->pw_counts.p, c->pw_hist.p};
+    const SplitRule rule = mkde_dev::point_rule(1, c->tune, true);
     if (!ec_on) HIPCHK(mkde_dev::fill_f32(c->stream, n, 1.0f, c->ewk.p));
     const int nb = (int)std::min<int64_t>(1024, (n + 255) / 256);
     for (int g0 = 0, gi = 0; g0 < K; g0 += MKDE_LM_K, ++gi) {
@@ -1229,9 +1257,8 @@ static int search_enqueue(mkde_ctx *c, int K, int ec_on, const PointIndex &I, in
                                         c->coefk.p + (MKDE_LM_K - kg) + j, MKDE_LM_K));
         }
         const double *a = c->s_a.p + (int64_t)gi * MKDE_LM_K, *t = c->s_t.p + (int64_t)gi * MKDE_LM_K;
-        HIPCHK(mkde_dev::point_plan(c->stream, I, 1, 0.0f, t, MKDE_LM_K, W, c->tune));
-        HIPCHK(mkde_dev::density_items(c->stream, (int)nw, W, (int)items_max, c->pw_items.p, c->pw_splits.p,
-                                       c->pw_order.p, c->pw_counts.p));
+        HIPCHK(mkde_dev::point_plan(c->stream, I, 0.0f, t, MKDE_LM_K, rule, W, nullptr));
+        HIPCHK(mkde_dev::work_items(c->stream, (int)nw, W, c->pw_items.p, c->pw_splits.p, c->pw_order.p));
         HIPCHK(mkde_dev::loo_multi(c->stream, I, c->coefk.p, a, t, kg, c->den1k.p, c->pw_order.p, c->pw_items.p,
                                    c->pw_cost.p, c->pw_partials.p, (int)items_max, c->pw_counts.p));
         HIPCHK(mkde_dev::point_merge(c->stream, n, MKDE_LM_K, kg, (int)nw, c->pw_splits.p, c->pw_partials.p,
@@ -1249,7 +1276,7 @@ static int loo_loglik_graph(mkde_ctx *c, int K, const std::vector<int> &ord, con
     *done = false;
     const int64_t n = c->n, nw = (n + 63) / 64;
     int64_t items_max = 0, slots_max = 0;
-    point_work_bounds(n, c->tune.loo_target, &items_max, &slots_max);
+    point_work_bounds(n, mkde_dev::point_rule(1, c->tune, true), &items_max, &slots_max);
     if (slots_max * 64 * MKDE_LM_K * (int64_t)sizeof(double) > MKDE_SEARCH_GRAPH_MAX_PARTIALS) return MKDE_OK;
     const int G = (K + MKDE_LM_K - 1) / MKDE_LM_K;
     // every buffer the graph touches, at its final size, before any capture
@@ -1265,16 +1292,8 @@ static int loo_loglik_graph(mkde_ctx *c, int K, const std::vector<int> &ord, con
     CHK(c->s_a.ensure((size_t)G * MKDE_LM_K));
     CHK(c->s_t.ensure((size_t)G * MKDE_LM_K));
     CHK(c->s_logl.ensure(K));
-    CHK(c->pw_cost.ensure(nw));
-    CHK(c->pw_parts.ensure(nw));
-    CHK(c->pw_item0.ensure(nw));
-    CHK(c->pw_slot0.ensure(nw));
-    CHK(c->pw_sidx.ensure(nw));
-    CHK(c->pw_sidx2.ensure(nw));
-    CHK(c->pw_chunks.ensure((nw + 1023) / 1024));
-    CHK(c->pw_counts.ensure(3));
-    CHK(c->pw_hist.ensure(32));
-    CHK(c->pw_total.ensure(1));
+    WorkList W;
+    CHK(point_list(c, nw, W));
     CHK(c->pw_items.ensure(items_max));
     CHK(c->pw_order.ensure(items_max));
     CHK(c->pw_splits.ensure(nw));
@@ -1321,11 +1340,10 @@ static int loo_loglik_graph(mkde_ctx *c, int K, const std::vector<int> &ord, con
                               (uint64_t)(uintptr_t)c->den1k.p, (uint64_t)(uintptr_t)c->s_h.p,
                               (uint64_t)(uintptr_t)c->s_a.p, (uint64_t)(uintptr_t)c->s_t.p,
                               (uint64_t)(uintptr_t)c->s_logl.p, (uint64_t)(uintptr_t)c->pw_cost.p,
-                              (uint64_t)(uintptr_t)c->pw_parts.p, (uint64_t)(uintptr_t)c->pw_item0.p,
+                              (uint64_t)(uintptr_t)c->pw_item0.p,
                               (uint64_t)(uintptr_t)c->pw_slot0.p, (uint64_t)(uintptr_t)c->pw_sidx.p,
-                              (uint64_t)(uintptr_t)c->pw_sidx2.p, (uint64_t)(uintptr_t)c->pw_chunks.p,
                               (uint64_t)(uintptr_t)c->pw_counts.p, (uint64_t)(uintptr_t)c->pw_hist.p,
-                              (uint64_t)(uintptr_t)c->pw_total.p, (uint64_t)(uintptr_t)c->pw_items.p,
+                              (uint64_t)(uintptr_t)c->pw_items.p,
                               (uint64_t)(uintptr_t)c->pw_order.p, (uint64_t)(uintptr_t)c->pw_splits.p,
                               (uint64_t)(uintptr_t)c->pw_partials.p, (uint64_t)(uintptr_t)c->partial.p,
                               (uint64_t)c->tune.ec_chunk, (uint64_t)c->tune.ec_wide_min, c->tune.loo_target};
@@ -1339,7 +1357,7 @@ static int loo_loglik_graph(mkde_ctx *c, int K, const std::vector<int> &ord, con
         c->s_key.clear();
         hipGraph_t graph = nullptr;
         HIPCHK(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-        const int st = search_enqueue(c, K, ec_on, I, items_max, nw, wcols);
+        const int st = search_enqueue(c, K, ec_on, I, items_max, nw, W, wcols);
         const hipError_t e = hipStreamEndCapture(c->stream, &graph);
         if (st != MKDE_OK) {
             if (graph) (void)hipGraphDestroy(graph);
@@ -1423,9 +1441,9 @@ extern "C" int mkde_loo_loglik(mkde_ctx *c, int K, const float *h_cand, int ec_o
         // the work estimate culls with the largest threshold (the top slot)
         CHK(plan_points(c, I, 1, 0.0f, c->tk.p, MKDE_LM_K, MKDE_LM_K, P));
         HIPCHK(mkde_dev::loo_multi(c->stream, I, c->coefk.p, c->ak.p, c->tk.p, kg, c->den1k.p, P.order, P.items,
-                                   c->pw_cost.p, c->pw_partials.p, P.n_items, nullptr));
+                                   c->pw_cost.p, c->pw_partials.p, P.n_items, P.n_items_dev));
         HIPCHK(mkde_dev::point_merge(c->stream, n, MKDE_LM_K, kg, P.n_split, c->pw_splits.p, c->pw_partials.p,
-                                     c->den1k.p, nullptr));
+                                     c->den1k.p, P.n_split_dev));
         HIPCHK(hipEventRecord(c->ev1, c->stream));
         CHK(sum_logs(c, c->den1k.p, kg, 1, c->dsum.p));
         std::vector<double> part(kg);
@@ -1669,28 +1687,22 @@ extern "C" int mkde_density_tile_resident(mkde_ctx *c)
     if (c->dt_order_on) {
         const int64_t nblk = mkde_dev::raster_blocks(c->tg, c->tl);
         CHK(c->blk_cost.ensure(nblk));
-        CHK(c->blk_parts.ensure(nblk));
         CHK(c->blk_item0.ensure(nblk));
         CHK(c->blk_slot0.ensure(nblk));
         CHK(c->blk_sidx.ensure(nblk));
-        CHK(c->blk_sidx2.ensure(nblk));
-        CHK(c->blk_chunks.ensure((nblk + 1023) / 1024));
-        CHK(c->blk_counts.ensure(3));
+        CHK(c->blk_counts.ensure(4));
         CHK(c->blk_hist.ensure(32));
-        CHK(c->blk_total.ensure(1));
-        DensityWork W{c->blk_cost.p, c->blk_parts.p,  c->blk_item0.p, c->blk_slot0.p, c->blk_sidx.p,
-                      c->blk_sidx2.p, c->blk_chunks.p, c->blk_total.p, c->blk_counts.p, c->blk_hist.p};
-        HIPCHK(mkde_dev::density_plan(c->stream, c->tg, tm, I, c->tl, W, c->tune));
-        unsigned cnt[3];
-        CHK(copy_d2h(c, cnt, c->blk_counts.p, sizeof cnt));
-        n_items = (int)cnt[0];
-        n_split = (int)cnt[2];
+        const WorkList W{c->blk_cost.p, c->blk_item0.p,  c->blk_slot0.p,
+                         c->blk_sidx.p, c->blk_counts.p, c->blk_hist.p};
+        HIPCHK(mkde_dev::density_plan(c->stream, c->tg, tm, I, c->tl, W, c->tune, c->host_words));
+        HIPCHK(hipStreamSynchronize(c->stream));
+        n_items = (int)c->host_words[0];
+        n_split = (int)c->host_words[2];
         CHK(c->dt_items.ensure(n_items));
         CHK(c->dt_order.ensure(n_items));
         CHK(c->dt_splits.ensure(n_split));
-        CHK(c->dt_partials.ensure((size_t)cnt[1] * MKDE_DT_CELLS));
-        HIPCHK(mkde_dev::density_items(c->stream, (int)nblk, W, n_items, c->dt_items.p, c->dt_splits.p,
-                                       c->dt_order.p, nullptr));
+        CHK(c->dt_partials.ensure((size_t)c->host_words[1] * MKDE_DT_CELLS));
+        HIPCHK(mkde_dev::work_items(c->stream, (int)nblk, W, c->dt_items.p, c->dt_splits.p, c->dt_order.p));
         order = c->dt_order.p;
     }
     HIPCHK(hipEventRecord(c->ev0, c->stream));

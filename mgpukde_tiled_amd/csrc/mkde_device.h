@@ -28,20 +28,43 @@ struct Tuning {
     unsigned long long dt_target;    // split target of the density-raster work list
 };
 
+// A work list cuts units (64-query waves, density blocks) whose cost exceeds a
+// threshold T into ceil(cost / T) parts.  T = max(ceil(total / target),
+// min(tmin, max(few_tmin, ceil(total / few)))): about `target` parts when there
+// is much work, none below tmin sources a part, but with little work in all
+// (few > 0) up to `few` smaller parts, down to few_tmin sources each, so that a
+// short list still fills the device.
+struct SplitRule {
+    unsigned tmin;
+    unsigned long long target;
+    unsigned few_tmin;
+    unsigned long long few;   // 0: no smaller parts
+};
+
 // Smallest split threshold of the point work lists (candidate sources per part).
-#define MKDE_PTS_TMIN 4096ull
+#define MKDE_PTS_TMIN 4096u
+// Leave-one-out lists: smaller parts while they are at most 4096 (a search on
+// 2,000 points is 32 waves: 0.90 ms for its pass uncut, 0.13 ms in parts of 256).
+#define MKDE_LOO_FEW_TMIN 256u
+#define MKDE_LOO_FEW 4096ull
 
 // Most items and split parts a point work list of nw 64-query waves can have:
-// each wave's cost is at most n sources, the threshold is T = max(tmin,
-// total / target), so split parts <= min(target, total / tmin) + the number
-// of split waves.
-inline void point_work_bounds(int64_t n, unsigned long long target, int64_t *items_max, int64_t *slots_max)
+// each wave's cost is at most n sources, so split parts <= min(target, total /
+// T) + the number of split waves.
+inline void point_work_bounds(int64_t n, const SplitRule &r, int64_t *items_max, int64_t *slots_max)
 {
     const int64_t nw = (n + 63) / 64;
     const double tot = (double)nw * (double)n;
-    const int64_t by_t = (int64_t)((tot + MKDE_PTS_TMIN - 1) / (double)MKDE_PTS_TMIN);
-    const int64_t parts = by_t < (int64_t)target ? by_t : (int64_t)target;
-    const int64_t split_waves = by_t < nw ? by_t : nw;
+    const int64_t by_t = (int64_t)((tot + r.tmin - 1) / (double)r.tmin);
+    int64_t parts = by_t < (int64_t)r.target ? by_t : (int64_t)r.target;
+    int64_t split_waves = by_t < nw ? by_t : nw;
+    if (r.few > 0) {
+        const int64_t by_f = (int64_t)((tot + r.few_tmin - 1) / (double)r.few_tmin);
+        const int64_t few = by_f < (int64_t)r.few ? by_f : (int64_t)r.few;
+        parts = parts > few ? parts : few;
+        const int64_t fw = few < nw ? few : nw;
+        split_waves = split_waves > fw ? split_waves : fw;
+    }
     *items_max = nw + parts + 1;
     *slots_max = parts + split_waves + 1;
 }
@@ -100,15 +123,13 @@ struct Tiling {
     double gt0, gt1, gt3, gt5;
 };
 
-// Device buffers of the density kernel's work list (per density block unless
-// noted): candidate counts, split parts, scans of parts / split parts / split
-// flags, scan scratch, the candidate total and the {items, slots, splits}
-// counts read back by the host.
-struct DensityWork {
-    unsigned *cost, *parts, *item0, *slot0, *sidx, *sidx2;
-    unsigned *chunks;              // (nblk + 1023) / 1024
-    unsigned long long *total;     // 1
-    unsigned *counts;              // 3
+// Device buffers of a work list (per unit unless noted): costs, the exclusive
+// scan of the parts, and for split units the first partial slot and the place
+// in the split list; the counts {items, slots, splits, T} and the places of the
+// 32 cost buckets in the visiting order.
+struct WorkList {
+    unsigned *cost, *item0, *slot0, *sidx;
+    unsigned *counts;              // 4
     unsigned *hist;                // 32
 };
 

@@ -857,18 +857,6 @@ __device__ __forceinline__ int cost_bucket(unsigned c)
     return c == 0 ? 31 : (__clz(c) < 31 ? __clz(c) : 30);
 }
 
-__global__ void k_bucket_scan(unsigned *hist)
-{
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        unsigned run = 0;
-        for (int k = 0; k < 32; ++k) {
-            unsigned c = hist[k];
-            hist[k] = run;
-            run += c;
-        }
-    }
-}
-
 // Sum of the K partials of each split block in part order (FP64), rounded
 // once to FP32; nodata cells keep the mask value.  splits[k] = {block, slot0, K}.
 __global__ __launch_bounds__(256) void k_density_merge(GridDesc g, Tiling tl, int nbx, const float *mask,
@@ -890,97 +878,168 @@ __global__ __launch_bounds__(256) void k_density_merge(GridDesc g, Tiling tl, in
     }
 }
 
-// ---- work list of the density kernel
+// ---- work lists
 //
-// cost[b] (candidates of block b) -> split threshold T = max(DT_TMIN,
-// ceil(total / DT_TARGET)), parts[b] = cost > T ? ceil(cost / T) : 1, exclusive
+// cost[b] of every unit (candidates of a density block or of a 64-query wave)
+// -> split threshold T, parts[b] = cost > T ? ceil(cost / T) : 1, exclusive
 // scans for item and slot offsets, items[], splits[], and a heaviest-first
-// order of the items by cost / parts.
+// order of the items by cost / parts.  Two launches after the costs: one
+// workgroup forms total, threshold, scans and the bucket sizes (k_work_scan),
+// then every unit writes its items and takes their places in the order
+// (k_work_items).  With each of those in a launch of its own a list took 16
+// launches, ~70 us of a small job; one workgroup needs 4 us at 1,000 units and
+// 25 us at 16,384.
 #define DT_TMIN 2048u
 #define DT_TARGET 4096ull
 
-__global__ void k_cost_total(int n, const unsigned *cost, unsigned long long *total)
+__device__ __forceinline__ unsigned split_threshold(unsigned long long total, const SplitRule &r)
 {
-    __shared__ unsigned long long s_w[4];
-    unsigned long long acc = 0;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) acc += cost[i];
-    for (int d = 32; d >= 1; d >>= 1) acc += __shfl_xor(acc, d, WAVE);
-    if ((threadIdx.x & 63) == 0) s_w[threadIdx.x >> 6] = acc;
-    __syncthreads();
-    if (threadIdx.x == 0) atomicAdd(total, s_w[0] + s_w[1] + s_w[2] + s_w[3]);
-}
-
-__device__ __forceinline__ unsigned split_threshold(unsigned long long total, unsigned tmin, unsigned long long target)
-{
-    const unsigned long long t = (total + target - 1) / target;
-    return t > tmin ? (unsigned)(t < 0xffffffffull ? t : 0xffffffffull) : tmin;
-}
-
-// Split parts of each unit: T = max(tmin, ceil(total / target)), parts =
-// cost > T ? ceil(cost / T) : 1.
-__global__ void k_parts(int n, const unsigned *cost, const unsigned long long *total, unsigned tmin,
-                        unsigned long long target, unsigned *parts, unsigned *sparts, unsigned *sflag)
-{
-    const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= n) return;
-    const unsigned T = split_threshold(*total, tmin, target);
-    const unsigned c = cost[b];
-    const unsigned k = c > T ? (unsigned)(((unsigned long long)c + T - 1) / T) : 1u;
-    parts[b] = k;
-    sparts[b] = k > 1 ? k : 0u;
-    sflag[b] = k > 1 ? 1u : 0u;
-}
-
-__global__ void k_items_fill(int n, const unsigned *parts, const unsigned *item0, const unsigned *slot0,
-                             const unsigned *sidx, int4 *items, int4 *splits)
-{
-    const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= n) return;
-    const int k = (int)parts[b];
-    const int i0 = (int)item0[b];
-    for (int j = 0; j < k; ++j) items[i0 + j] = make_int4(b, j, k, k > 1 ? (int)slot0[b] + j : -1);
-    if (k > 1) splits[sidx[b]] = make_int4(b, (int)slot0[b], k, 0);
-}
-
-// Heaviest-first order of the items: bucket counts and slots are reserved
-// once per workgroup (LDS counters, one global atomic per bucket), so the
-// few large buckets do not serialise every item on one address.
-__global__ __launch_bounds__(256) void k_item_hist(int n, const unsigned *n_dev, const int4 *items, const unsigned *cost,
-                                                   unsigned *hist)
-{
-    if (n_dev) n = (int)*n_dev;   // the item count on the device (grid sized for the most items)
-    __shared__ unsigned s_h[32];
-    if (threadIdx.x < 32) s_h[threadIdx.x] = 0;
-    __syncthreads();
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) {
-        const int4 it = items[i];
-        atomicAdd(&s_h[cost_bucket(cost[it.x] / (unsigned)it.z)], 1u);
+    const unsigned long long t = (total + r.target - 1) / r.target;
+    unsigned low = r.tmin;
+    if (r.few > 0) {
+        const unsigned long long f = (total + r.few - 1) / r.few;
+        if (f < low) low = f > r.few_tmin ? (unsigned)f : r.few_tmin;
     }
-    __syncthreads();
-    if (threadIdx.x < 32 && s_h[threadIdx.x]) atomicAdd(&hist[threadIdx.x], s_h[threadIdx.x]);
+    return t > low ? (unsigned)(t < 0xffffffffull ? t : 0xffffffffull) : low;
 }
 
-__global__ __launch_bounds__(256) void k_item_order(int n, const unsigned *n_dev, const int4 *items, const unsigned *cost,
-                                                    unsigned *offs,
-                                                    int *order)
+__device__ __forceinline__ unsigned split_parts(unsigned c, unsigned T)
 {
-    if (n_dev) n = (int)*n_dev;
+    return c > T ? (unsigned)(((unsigned long long)c + T - 1) / T) : 1u;
+}
+
+__device__ __forceinline__ unsigned wave_incl_scan(unsigned v, int lane)
+{
+    for (int d = 1; d < WAVE; d <<= 1) {
+        const unsigned o = __shfl_up(v, d, WAVE);
+        if (lane >= d) v += o;
+    }
+    return v;
+}
+
+// One workgroup of 1024 threads, four units per thread and step.  host
+// (nullable, pinned): also receives the counts.
+__global__ __launch_bounds__(1024) void k_work_scan(int n, SplitRule rule, WorkList W, unsigned *host)
+{
+    __shared__ unsigned long long s_t[16];
+    __shared__ unsigned s_w[16][3];
+    __shared__ unsigned s_h[32];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    unsigned long long acc = 0;
+    for (int i = tid; i < n; i += 1024) acc += W.cost[i];
+    for (int d = 32; d >= 1; d >>= 1) acc += __shfl_xor(acc, d, WAVE);
+    if (lane == 0) s_t[wave] = acc;
+    if (tid < 32) s_h[tid] = 0;
+    __syncthreads();
+    unsigned long long total = 0;
+    for (int w = 0; w < 16; ++w) total += s_t[w];
+    const unsigned T = split_threshold(total, rule);
+
+    unsigned run_i = 0, run_p = 0, run_s = 0;   // items, slots, splits before this step
+    for (int base = 0; base < n; base += 4096) {
+        const int b0 = base + 4 * tid;
+        unsigned k[4], c[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            c[j] = b0 + j < n ? W.cost[b0 + j] : 0u;
+            k[j] = b0 + j < n ? split_parts(c[j], T) : 0u;
+        }
+        unsigned ni = 0, np = 0, ns = 0;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            ni += k[j];
+            np += k[j] > 1 ? k[j] : 0u;
+            ns += k[j] > 1 ? 1u : 0u;
+        }
+        const unsigned ii = wave_incl_scan(ni, lane), ip = wave_incl_scan(np, lane), is = wave_incl_scan(ns, lane);
+        if (lane == WAVE - 1) {
+            s_w[wave][0] = ii;
+            s_w[wave][1] = ip;
+            s_w[wave][2] = is;
+        }
+        __syncthreads();
+        unsigned oi = run_i + ii - ni, op = run_p + ip - np, os = run_s + is - ns;
+        for (int w = 0; w < 16; ++w) {
+            const unsigned a0 = s_w[w][0], a1 = s_w[w][1], a2 = s_w[w][2];
+            if (w < wave) {
+                oi += a0;
+                op += a1;
+                os += a2;
+            }
+            run_i += a0;
+            run_p += a1;
+            run_s += a2;
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            if (b0 + j >= n) break;
+            W.item0[b0 + j] = oi;
+            oi += k[j];
+            if (k[j] > 1) {
+                W.slot0[b0 + j] = op;
+                W.sidx[b0 + j] = os++;
+                op += k[j];
+            }
+        }
+        // bucket sizes: the lanes of a wave share few buckets, so each is added
+        // once per wave
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int bk = k[j] ? cost_bucket(c[j] / k[j]) : -1;
+            uint64_t todo = __ballot(bk >= 0);
+            while (todo) {
+                const int b = __builtin_amdgcn_readlane(bk, __builtin_ctzll(todo));
+                const uint64_t same = __ballot(bk == b);
+                unsigned v = bk == b ? k[j] : 0u;
+                for (int d = 32; d >= 1; d >>= 1) v += __shfl_xor(v, d, WAVE);
+                if (lane == 0) atomicAdd(&s_h[b], v);
+                todo &= ~same;
+            }
+        }
+        __syncthreads();
+    }
+    if (tid == 0) {
+        const unsigned out[4] = {run_i, run_p, run_s, T};
+        for (int j = 0; j < 4; ++j) {
+            W.counts[j] = out[j];
+            if (host) host[j] = out[j];
+        }
+        unsigned run = 0;
+        for (int b = 0; b < 32; ++b) {
+            W.hist[b] = run;
+            run += s_h[b];
+        }
+    }
+}
+
+// Items, split list and visiting order.  Places in a bucket are reserved once
+// per workgroup (LDS counters, one global atomic per bucket), so the few large
+// buckets do not serialise every item on one address.
+__global__ __launch_bounds__(256) void k_work_items(int n, WorkList W, int4 *items, int4 *splits, int *order)
+{
     __shared__ unsigned s_h[32], s_base[32];
     if (threadIdx.x < 32) s_h[threadIdx.x] = 0;
     __syncthreads();
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    const int b = blockIdx.x * blockDim.x + threadIdx.x;
     int bk = 0;
-    unsigned r = 0;
-    if (i < n) {
-        const int4 it = items[i];
-        bk = cost_bucket(cost[it.x] / (unsigned)it.z);
-        r = atomicAdd(&s_h[bk], 1u);
+    unsigned k = 0, r = 0, i0 = 0;
+    if (b < n) {
+        const unsigned c = W.cost[b];
+        k = split_parts(c, W.counts[3]);
+        i0 = W.item0[b];
+        bk = cost_bucket(c / k);
+        r = atomicAdd(&s_h[bk], k);
     }
     __syncthreads();
-    if (threadIdx.x < 32 && s_h[threadIdx.x]) s_base[threadIdx.x] = atomicAdd(&offs[threadIdx.x], s_h[threadIdx.x]);
+    if (threadIdx.x < 32 && s_h[threadIdx.x]) s_base[threadIdx.x] = atomicAdd(&W.hist[threadIdx.x], s_h[threadIdx.x]);
     __syncthreads();
-    if (i < n) order[s_base[bk] + r] = i;
+    if (b >= n) return;
+    const int slot0 = k > 1 ? (int)W.slot0[b] : -1;
+    for (unsigned j = 0; j < k; ++j) {
+        items[i0 + j] = make_int4(b, (int)j, (int)k, k > 1 ? slot0 + (int)j : -1);
+        order[s_base[bk] + r + j] = (int)(i0 + j);
+    }
+    if (k > 1) splits[W.sidx[b]] = make_int4(b, slot0, (int)k, 0);
 }
 
 // ---- exclusive scan of unsigned values (1024 per workgroup, two levels)
@@ -1072,6 +1131,7 @@ struct PtsArgs {
     const unsigned *cost;
     double *partials;            // 64 per slot
     int n_items;
+    const unsigned *n_items_dev;   // non-null: the item count on the device (n_items: grid bound)
 };
 
 #define PD_BAND (1.0 / 1048576.0)
@@ -1146,7 +1206,8 @@ __global__ __launch_bounds__(256) void k_point_density_w(PtsArgs A)
     // the wave index and the work item are wave-uniform: made explicit so the
     // source records below are read with scalar loads
     const int64_t g = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    if (g >= (A.order ? (int64_t)A.n_items : (I.n + 63) / 64)) return;   // whole wave
+    const int64_t units = A.n_items_dev ? (int64_t)*A.n_items_dev : A.order ? (int64_t)A.n_items : (I.n + 63) / 64;
+    if (g >= units) return;   // whole wave
     const int4 item = uniform_item(A.order ? A.items[A.order[g]] : make_int4((int)g, 0, 1, -1));
     int win0 = 0, win1 = INT_MAX;   // candidate counts are below 2^31
     if (item.z > 1) {
@@ -2604,38 +2665,24 @@ static void scan_u32(hipStream_t s, int n, const unsigned *in, unsigned *out, un
     hipLaunchKernelGGL(k_scan_add, dim3(nblk_(n)), dim3(256), 0, s, n, out, chunks);
 }
 
-// Costs, split parts and the three scans; W.counts receives {items, slots, splits}.
+// Costs and scans of the density work list; W.counts and, when given, the
+// pinned host words receive {items, slots, splits, T}.
 hipError_t density_plan(hipStream_t s, const GridDesc &g, const float *mask, const PointIndex &idx, const Tiling &tl,
-                        const DensityWork &W, const Tuning &T)
+                        const WorkList &W, const Tuning &T, unsigned *host)
 {
     const int nbx = (int)((g.ncols + MKDE_DT_BW - 1) / MKDE_DT_BW);
     const int nblk = (int)raster_blocks(g, tl);
     hipLaunchKernelGGL(k_block_cost, dim3((unsigned)nblk), dim3(256), 0, s, g, mask, idx, nbx, tl, W.cost);
-    hipLaunchKernelGGL(k_fill_f32, dim3(1), dim3(64), 0, s, (int64_t)2, 0.0f, (float *)W.total);
-    const unsigned nred = (unsigned)std::min<int64_t>(1024, ((int64_t)nblk + 255) / 256);
-    hipLaunchKernelGGL(k_cost_total, dim3(nred), dim3(256), 0, s, nblk, W.cost, W.total);
-    hipLaunchKernelGGL(k_parts, dim3(nblk_(nblk)), dim3(256), 0, s, nblk, W.cost, W.total, DT_TMIN, T.dt_target, W.parts,
-                       W.item0, W.sidx);
-    // in place is not allowed: parts -> item0 scan reads parts; sparts / sflag
-    // were written to item0 / sidx and are scanned into slot0 / sidx2 below
-    scan_u32(s, nblk, W.item0, W.slot0, W.chunks, W.counts + 1);
-    scan_u32(s, nblk, W.sidx, W.sidx2, W.chunks, W.counts + 2);
-    scan_u32(s, nblk, W.parts, W.item0, W.chunks, W.counts + 0);
+    const SplitRule rule{DT_TMIN, T.dt_target, 0u, 0ull};
+    hipLaunchKernelGGL(k_work_scan, dim3(1), dim3(1024), 0, s, nblk, rule, W, host);
     return hipGetLastError();
 }
 
-// n_dev non-null: the item count is read on the device (W.counts[0]) and
-// n_items is only the grid bound (the most items the work list can have).
-hipError_t density_items(hipStream_t s, int nblk, const DensityWork &W, int n_items, int4 *items, int4 *splits,
-                         int *order, const unsigned *n_dev)
+// Items, splits and order of n units after their plan; the buffers hold the
+// planned counts (or the bounds of point_work_bounds).
+hipError_t work_items(hipStream_t s, int n, const WorkList &W, int4 *items, int4 *splits, int *order)
 {
-    hipLaunchKernelGGL(k_items_fill, dim3(nblk_(nblk)), dim3(256), 0, s, nblk, W.parts, W.item0, W.slot0, W.sidx2,
-                       items, splits);
-    hipLaunchKernelGGL(k_fill_f32, dim3(1), dim3(64), 0, s, (int64_t)32, 0.0f, (float *)W.hist);
-    hipLaunchKernelGGL(k_item_hist, dim3(nblk_(n_items)), dim3(256), 0, s, n_items, n_dev, items, W.cost, W.hist);
-    hipLaunchKernelGGL(k_bucket_scan, dim3(1), dim3(64), 0, s, W.hist);
-    hipLaunchKernelGGL(k_item_order, dim3(nblk_(n_items)), dim3(256), 0, s, n_items, n_dev, items, W.cost, W.hist,
-                       order);
+    hipLaunchKernelGGL(k_work_items, dim3(nblk_(n)), dim3(256), 0, s, n, W, items, splits, order);
     return hipGetLastError();
 }
 
@@ -2662,39 +2709,40 @@ hipError_t density_merge(hipStream_t s, const GridDesc &g, const Tiling &tl, con
     return hipGetLastError();
 }
 
-// Work list of the point kernels (64-query waves): costs, split parts (T =
-// max(tmin, total / target)) and scans; W.counts = {items, slots, splits}.
-// kind 0: density at points (h_fixed > 0: one bandwidth), 1: batched
-// leave-one-out with thresholds thr_k[0..K-1] ascending.
-hipError_t point_plan(hipStream_t s, const PointIndex &idx, int kind, float h_fixed, const double *thr_k, int K,
-                      const DensityWork &W, const Tuning &T)
+// Split rule of the point work lists.  kind 0: density at points, 1: the
+// leave-one-out sums (density at points without the query, or batched).
+SplitRule point_rule(int kind, const Tuning &T, bool batched)
+{
+    SplitRule r{MKDE_PTS_TMIN, batched ? T.loo_target : T.pts_target, 0u, 0ull};
+    if (kind == 1) {
+        r.few_tmin = MKDE_LOO_FEW_TMIN;
+        r.few = MKDE_LOO_FEW;
+    }
+    return r;
+}
+
+// Work list of the point kernels (64-query waves): costs and scans; W.counts
+// and, when given, the pinned host words receive {items, slots, splits, T}.
+// thr_k non-null: batched leave-one-out with thresholds thr_k[0..K-1]
+// ascending, else density at points (h_fixed > 0: one bandwidth).
+hipError_t point_plan(hipStream_t s, const PointIndex &idx, float h_fixed, const double *thr_k, int K,
+                      const SplitRule &rule, const WorkList &W, unsigned *host)
 {
     const int nw = (int)((idx.n + 63) / 64);
-    double lim_fixed = 0.0;
-    const double *lim_dev = nullptr;
-    if (kind == 1) {
-        lim_dev = thr_k + (K - 1);
-    } else if (h_fixed > 0.0f) {
-        lim_fixed = 9.0 * (double)(float)(h_fixed * h_fixed);
-    }
+    const double *lim_dev = thr_k ? thr_k + (K - 1) : nullptr;
+    const double lim_fixed = !thr_k && h_fixed > 0.0f ? 9.0 * (double)(float)(h_fixed * h_fixed) : 0.0;
     hipLaunchKernelGGL(k_wave_cost, dim3((unsigned)((nw + 3) / 4)), dim3(256), 0, s, idx, lim_fixed, lim_dev, W.cost);
-    hipLaunchKernelGGL(k_fill_f32, dim3(1), dim3(64), 0, s, (int64_t)2, 0.0f, (float *)W.total);
-    const unsigned nred = (unsigned)std::min<int64_t>(1024, ((int64_t)nw + 255) / 256);
-    hipLaunchKernelGGL(k_cost_total, dim3(nred), dim3(256), 0, s, nw, W.cost, W.total);
-    const unsigned tmin = (unsigned)MKDE_PTS_TMIN;
-    const unsigned long long target = kind == 1 ? T.loo_target : T.pts_target;
-    hipLaunchKernelGGL(k_parts, dim3(nblk_(nw)), dim3(256), 0, s, nw, W.cost, W.total, tmin, target, W.parts,
-                       W.item0, W.sidx);
-    scan_u32(s, nw, W.item0, W.slot0, W.chunks, W.counts + 1);
-    scan_u32(s, nw, W.sidx, W.sidx2, W.chunks, W.counts + 2);
-    scan_u32(s, nw, W.parts, W.item0, W.chunks, W.counts + 0);
+    hipLaunchKernelGGL(k_work_scan, dim3(1), dim3(1024), 0, s, nw, rule, W, host);
     return hipGetLastError();
 }
 
+// n_items_dev non-null (here and in loo_multi): the item count is read on the
+// device and n_items is only the grid bound.
 hipError_t point_density(hipStream_t s, const PointIndex &idx, int loo, float *den_sorted, float h_fixed,
-                         const int *order, const int4 *items, const unsigned *cost, double *partials, int n_items)
+                         const int *order, const int4 *items, const unsigned *cost, double *partials, int n_items,
+                         const unsigned *n_items_dev)
 {
-    PtsArgs A{idx, den_sorted, loo, 0.0, 0.0, order, items, cost, partials, n_items};
+    PtsArgs A{idx, den_sorted, loo, 0.0, 0.0, order, items, cost, partials, n_items, n_items_dev};
     if (idx.n <= 0) return hipSuccess;
     const int64_t units = order ? n_items : (idx.n + 63) / 64;
     const unsigned grid = (unsigned)((units + 3) / 4);
@@ -2711,8 +2759,6 @@ hipError_t point_density(hipStream_t s, const PointIndex &idx, int loo, float *d
     return hipGetLastError();
 }
 
-// n_items_dev non-null: the item count is read on the device and n_items is
-// only the grid bound.
 hipError_t loo_multi(hipStream_t s, const PointIndex &idx, const float *coefk, const double *a_k,
                      const double *thr_k, int K, float *den1, const int *order, const int4 *items,
                      const unsigned *cost, double *partials, int n_items,
