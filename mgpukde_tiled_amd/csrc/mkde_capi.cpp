@@ -407,7 +407,10 @@ static int copy_host(mkde_ctx *c, void *dst, const void *src, size_t bytes, bool
 {
     if (bytes == 0) return MKDE_OK;
     bool done = false;
-    if (bytes >= (c->shared_device ? mkde_copy::SHARED_MIN_BYTES : mkde_copy::MIN_BYTES)) {
+    const size_t least = c->shared_device ? mkde_copy::MIN_SHARED
+                         : to_host        ? mkde_copy::MIN_TO_HOST
+                                          : mkde_copy::MIN_TO_DEVICE;
+    if (bytes >= least) {
         HIPCHK(hipStreamSynchronize(c->stream));
         HIPCHK(mkde_copy::run(c->device, c->shared_device ? c->stream : nullptr, dst, src, bytes, to_host, &done));
     }

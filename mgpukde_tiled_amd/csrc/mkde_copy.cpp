@@ -14,7 +14,7 @@
 // the lanes' streams would share the few hardware queues with them and wait
 // behind them (a burst of 16 jobs: 14.9 ms against 13.6 ms): there the transfers
 // go through the context's own stream (the same raster call: 11.3 ms), and only
-// for copies of SHARED_MIN_BYTES and more.
+// for copies of MIN_SHARED and more.
 //
 // Lanes belong to the process: at most MAX_LANES exist, a copy borrows the free
 // ones it can use and gives them back, and all are freed when the last context
