@@ -61,7 +61,10 @@ hipError_t runs_count(hipStream_t, const GridDesc &, const uint8_t *, unsigned *
 hipError_t runs_fill(hipStream_t, const GridDesc &, const uint8_t *, const unsigned *, int2 *);
 hipError_t boundary(hipStream_t, const GridDesc &, const uint8_t *, uint8_t *, float2 *, unsigned long long *);
 hipError_t dist_boundary(hipStream_t, int64_t, const float *, const float *, const float2 *, int64_t, double *);
-hipError_t bt_build(hipStream_t, const GridDesc &, const uint8_t *, uint4 *, float4 *, const BndTree &);
+int64_t bt_level_size(const BndTree &, int);
+hipError_t boundary_leaf(hipStream_t, const GridDesc &, const uint8_t *, uint8_t *, const BndTree &, uint4 *, float4 *,
+                         unsigned long long *);
+hipError_t bt_build(hipStream_t, const BndTree &, float4 *);
 hipError_t dist_tree(hipStream_t, int64_t, const float *, const float *, const int *, const GridDesc &,
                      const BndTree &, double *);
 hipError_t ec_active(hipStream_t, int64_t, const GridDesc &, const float *, const float *, const double *,
@@ -223,7 +226,8 @@ struct mkde_ctx {
     bool blist_on = false;               // boundary centre list built (brute-force distances)
     bool bflags_ok = false;    // boundary flags / list enqueued for the current mask
     int64_t nboundary = -1;    // boundary cell count once read back
-    // boundary hierarchy (nearest-boundary search)
+    // boundary hierarchy (nearest-boundary search): leaves with bflags_ok, all
+    // levels with bt_ok
     DevBuf<uint4> bt_bits;
     DevBuf<float4> bt_box;
     BndTree bt{};
@@ -755,25 +759,56 @@ static bool btree_fits(const mkde_ctx *c)
     return nx <= 16384 && ny <= 16384;
 }
 
+// Shape of the hierarchy over the EC mask: 16x16-cell leaves up to one root.
+static int shape_btree(mkde_ctx *c)
+{
+    BndTree &T = c->bt;
+    T = BndTree{};
+    int nx = (int)((c->mg.ncols + MKDE_BT_S - 1) / MKDE_BT_S), ny = (int)((c->mg.nrows + MKDE_BT_S - 1) / MKDE_BT_S);
+    for (;;) {
+        T.nx[T.nlev] = nx;
+        T.ny[T.nlev] = ny;
+        T.nlev++;
+        if (nx == 1 && ny == 1) break;
+        nx = (nx + 1) / 2;
+        ny = (ny + 1) / 2;
+    }
+    T.nx[T.nlev] = T.ny[T.nlev] = 1;
+    int64_t total = 0;
+    for (int l = 0; l < T.nlev; ++l) {
+        T.off[l] = total;
+        total += mkde_dev::bt_level_size(T, l);
+    }
+    CHK(c->bt_bits.ensure(2 * (size_t)mkde_dev::bt_level_size(T, 0)));
+    CHK(c->bt_box.ensure(total));
+    T.bits = c->bt_bits.p;
+    T.box = c->bt_box.p;
+    return MKDE_OK;
+}
+
 static int ensure_boundary(mkde_ctx *c)
 {
     CHK(need_mask(c));
     if (c->bflags_ok) return MKDE_OK;
     const int64_t nc = c->mg.ncols * c->mg.nrows;
     // the list of boundary centres only feeds the brute-force distances
-    // (rasters too large for the hierarchy); otherwise only the count is
-    // kept, in counter slots (one atomic per wave to one address serialises
-    // across the device)
+    // (rasters too large for the hierarchy); otherwise the flags come with the
+    // hierarchy's leaves, and only the count is kept, in counter slots (one
+    // atomic per wave to one address serialises across the device)
     c->blist_on = !btree_fits(c);
+    c->bt_ok = false;
     const int64_t nw = mkde_dev::slot_words();
     CHK(c->bcount.ensure(nw));
     HIPCHK(hipMemsetAsync(c->bcount.p, 0, nw * sizeof(unsigned long long), c->stream));
     if (c->blist_on) {
+        c->bt = BndTree{};
         // upper bound of the boundary list: every valid cell
         CHK(c->blist.ensure(nc));
         HIPCHK(mkde_dev::boundary(c->stream, c->mg, c->valid.p, c->bflags.p, c->blist.p, c->bcount.p));
     } else {
-        HIPCHK(mkde_dev::boundary(c->stream, c->mg, c->valid.p, c->bflags.p, nullptr, c->bcount.p));
+        CHK(shape_btree(c));
+        HIPCHK(mkde_dev::boundary_leaf(c->stream, c->mg, c->valid.p, c->bflags.p, c->bt, c->bt_bits.p, c->bt_box.p,
+                                       c->bcount.p));
         HIPCHK(mkde_dev::fold_slots(c->stream, c->bcount.p));
     }
     c->bflags_ok = true;
@@ -801,32 +836,11 @@ extern "C" int mkde_mark_boundary(mkde_ctx *c, uint8_t *flags, int64_t *n_bounda
     return MKDE_OK;
 }
 
-// Hierarchy over the boundary flags of the EC mask: 16x16-cell leaves up to
-// one root.  Rasters wider or taller than 16384 leaves use the brute-force
-// kernel instead.
+// The levels above the leaves that ensure_boundary left.
 static int ensure_btree(mkde_ctx *c)
 {
-    if (c->bt_ok) return MKDE_OK;
-    BndTree &T = c->bt;
-    T = BndTree{};
-    if (!btree_fits(c)) return MKDE_OK;
-    int nx = (int)((c->mg.ncols + MKDE_BT_S - 1) / MKDE_BT_S), ny = (int)((c->mg.nrows + MKDE_BT_S - 1) / MKDE_BT_S);
-    int64_t total = 0;
-    for (;;) {
-        T.nx[T.nlev] = nx;
-        T.ny[T.nlev] = ny;
-        T.off[T.nlev] = total;
-        total += (int64_t)nx * ny;
-        T.nlev++;
-        if (nx == 1 && ny == 1) break;
-        nx = (nx + 1) / 2;
-        ny = (ny + 1) / 2;
-    }
-    CHK(c->bt_bits.ensure(2 * (size_t)T.nx[0] * T.ny[0]));
-    CHK(c->bt_box.ensure(total));
-    HIPCHK(mkde_dev::bt_build(c->stream, c->mg, c->bflags.p, c->bt_bits.p, c->bt_box.p, T));
-    T.bits = c->bt_bits.p;
-    T.box = c->bt_box.p;
+    if (c->bt_ok || c->blist_on) return MKDE_OK;
+    HIPCHK(mkde_dev::bt_build(c->stream, c->bt, c->bt_box.p));
     c->bt_ok = true;
     return MKDE_OK;
 }

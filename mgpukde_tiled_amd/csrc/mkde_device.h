@@ -136,16 +136,24 @@ struct WorkList {
 // Boundary-cell hierarchy for exact nearest-boundary distances: leaves of
 // 16 x 16 cells hold a 256-bit mask of their boundary cells; every level keeps
 // the bounding box {x0, y0, x1, y1} of the boundary cell centres below a node
-// (x0 > x1: empty); level l has nx[l] x ny[l] nodes starting at off[l].
+// (x0 > x1: empty); level l has nx[l] x ny[l] nodes starting at off[l], the four
+// children of a node next to each other (bt_node), missing ones empty, so that
+// a node's expansion reads one 64-byte line.
 #define MKDE_BT_S 16
 #define MKDE_BT_MAXL 15
 struct BndTree {
     const uint4 *bits;     // 2 per leaf (256 bits, row-major within the leaf)
     const float4 *box;     // all levels
     int nlev;
-    int nx[MKDE_BT_MAXL], ny[MKDE_BT_MAXL];
+    int nx[MKDE_BT_MAXL + 1], ny[MKDE_BT_MAXL + 1];   // one level above the root: 1 x 1
     int64_t off[MKDE_BT_MAXL];
 };
+
+// Place of node (ix, iy) in its level, pnx = nx of the level above.
+__host__ __device__ inline int64_t bt_node(int ix, int iy, int pnx)
+{
+    return (((int64_t)(iy >> 1) * pnx + (ix >> 1)) << 2) | ((iy & 1) << 1) | (ix & 1);
+}
 
 // Per-row runs of valid cells of a mask (CSR): runs of row r are
 // run_se[run_ptr[r] .. run_ptr[r+1]), each (start, end) inclusive, ascending.
