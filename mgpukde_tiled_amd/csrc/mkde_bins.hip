@@ -31,6 +31,58 @@ __global__ __launch_bounds__(256) void k_bin_key(int64_t n, const float *x, cons
     idx[i] = (int)i;
 }
 
+// Fine order: a bin's points along a Hilbert curve over its 16 x 16 sub-cells.
+// The curve runs from the bin's lower left to its lower right corner, next to
+// where the curve of the bin on its right begins, so that 64 consecutive points
+// that straddle two bins of a row are neighbours too.
+#define BIN_SUB_BITS 4
+
+__device__ __forceinline__ unsigned hilbert_sub(int x, int y)
+{
+    unsigned d = 0;
+#pragma unroll
+    for (int s = BIN_SUB_BITS - 1; s >= 0; --s) {
+        const int m = (1 << s) - 1, qx = (x >> s) & 1, qy = (y >> s) & 1;
+        const int q = qx ? 3 - qy : qy;   // quadrants in the order lower left, upper left, upper right, lower right
+        d = 4 * d + (unsigned)q;
+        x &= m;
+        y &= m;
+        // the first quadrant's curve is transposed, the last one's about the other diagonal
+        const int tx = x, ty = y;
+        if (q == 0) {
+            x = ty;
+            y = tx;
+        }
+        if (q == 3) {
+            x = m - ty;
+            y = m - tx;
+        }
+    }
+    return d;
+}
+
+__device__ __forceinline__ int sub_cell(double v, int b)
+{
+    const int top = (1 << BIN_SUB_BITS) - 1;
+    const int k = (int)((v - (double)b) * (double)(top + 1));
+    return k < 0 ? 0 : (k > top ? top : k);
+}
+
+// Key of point i: its bin (as k_bin_key), then its place on the bin's curve.
+__global__ __launch_bounds__(256) void k_fine_key(int64_t n, const float *x, const float *y, BinGrid bg,
+                                                  unsigned *key, int *idx)
+{
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const double vx = ((double)x[i] - bg.x0) / bg.size, vy = ((double)y[i] - bg.y0) / bg.size;
+    int bx = (int)floor(vx);
+    int by = (int)floor(vy);
+    bx = bx < 0 ? 0 : (bx > bg.nbx - 1 ? bg.nbx - 1 : bx);
+    by = by < 0 ? 0 : (by > bg.nby - 1 ? bg.nby - 1 : by);
+    key[i] = ((unsigned)(by * bg.nbx + bx) << (2 * BIN_SUB_BITS)) | hilbert_sub(sub_cell(vx, bx), sub_cell(vy, by));
+    idx[i] = (int)i;
+}
+
 // First position of every bin from the sorted bin numbers: position p (0..n)
 // opens the bins after its predecessor's, up to and including its own, so
 // each of the nbins + 1 entries is written once and start[nbins] = n.
@@ -62,12 +114,40 @@ static int key_bits(int nbins)
     return b;
 }
 
-// Temporary storage of the sort for n points in nbins bins.
+// Bits of a fine key: at most 4M bins, so they fit 32.
+static int fine_bits(int nbins)
+{
+    const int b = key_bits(nbins) + 2 * BIN_SUB_BITS;
+    return b < 32 ? b : 32;
+}
+
+// Temporary storage of either sort for n points in nbins bins.
 hipError_t bin_sort_bytes(int64_t n, int nbins, size_t *bytes)
 {
-    *bytes = 0;
-    return rocprim::radix_sort_pairs(nullptr, *bytes, (const unsigned *)nullptr, (unsigned *)nullptr,
-                                     (const int *)nullptr, (int *)nullptr, (size_t)n, 0, key_bits(nbins));
+    size_t coarse = 0, fine = 0;
+    hipError_t e = rocprim::radix_sort_pairs(nullptr, coarse, (const unsigned *)nullptr, (unsigned *)nullptr,
+                                             (const int *)nullptr, (int *)nullptr, (size_t)n, 0, key_bits(nbins));
+    if (e == hipSuccess)
+        e = rocprim::radix_sort_pairs(nullptr, fine, (const unsigned *)nullptr, (unsigned *)nullptr,
+                                      (const int *)nullptr, (int *)nullptr, (size_t)n, 0, fine_bits(nbins));
+    *bytes = coarse > fine ? coarse : fine;
+    return e;
+}
+
+// Fine order of n points (arguments as bin_points; the bin starts are the same).
+hipError_t fine_points(hipStream_t s, int64_t n, const float *x, const float *y, const BinGrid &bg, int nbins,
+                       unsigned *key, unsigned *skey, int *idx, int *perm, void *tmp, size_t tmp_bytes, float *xs,
+                       float *ys)
+{
+    if (n <= 0) return hipSuccess;
+    const unsigned nb = (unsigned)((n + 255) / 256);
+    hipLaunchKernelGGL(k_fine_key, dim3(nb), dim3(256), 0, s, n, x, y, bg, key, idx);
+    size_t bytes = tmp_bytes;
+    hipError_t e = rocprim::radix_sort_pairs(tmp, bytes, (const unsigned *)key, skey, (const int *)idx, perm,
+                                             (size_t)n, 0, fine_bits(nbins), s);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(k_gather_xy, dim3(nb), dim3(256), 0, s, n, (const int *)perm, x, y, xs, ys);
+    return hipGetLastError();
 }
 
 // Bin order of n points: key / skey / idx are n-element scratch, perm gets the

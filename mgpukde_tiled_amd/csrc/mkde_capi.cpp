@@ -32,6 +32,8 @@
 namespace mkde_dev {
 hipError_t prep_points(hipStream_t, int64_t, const int *, const float *, const float *, const float *, const float *,
                        const float *, float, PtRec *);
+hipError_t prep_fine(hipStream_t, int64_t, const int *, const float *, const float *, const float *, const float *,
+                     const float *, float, PtRec *, GroupInfo *);
 hipError_t bin_stats(hipStream_t, int, const int *, const PtRec *, BinInfo *, double *);
 int64_t raster_blocks(const GridDesc &, const Tiling &);
 hipError_t density_plan(hipStream_t, const GridDesc &, const float *, const PointIndex &, const Tiling &,
@@ -45,7 +47,7 @@ hipError_t density_merge(hipStream_t, const GridDesc &, const Tiling &, const fl
 SplitRule point_rule(int, const Tuning &, bool);
 hipError_t point_plan(hipStream_t, const PointIndex &, float, const double *, int, const SplitRule &,
                       const WorkList &, unsigned *);
-hipError_t point_density(hipStream_t, const PointIndex &, int, float *, float, const int *, const int4 *,
+hipError_t point_density(hipStream_t, const PointIndex &, bool, int, float *, float *, float, const int *, const int4 *,
                          const unsigned *, double *, int, const unsigned *);
 hipError_t loo_multi(hipStream_t, const PointIndex &, const float *, const double *, const double *, int, float *,
                      const int *, const int4 *, const unsigned *, double *, int, const unsigned *);
@@ -55,6 +57,8 @@ hipError_t range_fill(hipStream_t, const PointIndex &, const int64_t *, int32_t 
 hipError_t bin_sort_bytes(int64_t, int, size_t *);
 hipError_t bin_points(hipStream_t, int64_t, const float *, const float *, const BinGrid &, int, unsigned *, unsigned *,
                       int *, int *, void *, size_t, float *, float *, int *);
+hipError_t fine_points(hipStream_t, int64_t, const float *, const float *, const BinGrid &, int, unsigned *, unsigned *,
+                       int *, int *, void *, size_t, float *, float *);
 hipError_t valid_cells(hipStream_t, int64_t, const float *, float, uint8_t *);
 hipError_t runs_count(hipStream_t, const GridDesc &, const uint8_t *, unsigned *, unsigned *, unsigned *, unsigned *,
                       int64_t *);
@@ -196,7 +200,13 @@ struct mkde_ctx {
     DevBuf<uint8_t> bin_tmp;
     DevBuf<int> bin_start;      // nbins + 1
     DevBuf<float> xs, ys;       // bin order
-    DevBuf<PtRec> pts;          // bin order, per-job constants
+    // fine order (PointIndex): sorted on first use after an upload
+    DevBuf<int> fperm;
+    DevBuf<float> fxs, fys;
+    DevBuf<GroupInfo> grp;      // (n + 63) / 64
+    bool fine_ok = false;
+    bool pts_fine = false;      // the order of pts
+    DevBuf<PtRec> pts;          // bin or fine order, per-job constants
     DevBuf<BinInfo> bin_box;
     DevBuf<double> bin_thr;
     DevBuf<double> reach;       // 1 value
@@ -468,6 +478,7 @@ static void forget_points(mkde_ctx *c)
     c->h_set = false;
     c->h_fixed = 0.0f;
     c->dist_set = false;
+    c->fine_ok = false;
     c->pts_dirty = true;
 }
 
@@ -511,6 +522,10 @@ extern "C" int mkde_points_upload(mkde_ctx *c, int64_t n, const float *x, const 
     CHK(c->xs.ensure(n));
     CHK(c->ys.ensure(n));
     CHK(c->perm.ensure(n));
+    CHK(c->fxs.ensure(n));
+    CHK(c->fys.ensure(n));
+    CHK(c->fperm.ensure(n));
+    CHK(c->grp.ensure((n + 63) / 64));
     CHK(c->bin_key.ensure(n));
     CHK(c->bin_skey.ensure(n));
     CHK(c->bin_idx.ensure(n));
@@ -563,14 +578,27 @@ extern "C" int mkde_num_points(mkde_ctx *c, int64_t *n)
     return MKDE_OK;
 }
 
-// Rebuild the bin-order point records after bandwidths or EC weights changed.
-static int prep(mkde_ctx *c)
+// Rebuild the point records after bandwidths or EC weights changed, or for the
+// other order.
+static int prep(mkde_ctx *c, bool fine = false)
 {
-    if (!c->pts_dirty) return MKDE_OK;
-    HIPCHK(mkde_dev::prep_points(c->stream, c->n, c->perm.p, c->xs.p, c->ys.p, c->w.p, c->h.p, c->ew.p, c->h_fixed,
-                                 c->pts.p));
-    HIPCHK(mkde_dev::bin_stats(c->stream, c->nbins, c->bin_start.p, c->pts.p, c->bin_box.p, c->bin_thr.p));
-    HIPCHK(mkde_dev::reach(c->stream, c->nbins, c->bin_thr.p, c->reach.p));
+    if (!c->pts_dirty && c->pts_fine == fine) return MKDE_OK;
+    if (fine && !c->fine_ok) {
+        HIPCHK(mkde_dev::fine_points(c->stream, c->n, c->x.p, c->y.p, c->bg, c->nbins, c->bin_key.p, c->bin_skey.p,
+                                     c->bin_idx.p, c->fperm.p, c->bin_tmp.p, c->bin_tmp.n, c->fxs.p, c->fys.p));
+        c->fine_ok = true;
+    }
+    if (fine)
+        HIPCHK(mkde_dev::prep_fine(c->stream, c->n, c->fperm.p, c->fxs.p, c->fys.p, c->w.p, c->h.p, c->ew.p,
+                                   c->h_fixed, c->pts.p, c->grp.p));
+    else
+        HIPCHK(mkde_dev::prep_points(c->stream, c->n, c->perm.p, c->xs.p, c->ys.p, c->w.p, c->h.p, c->ew.p, c->h_fixed,
+                                     c->pts.p));
+    c->pts_fine = fine;
+    if (c->pts_dirty) {   // the bins hold the same points in either order
+        HIPCHK(mkde_dev::bin_stats(c->stream, c->nbins, c->bin_start.p, c->pts.p, c->bin_box.p, c->bin_thr.p));
+        HIPCHK(mkde_dev::reach(c->stream, c->nbins, c->bin_thr.p, c->reach.p));
+    }
     c->pts_dirty = false;
     return MKDE_OK;
 }
@@ -579,6 +607,7 @@ static PointIndex index_of(mkde_ctx *c)
 {
     PointIndex I;
     I.pts = c->pts.p;
+    I.grp = c->pts_fine ? c->grp.p : nullptr;
     I.bin_start = c->bin_start.p;
     I.bin_box = c->bin_box.p;
     I.bin_thr = c->bin_thr.p;
@@ -1095,14 +1124,21 @@ static int plan_points(mkde_ctx *c, const PointIndex &I, int loo, float h_fixed,
     return MKDE_OK;
 }
 
+// The order a point density runs in: bin order for one bandwidth with the query
+// itself included (the pilot), else fine order.
+static bool density_fine(const mkde_ctx *c, int loo) { return loo || !(c->h_fixed > 0.0f); }
+
+// Densities at the points in that order.
 static int density_points_sorted(mkde_ctx *c, int loo, float *den_sorted)
 {
-    CHK(prep(c));
+    const bool fine = density_fine(c, loo);
+    CHK(prep(c, fine));
     PointIndex I = index_of(c);
+    if (fine) CHK(c->den2.ensure(c->n));
     HIPCHK(hipEventRecord(c->ev0, c->stream));
     PointWork P;
     CHK(plan_points(c, I, loo, c->h_fixed, nullptr, 0, 1, P));
-    HIPCHK(mkde_dev::point_density(c->stream, I, loo, den_sorted, c->h_fixed, P.order, P.items, c->pw_cost.p,
+    HIPCHK(mkde_dev::point_density(c->stream, I, fine, loo, den_sorted, c->den2.p, c->h_fixed, P.order, P.items, c->pw_cost.p,
                                    c->pw_partials.p, P.n_items, P.n_items_dev));
     HIPCHK(mkde_dev::point_merge(c->stream, c->n, 1, 1, P.n_split, c->pw_splits.p, c->pw_partials.p, den_sorted,
                                  P.n_split_dev));
@@ -1116,7 +1152,7 @@ extern "C" int mkde_density_at_points(mkde_ctx *c, int loo, float *den)
     CHK(need_h(c));
     CHK(c->den2.ensure(c->n));
     CHK(density_points_sorted(c, loo ? 1 : 0, c->den.p));
-    HIPCHK(mkde_dev::unsort_f32(c->stream, c->n, c->perm.p, c->den.p, c->den2.p));
+    HIPCHK(mkde_dev::unsort_f32(c->stream, c->n, density_fine(c, loo) ? c->fperm.p : c->perm.p, c->den.p, c->den2.p));
     if (den) CHK(copy_d2h(c, den, c->den2.p, c->n * sizeof(float)));
     HIPCHK(hipEventSynchronize(c->ev1));
     HIPCHK(hipEventElapsedTime(&c->last_points_ms, c->ev0, c->ev1));
@@ -1173,7 +1209,8 @@ extern "C" int mkde_density_at_points_noalloc(mkde_ctx *c, int loo, float *den_d
     if (!cv.ok)
         return fail(MKDE_E_RANGE, "%lld points need %zu bytes of scratch, more than the %u available", (long long)n,
                     cv.used, MKDE_SCRATCH_BYTES);
-    CHK(prep(c));
+    const bool fine = density_fine(c, loo);
+    CHK(prep(c, fine));
     PointIndex I = index_of(c);
     const WorkList W{cost, item0, slot0, sidx, counts, hist};
     HIPCHK(mkde_dev::point_plan(c->stream, I, c->h_fixed, nullptr, 0, mkde_dev::point_rule(loo ? 1 : 0, c->tune, false),
@@ -1190,10 +1227,10 @@ extern "C" int mkde_density_at_points_noalloc(mkde_ctx *c, int loo, float *den_d
                     "the %u available",
                     (long long)n, cnt[0], cnt[1], cv.used, MKDE_SCRATCH_BYTES);
     HIPCHK(mkde_dev::work_items(c->stream, (int)nw, W, items, splits, order));
-    HIPCHK(mkde_dev::point_density(c->stream, I, loo ? 1 : 0, den_s, c->h_fixed, order, items, cost, partials,
+    HIPCHK(mkde_dev::point_density(c->stream, I, fine, loo ? 1 : 0, den_s, den_dev, c->h_fixed, order, items, cost, partials,
                                    (int)cnt[0], nullptr));
     HIPCHK(mkde_dev::point_merge(c->stream, n, 1, 1, (int)cnt[2], splits, partials, den_s, nullptr));
-    HIPCHK(mkde_dev::unsort_f32(c->stream, n, c->perm.p, den_s, den_dev));
+    HIPCHK(mkde_dev::unsort_f32(c->stream, n, fine ? c->fperm.p : c->perm.p, den_s, den_dev));
     HIPCHK(hipStreamSynchronize(c->stream));
     return MKDE_OK;
 }

@@ -91,14 +91,34 @@ struct __attribute__((aligned(32))) PtRec {
     double a, thr;
 };
 
+// One source of the point densities in fine order (PtRec's places for x, y,
+// coef and thr): af = (float)a, and lo / hi bracket thr so that a float squared
+// distance below lo is inside the cut-off and one above hi is not.
+struct __attribute__((aligned(32))) SrcRec {
+    float x, y, coef, af, lo, hi;
+    double thr;
+};
+
+// 64 consecutive points in fine order: their bounding box and the smallest and
+// largest cut-off threshold.
+struct GroupInfo {
+    float x0, y0, x1, y1;
+    double tmin, tmax;
+};
+
 // Per-bin summary used for culling: bounding box of the bin's points and the
 // largest cut-off threshold 9*h2f among them.
 struct BinInfo {
     float x0, y0, x1, y1;
 };
 
+// Two orders share the bins.  In bin order a bin's points keep the caller's
+// order; in fine order they follow a Hilbert curve through the bin, so that 64
+// consecutive points are close together.  The pilot densities, whose rounding
+// every adaptive bandwidth inherits, are summed in bin order.
 struct PointIndex {
-    const PtRec *pts;       // n, bin order
+    const PtRec *pts;       // n, bin order; fine order: SrcRec
+    const GroupInfo *grp;   // fine order: (n + 63) / 64
     const int *bin_start;   // nbins + 1
     const BinInfo *bin_box; // nbins
     const double *bin_thr;  // nbins

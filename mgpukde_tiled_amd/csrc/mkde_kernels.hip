@@ -7,8 +7,8 @@
 //   k_ec              per-point edge-correction integral, O(R) per point
 //                     (replaces CalcEdgeCorrectionWeights kde_kernel_kdtr.cu:117-265
 //                     and EdgeCorrectionWeightsExact tiled:2694-2807)
-//   k_point_density_w density at points over the cell-binned index, pilot and
-//                     leave-one-out forms (replaces DensityAtPointsKdtr
+//   k_pilot_density, k_point_density_f   density at points over the cell-binned
+//                     index, pilot and leave-one-out forms (replaces DensityAtPointsKdtr
 //                     kde_kernel_kdtr.cu:681-953 and the CPU scatter tiled:3312-3347)
 //   k_loo_multi_w     leave-one-out densities of up to 16 fixed bandwidths in one
 //                     pass over point pairs (batched LogLikelihood, tiled:3214-3368)
@@ -181,6 +181,50 @@ __global__ void k_prep_points(int64_t n, const int *perm, const float *xs, const
         r.thr = -1.0;
     }
     out[i] = r;
+}
+
+// The same in fine order (SrcRec, one wave per group of 64), with each group's
+// box and thresholds.
+__global__ __launch_bounds__(256) void k_prep_fine(int64_t n, const int *perm, const float *xs, const float *ys,
+                                                   const float *w_orig, const float *h_orig, const float *ew_orig,
+                                                   float h_fixed, SrcRec *out, GroupInfo *grp)
+{
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const bool on = i < n;
+    SrcRec r;
+    if (on) {
+        const int o = perm[i];
+        const float h = h_fixed > 0.0f ? h_fixed : (h_orig ? h_orig[o] : 0.0f);
+        const double h2 = (double)(float)(h * h);
+        r.x = xs[i];
+        r.y = ys[i];
+        r.coef = r.af = 0.0f;
+        r.thr = -1.0;
+        r.lo = r.hi = -1.0f;
+        if (h2 > 0.0 && h2 < 1e300) {
+            r.coef = (float)((double)w_orig[o] * (double)ew_orig[o] / (h2 * (double)MKDE_TWO_PI_F));
+            r.af = (float)(-MKDE_LOG2E / (2.0 * h2));
+            r.thr = 9.0 * h2;
+            // fl32(dx^2 + dy^2) is within 2^-22 relative where it neither
+            // overflows nor becomes subnormal; elsewhere nothing is taken as
+            // decided (lo = -1, a hi that holds for every distance in doubt)
+            const bool plain = r.thr > 1e-30 && r.thr < 1e37;
+            r.lo = plain ? (float)(r.thr * (1.0 - 1.0 / 1048576.0)) : -1.0f;
+            r.hi = plain ? (float)(r.thr * (1.0 + 1.0 / 1048576.0)) : r.thr > 1.0 ? INFINITY : 1e-29f;
+        }
+        out[i] = r;
+    }
+    float x0 = on ? r.x : FLT_MAX, y0 = on ? r.y : FLT_MAX, x1 = on ? r.x : -FLT_MAX, y1 = on ? r.y : -FLT_MAX;
+    double lo = on ? r.thr : DBL_MAX, hi = on ? r.thr : -DBL_MAX;
+    for (int d = 32; d >= 1; d >>= 1) {
+        x0 = fminf(x0, __shfl_xor(x0, d, WAVE));
+        x1 = fmaxf(x1, __shfl_xor(x1, d, WAVE));
+        y0 = fminf(y0, __shfl_xor(y0, d, WAVE));
+        y1 = fmaxf(y1, __shfl_xor(y1, d, WAVE));
+        lo = fmin(lo, __shfl_xor(lo, d, WAVE));
+        hi = fmax(hi, __shfl_xor(hi, d, WAVE));
+    }
+    if (on && (threadIdx.x & 63) == 0) grp[i >> 6] = GroupInfo{x0, y0, x1, y1, lo, hi};
 }
 
 // Per-bin bounding box of the points and largest threshold.
@@ -1106,23 +1150,26 @@ __global__ void k_scan_add(int n, unsigned *out, const unsigned *chunk_sums)
 
 // ==================================================== density at points ====
 //
-// One wave owns 64 consecutive query points in bin order (lane = query) and
-// walks the candidate bins of its bounding box; the source records are
-// wave-uniform and come in by scalar loads.  Each source uses its own
-// bandwidth (sample-point estimator); FIXED specialises the common case of
-// one bandwidth.  LOO excludes the query itself (same index); duplicates at
-// distance 0 are kept.  Waves are launched heaviest first (k_wave_cost).
+// One wave owns 64 consecutive query points (lane = query) and walks the
+// candidate bins of its bounding box; a source's record is wave-uniform and
+// comes in by scalar loads.  Two forms:
+//   k_pilot_density    one bandwidth, the query itself included, bin order: the
+//                      densities the adaptive bandwidths come from
+//   k_point_density_f  every other case (a bandwidth per source, leave-one-out),
+//                      fine order, with sums over whole groups of sources
+// Duplicates at distance 0 are kept in both.  Waves run heaviest first
+// (k_wave_cost).
 //
 // Cut-off test: d2f = fl32(dx*dx + dy*dy) decides unless it lies within a
 // relative 2^-20 band around the threshold (its error is below 2^-22
-// relative); for a wave with any lane in the band the exact FP64 test
+// relative); where any lane is in the band the exact FP64 test
 // fl64(dx^2 + dy^2) < thr is evaluated instead, so the result is exact.
 
 struct PtsArgs {
     PointIndex idx;
-    float *den;   // output, bin order
-    int loo;
-    double thr_fixed, a_fixed;   // FIXED kernels only
+    float *den;   // output, the index's order
+    float *res;   // n floats of scratch (fine order)
+    double thr_fixed, a_fixed;   // k_pilot_density only
     // work items (nullable order: one item per wave): {wave, part j, parts K,
     // partial slot}; part j of a wave takes candidate ordinals
     // [C j / K, C (j+1) / K) of its C candidate sources (cost[wave])
@@ -1136,12 +1183,6 @@ struct PtsArgs {
 
 #define PD_BAND (1.0 / 1048576.0)
 
-// Per-wave variant: each wave owns 64 consecutive queries in bin order and
-// walks the candidate bins of its own bounding box; a source's record is
-// wave-uniform, so it is read with scalar loads into SGPRs (no LDS, and the
-// VALU reads SGPR operands for free).  FIXED: FP32 screen with the FP64
-// re-check of a 32-source chunk when any lane is inside the 2^-20 band;
-// otherwise (per-source bandwidths) the exact FP64 test for every pair.
 __device__ __forceinline__ float wave_min(float v)
 {
     for (int d = 32; d >= 1; d >>= 1) v = fminf(v, __shfl_xor(v, d, WAVE));
@@ -1198,8 +1239,10 @@ __global__ __launch_bounds__(256) void k_wave_cost(PointIndex I, double lim_fixe
     if (lane == 0) cost[wv] = acc;
 }
 
-template <bool FIXED, bool LOO>
-__global__ __launch_bounds__(256) void k_point_density_w(PtsArgs A)
+// Pilot densities at one bandwidth.  Kept as it is, operation by operation: the
+// adaptive bandwidths h_i follow from these sums, and a bandwidth that moves by
+// one rounding takes pairs across the hard cut-off.
+__global__ __launch_bounds__(256) void k_pilot_density(PtsArgs A)
 {
     const PointIndex &I = A.idx;
     const int lane = threadIdx.x & 63;
@@ -1226,7 +1269,7 @@ __global__ __launch_bounds__(256) void k_point_density_w(PtsArgs A)
     }
     const float mnx = uni(wave_min(qv ? qx : FLT_MAX)), mxx = uni(wave_max(qv ? qx : -FLT_MAX));
     const float mny = uni(wave_min(qv ? qy : FLT_MAX)), mxy = uni(wave_max(qv ? qy : -FLT_MAX));
-    const double reach = FIXED ? sqrt(fmax(A.thr_fixed, 0.0)) * 1.000001 + 1e-6 : *I.reach_p;
+    const double reach = sqrt(fmax(A.thr_fixed, 0.0)) * 1.000001 + 1e-6;
     int bxa, bxb, bya, byb;
     bin_range(I.bg, mnx, mxx, mny, mxy, reach, bxa, bxb, bya, byb);
     bxa = __builtin_amdgcn_readfirstlane(bxa);
@@ -1234,9 +1277,9 @@ __global__ __launch_bounds__(256) void k_point_density_w(PtsArgs A)
     bya = __builtin_amdgcn_readfirstlane(bya);
     byb = __builtin_amdgcn_readfirstlane(byb);
 
-    const float f_thr_lo = FIXED ? (float)(A.thr_fixed * (1.0 - PD_BAND)) : 0.0f;
-    const float f_thr_hi = FIXED ? fmaxf((float)(A.thr_fixed * (1.0 + PD_BAND)), FLT_MIN) : 0.0f;
-    const float f_a = FIXED ? (float)A.a_fixed : 0.0f;
+    const float f_thr_lo = (float)(A.thr_fixed * (1.0 - PD_BAND));
+    const float f_thr_hi = fmaxf((float)(A.thr_fixed * (1.0 + PD_BAND)), FLT_MIN);
+    const float f_a = (float)A.a_fixed;
     float acc = 0.0f, sum = 0.0f, comp = 0.0f;
     int ord = 0;   // candidate ordinal at the start of the next candidate bin
     for (int by = bya; by <= byb; ++by) {
@@ -1244,22 +1287,15 @@ __global__ __launch_bounds__(256) void k_point_density_w(PtsArgs A)
             const int b = by * I.bg.nbx + bx;
             const int bst = I.bin_start[b], ben = I.bin_start[b + 1];
             if (bst == ben) continue;
-            const double lim = FIXED ? A.thr_fixed : I.bin_thr[b];
             const BinInfo bb = I.bin_box[b];
-            if (!__builtin_amdgcn_readfirstlane((int)(box_gap2(bb, mnx, mxx, mny, mxy) < lim))) continue;
-            // FIXED: every pair of the bin and the wave is inside the screen
-            // when the largest fl32 offsets give d2f below it (fl32 of a
-            // difference, the product and the fma are monotone in |offset|,
-            // so no pair's d2f exceeds this one): such a bin's sources need no
-            // compare and no select, and add the same terms.  LOO keeps the
-            // tests for the bin holding the wave's own queries.
-            bool all_in = false;
-            if (FIXED) {
-                const float gx = fmaxf(bb.x1 - mnx, mxx - bb.x0), gy = fmaxf(bb.y1 - mny, mxy - bb.y0);
-                all_in = __builtin_fmaf(gy, gy, gx * gx) < f_thr_lo &&
-                         (!LOO || (int64_t)ben <= q0 || (int64_t)bst >= q0 + 64);
-                all_in = __builtin_amdgcn_readfirstlane((int)all_in);
-            }
+            if (!__builtin_amdgcn_readfirstlane((int)(box_gap2(bb, mnx, mxx, mny, mxy) < A.thr_fixed))) continue;
+            // every pair of the bin and the wave is inside the screen when the
+            // largest fl32 offsets give d2f below it (fl32 of a difference,
+            // the product and the fma are monotone in |offset|, so no pair's
+            // d2f exceeds this one): such a bin's sources need no compare and
+            // no select, and add the same terms
+            const float gx = fmaxf(bb.x1 - mnx, mxx - bb.x0), gy = fmaxf(bb.y1 - mny, mxy - bb.y0);
+            const bool all_in = __builtin_amdgcn_readfirstlane((int)(__builtin_fmaf(gy, gy, gx * gx) < f_thr_lo));
             // this part's share of the candidate sequence
             const int o0 = ord, o1 = ord + (ben - bst);
             ord = o1;
@@ -1270,7 +1306,7 @@ __global__ __launch_bounds__(256) void k_point_density_w(PtsArgs A)
                 const int c1 = c0 + 32 < en ? c0 + 32 : en;
                 // four records are loaded before their arithmetic, so the
                 // scalar loads overlap
-                if (FIXED && all_in) {
+                if (all_in) {
                     int si = c0;
                     for (; si + 4 <= c1; si += 4) {
                         const PtRec p0 = I.pts[si], p1 = I.pts[si + 1], p2 = I.pts[si + 2], p3 = I.pts[si + 3];
@@ -1286,56 +1322,36 @@ __global__ __launch_bounds__(256) void k_point_density_w(PtsArgs A)
                         const float d2f = __builtin_fmaf(dy, dy, dx * dx);
                         acc = __builtin_fmaf(fast_exp2(d2f * f_a), p.coef, acc);
                     }
-                } else if (FIXED) {
+                } else {
                     bool band = false;
-                    auto body = [&](const PtRec &p, int si) {
+                    auto body = [&](const PtRec &p) {
                         const float dx = p.x - qx, dy = p.y - qy;
                         const float d2f = __builtin_fmaf(dy, dy, dx * dx);
-                        bool in = d2f < f_thr_lo;
+                        const bool in = d2f < f_thr_lo;
                         band |= (d2f < f_thr_hi) != in;
-                        if (LOO && (int64_t)si == q) in = false;
                         const float e = fast_exp2(d2f * f_a);
                         acc = __builtin_fmaf(in ? e : 0.0f, p.coef, acc);
                     };
                     int si = c0;
                     for (; si + 4 <= c1; si += 4) {
                         const PtRec p0 = I.pts[si], p1 = I.pts[si + 1], p2 = I.pts[si + 2], p3 = I.pts[si + 3];
-                        body(p0, si);
-                        body(p1, si + 1);
-                        body(p2, si + 2);
-                        body(p3, si + 3);
+                        body(p0);
+                        body(p1);
+                        body(p2);
+                        body(p3);
                     }
-                    for (; si < c1; ++si) body(I.pts[si], si);
+                    for (; si < c1; ++si) body(I.pts[si]);
                     if (__any(band)) {   // rare: exact FP64 test for the chunk
                         acc = 0.0f;
                         for (int sj = c0; sj < c1; ++sj) {
                             const PtRec p = I.pts[sj];
                             const float dx = p.x - qx, dy = p.y - qy;
                             const float d2f = __builtin_fmaf(dy, dy, dx * dx);
-                            bool in = sq2(dx, dy) < A.thr_fixed;
-                            if (LOO && (int64_t)sj == q) in = false;
+                            const bool in = sq2(dx, dy) < A.thr_fixed;
                             const float e = fast_exp2(d2f * f_a);
                             acc = __builtin_fmaf(in ? e : 0.0f, p.coef, acc);
                         }
                     }
-                } else {
-                    auto body = [&](const PtRec &p, int si) {
-                        const float dx = p.x - qx, dy = p.y - qy;
-                        const float d2f = __builtin_fmaf(dy, dy, dx * dx);
-                        bool in = sq2(dx, dy) < p.thr;
-                        if (LOO && (int64_t)si == q) in = false;
-                        const float e = fast_exp2(d2f * (float)p.a);
-                        acc = __builtin_fmaf(in ? e : 0.0f, p.coef, acc);
-                    };
-                    int si = c0;
-                    for (; si + 4 <= c1; si += 4) {
-                        const PtRec p0 = I.pts[si], p1 = I.pts[si + 1], p2 = I.pts[si + 2], p3 = I.pts[si + 3];
-                        body(p0, si);
-                        body(p1, si + 1);
-                        body(p2, si + 2);
-                        body(p3, si + 3);
-                    }
-                    for (; si < c1; ++si) body(I.pts[si], si);
                 }
                 kahan_fold(acc, sum, comp);
                 acc = 0.0f;
@@ -1344,6 +1360,311 @@ __global__ __launch_bounds__(256) void k_point_density_w(PtsArgs A)
     }
     if (item.z > 1) A.partials[(int64_t)item.w * 64 + lane] = (double)sum - (double)comp;
     else if (qv) A.den[q] = sum;
+}
+
+// Whole groups of sources.  For a group of 64 sources whose every pair with the
+// wave is inside the cut-off, and a wave whose points lie close together
+// compared with the sources' bandwidths, the 64 kernels are expanded about the
+// centre c of the wave's box: with d = s - c, t = q - c, b = 1 / (2 h^2)
+//   exp(-b |t - d|^2) = exp(-b d^2) sum_ij m_i(dx) m_j(dy) tx^i ty^j / (i! j!),
+//   m_0 = 1, m_1 = 2 b d, m_(k+1) = 2 b d m_k - 2 b k m_(k-1)
+// (the Hermite generating function), so a source adds coef exp(-b d^2) m_i m_j
+// to 36 moments (i + j < PF_P), one source per lane, and the polynomial is
+// evaluated once per query at the end of the walk.  About 100 instructions a
+// group instead of 64 times 8.  Moments are FP64 (its rate is that of FP32
+// here).  What is left out is below 0.025 tau^8 of a source's kernel, tau =
+// |t| / h <= PF_TAU: 1.1e-8, under the rounding of the FP32 exponentials.
+#define PF_P 8
+#define PF_NM (PF_P * (PF_P + 1) / 2)
+#define PF_TAU 0.16
+
+__device__ __forceinline__ void group_moments(const SrcRec &p, bool on, double cx, double cy, double (&M)[PF_NM])
+{
+    const double dx = (double)p.x - cx, dy = (double)p.y - cy;
+    const double d2 = __builtin_fma(dy, dy, dx * dx);
+    const double af = p.af;
+    const double b2 = af * (-2.0 * 0.69314718055994530942);   // 1 / h^2
+    const double ux = b2 * dx, uy = b2 * dy;
+    double gx[PF_P], gy[PF_P];
+    gx[0] = on ? (double)p.coef * (double)fast_exp2((float)(d2 * af)) : 0.0;
+    gx[1] = ux * gx[0];
+    gy[0] = 1.0;
+    gy[1] = uy;
+#pragma unroll
+    for (int k = 1; k + 1 < PF_P; ++k) {
+        const double v = b2 * (double)k;
+        gx[k + 1] = __builtin_fma(ux, gx[k], -v * gx[k - 1]);
+        gy[k + 1] = __builtin_fma(uy, gy[k], -v * gy[k - 1]);
+    }
+    int o = 0;
+#pragma unroll
+    for (int i = 0; i < PF_P; ++i)
+#pragma unroll
+        for (int j = 0; j < PF_P - i; ++j, ++o) M[o] = __builtin_fma(gx[i], gy[j], M[o]);
+}
+
+// A work item of the fine-order kernels and its wave's box.
+struct FineItem {
+    int4 item;
+    int win0, win1;     // candidate ordinals of this part
+    int q;              // this lane's query
+    GroupInfo W;
+    int bxa, bxb, bya, byb;
+    double cx, cy;      // centre of the box
+    double wide;        // groups are taken whole from this smallest 9 h^2 on
+};
+
+// false: the grid is larger than the list (whole wave).
+__device__ __forceinline__ bool fine_item(const PtsArgs &A, FineItem &F)
+{
+    const PointIndex &I = A.idx;
+    // the wave index and the work item are wave-uniform: made explicit so the
+    // source records are read with scalar loads
+    const int64_t g = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t units = A.n_items_dev ? (int64_t)*A.n_items_dev : A.order ? (int64_t)A.n_items : (I.n + 63) / 64;
+    if (g >= units) return false;
+    F.item = uniform_item(A.order ? A.items[A.order[g]] : make_int4((int)g, 0, 1, -1));
+    F.win0 = 0;
+    F.win1 = INT_MAX;   // candidate counts are below 2^31
+    if (F.item.z > 1) {
+        const int64_t C = A.cost[F.item.x];
+        if (F.item.y > 0) F.win0 = (int)(C * F.item.y / F.item.z);
+        if (F.item.y < F.item.z - 1) F.win1 = (int)(C * (F.item.y + 1) / F.item.z);
+    }
+    F.q = F.item.x * 64 + (int)(threadIdx.x & 63);   // below 2^30
+    F.W = I.grp[F.item.x];
+    const GroupInfo &W = F.W;
+    bin_range(I.bg, W.x0, W.x1, W.y0, W.y1, *I.reach_p, F.bxa, F.bxb, F.bya, F.byb);
+    F.bxa = __builtin_amdgcn_readfirstlane(F.bxa);
+    F.bxb = __builtin_amdgcn_readfirstlane(F.bxb);
+    F.bya = __builtin_amdgcn_readfirstlane(F.bya);
+    F.byb = __builtin_amdgcn_readfirstlane(F.byb);
+    F.cx = 0.5 * ((double)W.x0 + (double)W.x1);
+    F.cy = 0.5 * ((double)W.y0 + (double)W.y1);
+    const double hx = (double)W.x1 - F.cx, hy = (double)W.y1 - F.cy;
+    F.wide = fmax((hx * hx + hy * hy) * (9.0 / (PF_TAU * PF_TAU)), 1e-30);
+    return true;
+}
+
+// What lane l sees of group gb + l of a row of bins, whose sources s0 .. s1 - 1
+// are consecutive: its share c0 .. c1 - 1 of them and cls 0: no pair with the
+// wave's box W is inside the cut-off, 1: some may be, 2: all are (the largest
+// fl32 offsets are, and sq2 is monotone), 3: all are and the group is taken
+// whole.  own: the wave's group (LOO) or -1; wide: FineItem::wide.
+__device__ __forceinline__ int group_class(const PointIndex &I, const GroupInfo &W, int gb, int s0, int s1, int own,
+                                           double wide, int &c0, int &c1)
+{
+    const int g = gb + (int)(threadIdx.x & 63);
+    const bool on = g <= (s1 - 1) >> 6;
+    const GroupInfo G = I.grp[on ? g : gb];
+    c0 = s0 > g * 64 ? s0 : g * 64;
+    c1 = s1 < g * 64 + 64 ? s1 : g * 64 + 64;
+    const float fx = fmaxf(G.x1 - W.x0, W.x1 - G.x0), fy = fmaxf(G.y1 - W.y0, W.y1 - G.y0);
+    const bool near = on && box_gap2(BinInfo{G.x0, G.y0, G.x1, G.y1}, W.x0, W.x1, W.y0, W.y1) < G.tmax;
+    const bool full = sq2(fx, fy) < G.tmin && g != own;
+    const bool whole = full && G.tmin >= wide && G.tmin < 1e37;
+    return near ? 1 + (int)full + (int)whole : 0;
+}
+
+// Walks an item's candidate groups, 64 at a time (one per lane), and calls
+// fn(c0, c1, all) for those taken whole (WHOLE) or for the others; all: every
+// pair is inside.  (Group by group with wave-uniform tests the walks took a
+// third of the kernels' instructions.)
+template <bool LOO, bool WHOLE, class F>
+__device__ __forceinline__ void fine_walk(const PointIndex &I, const FineItem &T, F fn)
+{
+    const int lane = threadIdx.x & 63;
+    int ord = 0;   // candidate ordinal of the next group
+    for (int by = T.bya; by <= T.byb; ++by) {
+        const int row = by * I.bg.nbx;
+        const int s0 = I.bin_start[row + T.bxa], s1 = I.bin_start[row + T.bxb + 1];
+        for (int gb = s0 >> 6; gb * 64 < s1; gb += 64) {
+            int c0, c1;
+            int cls = group_class(I, T.W, gb, s0, s1, LOO ? T.item.x : -1, T.wide, c0, c1);
+            if (T.item.z > 1) {
+                // this part's share of the candidate sequence
+                const int cnt = cls ? c1 - c0 : 0;
+                const int o1 = ord + (int)wave_incl_scan((unsigned)cnt, lane), o0 = o1 - cnt;
+                ord = __builtin_amdgcn_readlane(o1, 63);
+                if (o1 <= T.win0 || o0 >= T.win1) cls = 0;
+                if (T.win0 > o0) c0 += T.win0 - o0;
+                if (T.win1 < o1) c1 -= o1 - T.win1;
+            }
+            if (cls == 3 && c1 - c0 < 12) cls = 2;   // cheaper source by source
+            uint64_t m = __ballot(WHOLE ? cls == 3 : cls == 1 || cls == 2);
+            const uint64_t all = __ballot(cls >= 2);
+            while (m) {
+                const int l = __builtin_ctzll(m);
+                m &= m - 1ull;
+                fn(__builtin_amdgcn_readlane(c0, l), __builtin_amdgcn_readlane(c1, l), (bool)((all >> l) & 1ull));
+            }
+        }
+    }
+}
+
+// Work estimate of each fine-order wave: the sources of its candidate groups.
+__global__ __launch_bounds__(256) void k_fine_cost(PointIndex I, unsigned *cost)
+{
+    const int lane = threadIdx.x & 63;
+    const int wv = (int)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if ((int64_t)wv * 64 >= I.n) return;
+    const GroupInfo W = I.grp[wv];
+    int bxa, bxb, bya, byb;
+    bin_range(I.bg, W.x0, W.x1, W.y0, W.y1, *I.reach_p, bxa, bxb, bya, byb);
+    unsigned acc = 0;
+    for (int by = bya; by <= byb; ++by) {
+        const int row = by * I.bg.nbx;
+        const int s0 = I.bin_start[row + bxa], s1 = I.bin_start[row + bxb + 1];
+        for (int gb = s0 >> 6; gb * 64 < s1; gb += 64) {
+            int c0, c1;
+            if (group_class(I, W, gb, s0, s1, -1, 1e300, c0, c1)) acc += (unsigned)(c1 - c0);
+        }
+    }
+    for (int d = 32; d >= 1; d >>= 1) acc += __shfl_xor(acc, d, WAVE);
+    if (lane == 0) cost[wv] = acc;
+}
+
+// The sources taken in whole groups.  Runs before k_point_density_f and
+// leaves an unsplit wave's sum as a pair of floats in den and res, a part's in
+// its slot of the partials.  A kernel of its own: with its moments it takes 4
+// waves per SIMD, while the other sources' scalar loads want 8 to hide behind.
+// 1M clustered points, adaptive bandwidths, leave-one-out: 8.8 ms pair by pair
+// with an FP64 test each, 0.63 + 3.63 ms now (12.0 ms with both in one kernel).
+template <bool LOO>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_group_density_f(PtsArgs A)
+{
+    const PointIndex &I = A.idx;
+    const SrcRec *src = (const SrcRec *)I.pts;
+    const int lane = threadIdx.x & 63;
+    FineItem T;
+    if (!fine_item(A, T)) return;
+    double v = 0.0;
+    // no source is wide enough when the largest cut-off radius is not
+    if ((*I.reach_p) * (*I.reach_p) >= T.wide) {
+        double M[PF_NM];
+#pragma unroll
+        for (int k = 0; k < PF_NM; ++k) M[k] = 0.0;
+        // a group's records are loaded while the one before is summed
+        SrcRec next;
+        bool next_on = false, any = false;
+        fine_walk<LOO, true>(I, T, [&](int c0, int c1, bool) {
+            const bool on = c0 + lane < c1;
+            const SrcRec p = next;
+            next = src[on ? c0 + lane : c0];
+            if (any) group_moments(p, next_on, T.cx, T.cy, M);
+            next_on = on;
+            any = true;
+        });
+        if (any) {
+            group_moments(next, next_on, T.cx, T.cy, M);
+            // moments over the lanes, then this query's polynomial (Horner in
+            // both variables, with the factorials)
+            const bool qv = T.q < I.n;
+            const double tx = (qv ? (double)src[T.q].x : T.cx) - T.cx, ty = (qv ? (double)src[T.q].y : T.cy) - T.cy;
+            int o = PF_NM;
+#pragma unroll
+            for (int i = PF_P - 1; i >= 0; --i) {
+                double row = 0.0;
+#pragma unroll
+                for (int j = PF_P - 1 - i; j >= 0; --j) {
+                    double m = M[--o];
+                    for (int d = 32; d >= 1; d >>= 1) m += __shfl_xor(m, d, WAVE);
+                    row = __builtin_fma(row, ty * (1.0 / (double)(j + 1)), m);
+                    __builtin_amdgcn_sched_barrier(0);   // one moment after the other, few registers
+                }
+                v = __builtin_fma(v, tx * (1.0 / (double)(i + 1)), row);
+            }
+        }
+    }
+    if (T.item.z > 1) {
+        A.partials[(int64_t)T.item.w * 64 + lane] = v;
+    } else if (T.q < I.n) {
+        const float hi = (float)v;
+        A.den[T.q] = hi;
+        A.res[T.q] = (float)(v - (double)hi);
+    }
+}
+
+typedef float f32x8 __attribute__((ext_vector_type(8)));
+
+// The other sources, pair by pair, and the total.
+template <bool LOO>
+__global__ __launch_bounds__(256) void k_point_density_f(PtsArgs A)
+{
+    const PointIndex &I = A.idx;
+    const SrcRec *src = (const SrcRec *)I.pts;
+    const int lane = threadIdx.x & 63;
+    FineItem T;
+    if (!fine_item(A, T)) return;
+    const int q = T.q;
+    const bool qv = q < I.n;
+    const float qx = qv ? src[q].x : T.W.x0, qy = qv ? src[q].y : T.W.y0;
+    float acc = 0.0f, sum = 0.0f, comp = 0.0f;
+    fine_walk<LOO, false>(I, T, [&](int c0, int c1, bool all) {
+        // the query itself is left out of its own group's sums
+        const bool self = LOO && (c0 >> 6) == T.item.x;
+        for (int s0 = c0; s0 < c1; s0 += 32) {
+            const int s1 = s0 + 32 < c1 ? s0 + 32 : c1;
+            // four records are loaded before their arithmetic, so the scalar
+            // loads overlap
+            if (all) {
+                auto body = [&](const SrcRec &p) {
+                    const float dx = p.x - qx, dy = p.y - qy;
+                    const float d2f = __builtin_fmaf(dy, dy, dx * dx);
+                    acc = __builtin_fmaf(fast_exp2(d2f * p.af), p.coef, acc);
+                };
+                int si = s0;
+                for (; si + 4 <= s1; si += 4) {
+                    const SrcRec p0 = src[si], p1 = src[si + 1], p2 = src[si + 2], p3 = src[si + 3];
+                    body(p0);
+                    body(p1);
+                    body(p2);
+                    body(p3);
+                }
+                for (; si < s1; ++si) body(src[si]);
+            } else {
+                bool band = self;
+                auto body = [&](const f32x8 &p) {
+                    const float dx = p[0] - qx, dy = p[1] - qy;
+                    const float d2f = __builtin_fmaf(dy, dy, dx * dx);
+                    const bool in = d2f < p[4];
+                    band |= !(d2f > p[5]) != in;
+                    const float e = fast_exp2(d2f * p[3]);
+                    acc = __builtin_fmaf(in ? e : 0.0f, p[2], acc);
+                };
+                // whole records, one scalar load each
+                const f32x8 *rec = (const f32x8 *)src;
+                int si = s0;
+                if (!self) {
+                    for (; si + 4 <= s1; si += 4) {
+                        const f32x8 p0 = rec[si], p1 = rec[si + 1], p2 = rec[si + 2], p3 = rec[si + 3];
+                        body(p0);
+                        body(p1);
+                        body(p2);
+                        body(p3);
+                    }
+                    for (; si < s1; ++si) body(rec[si]);
+                }
+                if (__any(band)) {   // rare, and the wave's own group: exact FP64 test
+                    acc = 0.0f;
+                    for (int sj = s0; sj < s1; ++sj) {
+                        const SrcRec p = src[sj];
+                        const float dx = p.x - qx, dy = p.y - qy;
+                        const float d2f = __builtin_fmaf(dy, dy, dx * dx);
+                        bool in = sq2(dx, dy) < p.thr;
+                        if (LOO && sj == q) in = false;
+                        const float e = fast_exp2(d2f * p.af);
+                        acc = __builtin_fmaf(in ? e : 0.0f, p.coef, acc);
+                    }
+                }
+            }
+            kahan_fold(acc, sum, comp);
+            acc = 0.0f;
+        }
+    });
+    const double den = (double)sum - (double)comp;
+    if (T.item.z > 1) A.partials[(int64_t)T.item.w * 64 + lane] += den;
+    else if (qv) A.den[q] = (float)(den + ((double)A.den[q] + (double)A.res[q]));
 }
 
 // Exclusive scan of one int per thread across a 256-thread block.
@@ -2786,6 +3107,14 @@ hipError_t prep_points(hipStream_t s, int64_t n, const int *perm, const float *x
     return hipGetLastError();
 }
 
+hipError_t prep_fine(hipStream_t s, int64_t n, const int *perm, const float *xs, const float *ys, const float *w,
+                     const float *h, const float *ew, float h_fixed, PtRec *out, GroupInfo *grp)
+{
+    if (n > 0) hipLaunchKernelGGL(k_prep_fine, dim3(nblk(n, 256)), dim3(256), 0, s, n, perm, xs, ys, w, h, ew, h_fixed,
+                                  (SrcRec *)out, grp);
+    return hipGetLastError();
+}
+
 hipError_t bin_stats(hipStream_t s, int nbins, const int *bin_start, const PtRec *pts, BinInfo *box, double *thr)
 {
     hipLaunchKernelGGL(k_bin_stats, dim3(nblk(nbins, 4)), dim3(256), 0, s, nbins, bin_start, pts, box, thr);
@@ -2869,37 +3198,46 @@ SplitRule point_rule(int kind, const Tuning &T, bool batched)
 // Work list of the point kernels (64-query waves): costs and scans; W.counts
 // and, when given, the pinned host words receive {items, slots, splits, T}.
 // thr_k non-null: batched leave-one-out with thresholds thr_k[0..K-1]
-// ascending, else density at points (h_fixed > 0: one bandwidth).
+// ascending, else density at points (h_fixed > 0: one bandwidth), in the
+// index's order.
 hipError_t point_plan(hipStream_t s, const PointIndex &idx, float h_fixed, const double *thr_k, int K,
                       const SplitRule &rule, const WorkList &W, unsigned *host)
 {
     const int nw = (int)((idx.n + 63) / 64);
     const double *lim_dev = thr_k ? thr_k + (K - 1) : nullptr;
     const double lim_fixed = !thr_k && h_fixed > 0.0f ? 9.0 * (double)(float)(h_fixed * h_fixed) : 0.0;
-    hipLaunchKernelGGL(k_wave_cost, dim3((unsigned)((nw + 3) / 4)), dim3(256), 0, s, idx, lim_fixed, lim_dev, W.cost);
+    if (idx.grp) hipLaunchKernelGGL(k_fine_cost, dim3((unsigned)((nw + 3) / 4)), dim3(256), 0, s, idx, W.cost);
+    else hipLaunchKernelGGL(k_wave_cost, dim3((unsigned)((nw + 3) / 4)), dim3(256), 0, s, idx, lim_fixed, lim_dev, W.cost);
     hipLaunchKernelGGL(k_work_scan, dim3(1), dim3(1024), 0, s, nw, rule, W, host);
     return hipGetLastError();
 }
 
 // n_items_dev non-null (here and in loo_multi): the item count is read on the
 // device and n_items is only the grid bound.
-hipError_t point_density(hipStream_t s, const PointIndex &idx, int loo, float *den_sorted, float h_fixed,
-                         const int *order, const int4 *items, const unsigned *cost, double *partials, int n_items,
-                         const unsigned *n_items_dev)
+// fine: the index is in fine order and res is scratch for n floats; else one
+// bandwidth h_fixed > 0, the query itself included.
+hipError_t point_density(hipStream_t s, const PointIndex &idx, bool fine, int loo, float *den_sorted, float *res,
+                         float h_fixed, const int *order, const int4 *items, const unsigned *cost,
+                         double *partials, int n_items, const unsigned *n_items_dev)
 {
-    PtsArgs A{idx, den_sorted, loo, 0.0, 0.0, order, items, cost, partials, n_items, n_items_dev};
+    PtsArgs A{idx, den_sorted, res, 0.0, 0.0, order, items, cost, partials, n_items, n_items_dev};
     if (idx.n <= 0) return hipSuccess;
     const int64_t units = order ? n_items : (idx.n + 63) / 64;
     const unsigned grid = (unsigned)((units + 3) / 4);
-    if (h_fixed > 0.0f) {
+    if (fine) {
+        if (loo) {
+            hipLaunchKernelGGL(k_group_density_f<true>, dim3(grid), dim3(256), 0, s, A);
+            hipLaunchKernelGGL(k_point_density_f<true>, dim3(grid), dim3(256), 0, s, A);
+        } else {
+            hipLaunchKernelGGL(k_group_density_f<false>, dim3(grid), dim3(256), 0, s, A);
+            hipLaunchKernelGGL(k_point_density_f<false>, dim3(grid), dim3(256), 0, s, A);
+        }
+    } else {
+        if (loo || !(h_fixed > 0.0f)) return hipErrorInvalidValue;
         const double h2 = (double)(float)(h_fixed * h_fixed);
         A.thr_fixed = 9.0 * h2;
         A.a_fixed = -MKDE_LOG2E / (2.0 * h2);
-        if (loo) hipLaunchKernelGGL(HIP_KERNEL_NAME(k_point_density_w<true, true>), dim3(grid), dim3(256), 0, s, A);
-        else hipLaunchKernelGGL(HIP_KERNEL_NAME(k_point_density_w<true, false>), dim3(grid), dim3(256), 0, s, A);
-    } else {
-        if (loo) hipLaunchKernelGGL(HIP_KERNEL_NAME(k_point_density_w<false, true>), dim3(grid), dim3(256), 0, s, A);
-        else hipLaunchKernelGGL(HIP_KERNEL_NAME(k_point_density_w<false, false>), dim3(grid), dim3(256), 0, s, A);
+        hipLaunchKernelGGL(k_pilot_density, dim3(grid), dim3(256), 0, s, A);
     }
     return hipGetLastError();
 }
