@@ -62,7 +62,7 @@ hipError_t fine_points(hipStream_t, int64_t, const float *, const float *, const
 hipError_t valid_cells(hipStream_t, int64_t, const float *, float, uint8_t *);
 hipError_t runs_count(hipStream_t, const GridDesc &, const uint8_t *, unsigned *, unsigned *, unsigned *, unsigned *,
                       int64_t *);
-hipError_t runs_fill(hipStream_t, const GridDesc &, const uint8_t *, const unsigned *, int2 *);
+hipError_t runs_fill(hipStream_t, const GridDesc &, const uint8_t *, const unsigned *, int2 *, int2 *);
 hipError_t boundary(hipStream_t, const GridDesc &, const uint8_t *, uint8_t *, float2 *, unsigned long long *);
 hipError_t dist_boundary(hipStream_t, int64_t, const float *, const float *, const float2 *, int64_t, double *);
 int64_t bt_level_size(const BndTree &, int);
@@ -227,7 +227,7 @@ struct mkde_ctx {
     DevBuf<float> mask;
     DevBuf<uint8_t> valid;
     DevBuf<int64_t> run_ptr;
-    DevBuf<int2> run_se;
+    DevBuf<int2> run_se, row_run;
     DevBuf<unsigned> run_cnt, run_first, run_chunks, run_total;   // building the runs
     DevBuf<float> colx, rowy;   // cell-centre tables of the mask grid
     DevBuf<uint8_t> bflags;
@@ -747,6 +747,7 @@ extern "C" int mkde_mask_upload(mkde_ctx *c, const mkde_grid *g, const float *va
     CHK(c->valid.ensure(nc));
     CHK(c->bflags.ensure(nc));
     CHK(c->run_ptr.ensure(g->nrows + 1));
+    CHK(c->row_run.ensure(g->nrows));
     CHK(c->run_cnt.ensure(g->nrows));
     CHK(c->run_first.ensure(g->nrows));
     CHK(c->run_chunks.ensure((g->nrows + 1023) / 1024));
@@ -763,7 +764,7 @@ extern "C" int mkde_mask_upload(mkde_ctx *c, const mkde_grid *g, const float *va
     unsigned nruns = 0;
     CHK(copy_d2h(c, &nruns, c->run_total.p, sizeof nruns));
     CHK(c->run_se.ensure(std::max<int64_t>(nruns, 1)));
-    HIPCHK(mkde_dev::runs_fill(c->stream, gd, c->valid.p, c->run_first.p, c->run_se.p));
+    HIPCHK(mkde_dev::runs_fill(c->stream, gd, c->valid.p, c->run_first.p, c->run_se.p, c->row_run.p));
     HIPCHK(mkde_dev::centres(c->stream, gd, c->colx.p, c->rowy.p));
     HIPCHK(hipStreamSynchronize(c->stream));
     c->mg = gd;
@@ -975,7 +976,7 @@ static int run_ec(mkde_ctx *c, const float *h, float hf, float *ew_out, unsigned
                                ec_wide_cols(c, hf)));
     int cnt3[3] = {0, 0, 0};   // narrow points, wide points, widest box
     CHK(copy_d2h(c, cnt3, c->icount.p, sizeof cnt3));
-    MaskRuns R{c->run_ptr.p, c->run_se.p};
+    MaskRuns R{c->run_ptr.p, c->run_se.p, c->row_run.p};
     HIPCHK(hipEventRecord(c->ev0, c->stream));
     HIPCHK(mkde_dev::ec(c->stream, c->n, cnt3[0], cnt3[1], cnt3[2], c->mg, R, c->colx.p, c->rowy.p, c->x.p, c->y.p,
                         h, hf, c->list.p, ew_out, c->ucount.p, c->tune.ec_chunk, c->mg_cx32));
@@ -1290,7 +1291,7 @@ static int search_enqueue(mkde_ctx *c, int K, int ec_on, const PointIndex &I, in
                           const WorkList &W, const std::vector<int> &wcols)
 {
     const int64_t n = c->n;
-    MaskRuns R{c->run_ptr.p, c->run_se.p};
+    MaskRuns R{c->run_ptr.p, c->run_se.p, c->row_run.p};
     const SplitRule rule = mkde_dev::point_rule(1, c->tune, true);
     if (!ec_on) HIPCHK(mkde_dev::fill_f32(c->stream, n, 1.0f, c->ewk.p));
     const int nb = (int)std::min<int64_t>(1024, (n + 255) / 256);
@@ -1381,7 +1382,8 @@ static int loo_loglik_graph(mkde_ctx *c, int K, const std::vector<int> &ord, con
                               (uint64_t)(uintptr_t)c->y.p, (uint64_t)(uintptr_t)c->w.p,
                               (uint64_t)(uintptr_t)c->perm.p, (uint64_t)(uintptr_t)c->dist.p,
                               (uint64_t)(uintptr_t)c->mask.p, (uint64_t)(uintptr_t)c->run_ptr.p,
-                              (uint64_t)(uintptr_t)c->run_se.p, (uint64_t)(uintptr_t)c->colx.p,
+                              (uint64_t)(uintptr_t)c->run_se.p, (uint64_t)(uintptr_t)c->row_run.p,
+                              (uint64_t)(uintptr_t)c->colx.p,
                               (uint64_t)(uintptr_t)c->rowy.p, (uint64_t)c->mg.ncols, (uint64_t)c->mg.nrows,
                               (uint64_t)__builtin_bit_cast(uint32_t, c->mg.xll),
                               (uint64_t)__builtin_bit_cast(uint32_t, c->mg.yll),
@@ -1829,7 +1831,7 @@ extern "C" int mkde_count_density_pairs(mkde_ctx *c, const mkde_grid *tile, cons
     const int64_t nw = mkde_dev::slot_words();
     CHK(c->ucount.ensure(nw));
     HIPCHK(hipMemsetAsync(c->ucount.p, 0, nw * sizeof(unsigned long long), c->stream));
-    MaskRuns MR{rp.p, rs.p};
+    MaskRuns MR{rp.p, rs.p, nullptr};   // pairs are counted from the run lists
     PointIndex I = index_of(c);
     GridDesc g = to_desc(tile);
     HIPCHK(mkde_dev::count_pairs(c->stream, g, MR, I, c->ucount.p));

@@ -177,7 +177,10 @@ __host__ __device__ inline int64_t bt_node(int ix, int iy, int pnx)
 
 // Per-row runs of valid cells of a mask (CSR): runs of row r are
 // run_se[run_ptr[r] .. run_ptr[r+1]), each (start, end) inclusive, ascending.
+// row_run[r] is the run of a row with one, (1, 0) for a row without, and
+// (-1, 0) for a row with more.
 struct MaskRuns {
     const int64_t *run_ptr;
     const int2 *run_se;
+    const int2 *row_run;
 };
