@@ -44,13 +44,15 @@ hipError_t density_tile(hipStream_t, const GridDesc &, const float *, float *, c
                         const Tiling &);
 hipError_t density_merge(hipStream_t, const GridDesc &, const Tiling &, const float *, int, const int4 *,
                          const double *, float *);
-SplitRule point_rule(int, const Tuning &, bool);
+SplitRule point_rule(int, const Tuning &, bool, bool);
 hipError_t point_plan(hipStream_t, const PointIndex &, float, const double *, int, const SplitRule &,
                       const WorkList &, unsigned *);
 hipError_t point_density(hipStream_t, const PointIndex &, bool, int, float *, float *, float, const int *, const int4 *,
                          const unsigned *, double *, int, const unsigned *);
 hipError_t loo_multi(hipStream_t, const PointIndex &, const float *, const double *, const double *, int, float *,
                      const int *, const int4 *, const unsigned *, double *, int, const unsigned *);
+hipError_t loo_density(hipStream_t, const PointIndex &, float *, const int *, const int4 *, const unsigned *, double *,
+                       int, const unsigned *);
 hipError_t point_merge(hipStream_t, int64_t, int, int, int, const int4 *, const double *, float *, const unsigned *);
 hipError_t range_count(hipStream_t, const PointIndex &, int64_t *);
 hipError_t range_fill(hipStream_t, const PointIndex &, const int64_t *, int32_t *);
@@ -91,8 +93,8 @@ hipError_t sumlog(hipStream_t, int64_t, int, const float *, int, double *, int, 
 hipError_t abramson(hipStream_t, int64_t, const int *, const float *, const double *, float, float, float *);
 hipError_t unsort_f32(hipStream_t, int64_t, const int *, const float *, float *);
 hipError_t sort_f32(hipStream_t, int64_t, const int *, const float *, float *);
-hipError_t coef_k(hipStream_t, int64_t, const int *, const float *, const float *, double, float *, int);
-hipError_t coef_k_dev(hipStream_t, int64_t, const int *, const float *, const float *, const float *, float *, int);
+hipError_t coef_k(hipStream_t, int64_t, const int *, const float *, const float *, double, float *);
+hipError_t coef_k_dev(hipStream_t, int64_t, const int *, const float *, const float *, const float *, float *);
 hipError_t fill_f32(hipStream_t, int64_t, float, float *);
 hipError_t scratch_address(int, void **);
 }  // namespace mkde_dev
@@ -881,7 +883,6 @@ static int ensure_dist(mkde_ctx *c)
     CHK(ensure_boundary(c));
     CHK(ensure_btree(c));
     if (c->bt.nlev > 0) {
-        CHK(prep(c));
         HIPCHK(mkde_dev::dist_tree(c->stream, c->n, c->xs.p, c->ys.p, c->perm.p, c->mg, c->bt, c->dist.p));
     } else {
         CHK(boundary_count(c));
@@ -1099,7 +1100,7 @@ static int plan_points(mkde_ctx *c, const PointIndex &I, int loo, float h_fixed,
     if (nw == 0) return MKDE_OK;
     WorkList W;
     CHK(point_list(c, nw, W));
-    const SplitRule rule = mkde_dev::point_rule(loo, c->tune, thr_k != nullptr);
+    const SplitRule rule = mkde_dev::point_rule(loo, c->tune, thr_k != nullptr, !I.grp);
     int64_t items_max = 0, slots_max = 0;
     point_work_bounds(c->n, rule, &items_max, &slots_max);
     const bool dev = slots_max * 64 * m * (int64_t)sizeof(double) <= MKDE_POINT_DEV_PARTIALS;
@@ -1128,6 +1129,24 @@ static int plan_points(mkde_ctx *c, const PointIndex &I, int loo, float h_fixed,
 // The order a point density runs in: bin order for one bandwidth with the query
 // itself included (the pilot), else fine order.
 static bool density_fine(const mkde_ctx *c, int loo) { return loo || !(c->h_fixed > 0.0f); }
+
+// Leave-one-out densities in bin order, for the log-likelihoods.  (Not the fine
+// order of the densities that are returned: a sum of logarithms of densities with
+// heavy-tailed weights moves by a few 1e-9 with the order of the float sums.)
+static int loo_density_binned(mkde_ctx *c, float *den_sorted)
+{
+    CHK(prep(c));
+    PointIndex I = index_of(c);
+    HIPCHK(hipEventRecord(c->ev0, c->stream));
+    PointWork P;
+    CHK(plan_points(c, I, 1, 0.0f, nullptr, 0, 1, P));
+    HIPCHK(mkde_dev::loo_density(c->stream, I, den_sorted, P.order, P.items, c->pw_cost.p,
+                                 c->pw_partials.p, P.n_items, P.n_items_dev));
+    HIPCHK(mkde_dev::point_merge(c->stream, c->n, 1, 1, P.n_split, c->pw_splits.p, c->pw_partials.p, den_sorted,
+                                 P.n_split_dev));
+    HIPCHK(hipEventRecord(c->ev1, c->stream));
+    return MKDE_OK;
+}
 
 // Densities at the points in that order.
 static int density_points_sorted(mkde_ctx *c, int loo, float *den_sorted)
@@ -1214,7 +1233,7 @@ extern "C" int mkde_density_at_points_noalloc(mkde_ctx *c, int loo, float *den_d
     CHK(prep(c, fine));
     PointIndex I = index_of(c);
     const WorkList W{cost, item0, slot0, sidx, counts, hist};
-    HIPCHK(mkde_dev::point_plan(c->stream, I, c->h_fixed, nullptr, 0, mkde_dev::point_rule(loo ? 1 : 0, c->tune, false),
+    HIPCHK(mkde_dev::point_plan(c->stream, I, c->h_fixed, nullptr, 0, mkde_dev::point_rule(loo ? 1 : 0, c->tune, false, !I.grp),
                                 W, c->host_words));
     HIPCHK(hipStreamSynchronize(c->stream));
     const unsigned cnt[3] = {c->host_words[0], c->host_words[1], c->host_words[2]};   // items, slots, split waves
@@ -1292,7 +1311,7 @@ static int search_enqueue(mkde_ctx *c, int K, int ec_on, const PointIndex &I, in
 {
     const int64_t n = c->n;
     MaskRuns R{c->run_ptr.p, c->run_se.p, c->row_run.p};
-    const SplitRule rule = mkde_dev::point_rule(1, c->tune, true);
+    const SplitRule rule = mkde_dev::point_rule(1, c->tune, true, true);
     if (!ec_on) HIPCHK(mkde_dev::fill_f32(c->stream, n, 1.0f, c->ewk.p));
     const int nb = (int)std::min<int64_t>(1024, (n + 255) / 256);
     for (int g0 = 0, gi = 0; g0 < K; g0 += MKDE_LM_K, ++gi) {
@@ -1308,11 +1327,10 @@ static int search_enqueue(mkde_ctx *c, int K, int ec_on, const PointIndex &I, in
                                         c->icount.p, c->list.p, c->ewk.p, c->tune.ec_chunk, cw_narrow,
                                         wcols[g0 + j], c->mg_cx32));
             }
-            HIPCHK(mkde_dev::coef_k_dev(c->stream, n, c->perm.p, c->w.p, c->ewk.p, hd,
-                                        c->coefk.p + (MKDE_LM_K - kg) + j, MKDE_LM_K));
+            HIPCHK(mkde_dev::coef_k_dev(c->stream, n, c->perm.p, c->w.p, c->ewk.p, hd, c->coefk.p + (int64_t)j * n));
         }
         const double *a = c->s_a.p + (int64_t)gi * MKDE_LM_K, *t = c->s_t.p + (int64_t)gi * MKDE_LM_K;
-        HIPCHK(mkde_dev::point_plan(c->stream, I, 0.0f, t, MKDE_LM_K, rule, W, nullptr));
+        HIPCHK(mkde_dev::point_plan(c->stream, I, 0.0f, t, kg, rule, W, nullptr));
         HIPCHK(mkde_dev::work_items(c->stream, (int)nw, W, c->pw_items.p, c->pw_splits.p, c->pw_order.p));
         HIPCHK(mkde_dev::loo_multi(c->stream, I, c->coefk.p, a, t, kg, c->den1k.p, c->pw_order.p, c->pw_items.p,
                                    c->pw_cost.p, c->pw_partials.p, (int)items_max, c->pw_counts.p));
@@ -1331,7 +1349,7 @@ static int loo_loglik_graph(mkde_ctx *c, int K, const std::vector<int> &ord, con
     *done = false;
     const int64_t n = c->n, nw = (n + 63) / 64;
     int64_t items_max = 0, slots_max = 0;
-    point_work_bounds(n, mkde_dev::point_rule(1, c->tune, true), &items_max, &slots_max);
+    point_work_bounds(n, mkde_dev::point_rule(1, c->tune, true, true), &items_max, &slots_max);
     if (slots_max * 64 * MKDE_LM_K * (int64_t)sizeof(double) > MKDE_SEARCH_GRAPH_MAX_PARTIALS) return MKDE_OK;
     const int G = (K + MKDE_LM_K - 1) / MKDE_LM_K;
     // every buffer the graph touches, at its final size, before any capture
@@ -1355,9 +1373,9 @@ static int loo_loglik_graph(mkde_ctx *c, int K, const std::vector<int> &ord, con
     CHK(c->pw_partials.ensure((size_t)slots_max * 64 * MKDE_LM_K));
     const int nb = (int)std::min<int64_t>(1024, (n + 255) / 256);
     CHK(c->partial.ensure((size_t)nb * MKDE_LM_K));
-    // the device inputs of this search: candidates ascending, slot constants
+    // the device inputs of this search: candidates ascending and their constants
     std::vector<float> hs(K);
-    std::vector<double> a((size_t)G * MKDE_LM_K, 0.0), t((size_t)G * MKDE_LM_K, -1.0);
+    std::vector<double> a((size_t)G * MKDE_LM_K, 0.0), t((size_t)G * MKDE_LM_K, 0.0);
     for (int k = 0; k < K; ++k) hs[k] = h_cand[ord[k]];
     // each candidate's widest wide EC box: the LDS of its wide launch (part
     // of the key, so new candidates that need other sizes recapture)
@@ -1367,8 +1385,8 @@ static int loo_loglik_graph(mkde_ctx *c, int K, const std::vector<int> &ord, con
         const int kg = std::min(MKDE_LM_K, K - g0);
         for (int j = 0; j < kg; ++j) {
             const double h2 = (double)(float)(hs[g0 + j] * hs[g0 + j]);
-            a[(size_t)gi * MKDE_LM_K + MKDE_LM_K - kg + j] = -1.4426950408889634073599 / (2.0 * h2);
-            t[(size_t)gi * MKDE_LM_K + MKDE_LM_K - kg + j] = 9.0 * h2;
+            a[(size_t)gi * MKDE_LM_K + j] = -1.4426950408889634073599 / (2.0 * h2);
+            t[(size_t)gi * MKDE_LM_K + j] = 9.0 * h2;
         }
     }
     CHK(copy_h2d(c, c->s_h.p, hs.data(), K * sizeof(float)));
@@ -1467,7 +1485,7 @@ extern "C" int mkde_loo_loglik(mkde_ctx *c, int K, const float *h_cand, int ec_o
     }
     PointIndex I = index_of(c);
     const int G = std::min(K, MKDE_LM_K);
-    CHK(c->coefk.ensure((size_t)MKDE_LM_K * n));   // [n][MKDE_LM_K]: a point's candidate slots contiguous
+    CHK(c->coefk.ensure((size_t)G * n));
     CHK(c->den1k.ensure((size_t)G * n));
     CHK(c->ewk.ensure(n));
     CHK(c->ak.ensure(MKDE_LM_K));
@@ -1476,26 +1494,22 @@ extern "C" int mkde_loo_loglik(mkde_ctx *c, int K, const float *h_cand, int ec_o
     std::vector<double> res(K);
     for (int g0 = 0; g0 < K; g0 += MKDE_LM_K) {
         const int kg = std::min(MKDE_LM_K, K - g0);
-        // the pass's kg candidates (ascending) in slots MKDE_LM_K - kg ..
-        // MKDE_LM_K - 1; the slots below hold a threshold no pair passes
-        std::vector<double> a(MKDE_LM_K, 0.0), t(MKDE_LM_K, -1.0);
+        std::vector<double> a(MKDE_LM_K, 0.0), t(MKDE_LM_K, 0.0);
         for (int j = 0; j < kg; ++j) {
             const float hk = h_cand[ord[g0 + j]];
             const double h2 = (double)(float)(hk * hk);
-            a[MKDE_LM_K - kg + j] = -1.4426950408889634073599 / (2.0 * h2);
-            t[MKDE_LM_K - kg + j] = 9.0 * h2;
+            a[j] = -1.4426950408889634073599 / (2.0 * h2);
+            t[j] = 9.0 * h2;
             if (ec_on) CHK(run_ec(c, nullptr, hk, c->ewk.p, nullptr));
             else HIPCHK(mkde_dev::fill_f32(c->stream, n, 1.0f, c->ewk.p));
-            // candidate j of this pass in coefficient slot MKDE_LM_K - kg + j
-            HIPCHK(mkde_dev::coef_k(c->stream, n, c->perm.p, c->w.p, c->ewk.p, h2, c->coefk.p + (MKDE_LM_K - kg) + j,
-                                    MKDE_LM_K));
+            HIPCHK(mkde_dev::coef_k(c->stream, n, c->perm.p, c->w.p, c->ewk.p, h2, c->coefk.p + (int64_t)j * n));
         }
         CHK(copy_h2d(c, c->ak.p, a.data(), MKDE_LM_K * sizeof(double)));
         CHK(copy_h2d(c, c->tk.p, t.data(), MKDE_LM_K * sizeof(double)));
         HIPCHK(hipEventRecord(c->ev0, c->stream));
         PointWork P;
-        // the work estimate culls with the largest threshold (the top slot)
-        CHK(plan_points(c, I, 1, 0.0f, c->tk.p, MKDE_LM_K, MKDE_LM_K, P));
+        // the work estimate culls with the largest threshold
+        CHK(plan_points(c, I, 1, 0.0f, c->tk.p, kg, MKDE_LM_K, P));
         HIPCHK(mkde_dev::loo_multi(c->stream, I, c->coefk.p, c->ak.p, c->tk.p, kg, c->den1k.p, P.order, P.items,
                                    c->pw_cost.p, c->pw_partials.p, P.n_items, P.n_items_dev));
         HIPCHK(mkde_dev::point_merge(c->stream, n, MKDE_LM_K, kg, P.n_split, c->pw_splits.p, c->pw_partials.p,
@@ -1575,7 +1589,7 @@ extern "C" int mkde_loo_loglik_adaptive(mkde_ctx *c, int K, const float *h, cons
         CHK(abramson_core(c, h[k], alpha[k], ec_on));
         if (ec_on) CHK(run_ec(c, c->h.p, 0.0f, c->ew.p, nullptr));
         c->pts_dirty = true;
-        CHK(density_points_sorted(c, 1, c->den.p));
+        CHK(loo_density_binned(c, c->den.p));
         CHK(sum_logs(c, c->den.p, 1, 1, c->dsum.p));
         CHK(copy_d2h(c, &logL[k], c->dsum.p, sizeof(double)));
     }

@@ -43,10 +43,13 @@ struct SplitRule {
 
 // Smallest split threshold of the point work lists (candidate sources per part).
 #define MKDE_PTS_TMIN 4096u
-// Leave-one-out lists: smaller parts while they are at most 4096 (a search on
-// 2,000 points is 32 waves: 0.90 ms for its pass uncut, 0.13 ms in parts of 256).
+// Leave-one-out lists in fine order: smaller parts while they are at most 4096.
 #define MKDE_LOO_FEW_TMIN 256u
 #define MKDE_LOO_FEW 4096ull
+// The batched pass gives each wave fewer candidates until it has this many waves.
+#define MKDE_LOO_WAVES 4096
+// Lists of at most so many waves (times candidates) run with 16 queries a wave.
+#define MKDE_SUM_SHORT 8192
 
 // Most items and split parts a point work list of nw 64-query waves can have:
 // each wave's cost is at most n sources, so split parts <= min(target, total /

@@ -7,10 +7,10 @@
 //   k_ec              per-point edge-correction integral, O(R) per point
 //                     (replaces CalcEdgeCorrectionWeights kde_kernel_kdtr.cu:117-265
 //                     and EdgeCorrectionWeightsExact tiled:2694-2807)
-//   k_pilot_density, k_point_density_f   density at points over the cell-binned
+//   k_point_sums, k_point_density_f   density at points over the cell-binned
 //                     index, pilot and leave-one-out forms (replaces DensityAtPointsKdtr
 //                     kde_kernel_kdtr.cu:681-953 and the CPU scatter tiled:3312-3347)
-//   k_loo_multi_w     leave-one-out densities of up to 16 fixed bandwidths in one
+//   k_loo_multi       leave-one-out densities of up to 16 fixed bandwidths in one
 //                     pass over point pairs (batched LogLikelihood, tiled:3214-3368)
 //   k_boundary, k_dist_boundary   MarkBoundary / CalcDist2Boundary
 //                     (kde_kernel_kdtr.cu:1209-1353, tiled:3993-4131)
@@ -184,6 +184,17 @@ __global__ void k_prep_points(int64_t n, const int *perm, const float *xs, const
     out[i] = r;
 }
 
+// A float squared distance below lo is inside the cut-off thr, one above hi is
+// not.  fl32(dx^2 + dy^2) is within 2^-22 relative where it neither overflows nor
+// becomes subnormal; elsewhere nothing is taken as decided (lo = -1, a hi that
+// holds for every distance in doubt).  thr < 0: nothing is inside.
+__device__ __forceinline__ void thr_bracket(double thr, float &lo, float &hi)
+{
+    const bool plain = thr > 1e-30 && thr < 1e37;
+    lo = plain ? (float)(thr * (1.0 - 1.0 / 1048576.0)) : -1.0f;
+    hi = plain ? (float)(thr * (1.0 + 1.0 / 1048576.0)) : thr > 1.0 ? INFINITY : thr < 0.0 ? -1.0f : 1e-29f;
+}
+
 // The same in fine order (SrcRec, one wave per group of 64), with each group's
 // box and thresholds.
 __global__ __launch_bounds__(256) void k_prep_fine(int64_t n, const int *perm, const float *xs, const float *ys,
@@ -206,12 +217,7 @@ __global__ __launch_bounds__(256) void k_prep_fine(int64_t n, const int *perm, c
             r.coef = (float)((double)w_orig[o] * (double)ew_orig[o] / (h2 * (double)MKDE_TWO_PI_F));
             r.af = (float)(-MKDE_LOG2E / (2.0 * h2));
             r.thr = 9.0 * h2;
-            // fl32(dx^2 + dy^2) is within 2^-22 relative where it neither
-            // overflows nor becomes subnormal; elsewhere nothing is taken as
-            // decided (lo = -1, a hi that holds for every distance in doubt)
-            const bool plain = r.thr > 1e-30 && r.thr < 1e37;
-            r.lo = plain ? (float)(r.thr * (1.0 - 1.0 / 1048576.0)) : -1.0f;
-            r.hi = plain ? (float)(r.thr * (1.0 + 1.0 / 1048576.0)) : r.thr > 1.0 ? INFINITY : 1e-29f;
+            thr_bracket(r.thr, r.lo, r.hi);
         }
         out[i] = r;
     }
@@ -1151,14 +1157,13 @@ __global__ void k_scan_add(int n, unsigned *out, const unsigned *chunk_sums)
 
 // ==================================================== density at points ====
 //
-// One wave owns 64 consecutive query points (lane = query) and walks the
-// candidate bins of its bounding box; a source's record is wave-uniform and
-// comes in by scalar loads.  Two forms:
-//   k_pilot_density    one bandwidth, the query itself included, bin order: the
-//                      densities the adaptive bandwidths come from
-//   k_point_density_f  every other case (a bandwidth per source, leave-one-out),
-//                      fine order, with sums over whole groups of sources
-// Duplicates at distance 0 are kept in both.  Waves run heaviest first
+// One wave owns consecutive query points (lane = query) and walks the candidate
+// bins of its bounding box; every source is taken up by the whole wave at once.
+//   k_point_sums, k_loo_multi   bin order: pilot densities, and the leave-one-out
+//                      densities whose logarithms are summed
+//   k_point_density_f  fine order: the densities that are an output (a bandwidth
+//                      per source, leave-one-out), with sums over whole groups
+// Duplicates at distance 0 are kept.  Waves run heaviest first
 // (k_wave_cost).
 //
 // Cut-off test: d2f = fl32(dx*dx + dy*dy) decides unless it lies within a
@@ -1170,7 +1175,6 @@ struct PtsArgs {
     PointIndex idx;
     float *den;   // output, the index's order
     float *res;   // n floats of scratch (fine order)
-    double thr_fixed, a_fixed;   // k_pilot_density only
     // work items (nullable order: one item per wave): {wave, part j, parts K,
     // partial slot}; part j of a wave takes candidate ordinals
     // [C j / K, C (j+1) / K) of its C candidate sources (cost[wave])
@@ -1182,7 +1186,13 @@ struct PtsArgs {
     const unsigned *n_items_dev;   // non-null: the item count on the device (n_items: grid bound)
 };
 
-#define PD_BAND (1.0 / 1048576.0)
+// Orders LDS accesses of the lanes of one wave (its LDS operations complete in
+// order, so only the compiler has to keep them).
+__device__ __forceinline__ void wave_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
 
 __device__ __forceinline__ float wave_min(float v)
 {
@@ -1238,129 +1248,6 @@ __global__ __launch_bounds__(256) void k_wave_cost(PointIndex I, double lim_fixe
     }
     for (int d = 32; d >= 1; d >>= 1) acc += __shfl_xor(acc, d, WAVE);
     if (lane == 0) cost[wv] = acc;
-}
-
-// Pilot densities at one bandwidth.  Kept as it is, operation by operation: the
-// adaptive bandwidths h_i follow from these sums, and a bandwidth that moves by
-// one rounding takes pairs across the hard cut-off.
-__global__ __launch_bounds__(256) void k_pilot_density(PtsArgs A)
-{
-    const PointIndex &I = A.idx;
-    const int lane = threadIdx.x & 63;
-    // the wave index and the work item are wave-uniform: made explicit so the
-    // source records below are read with scalar loads
-    const int64_t g = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int64_t units = A.n_items_dev ? (int64_t)*A.n_items_dev : A.order ? (int64_t)A.n_items : (I.n + 63) / 64;
-    if (g >= units) return;   // whole wave
-    const int4 item = uniform_item(A.order ? A.items[A.order[g]] : make_int4((int)g, 0, 1, -1));
-    int win0 = 0, win1 = INT_MAX;   // candidate counts are below 2^31
-    if (item.z > 1) {
-        const int64_t C = A.cost[item.x];
-        if (item.y > 0) win0 = (int)(C * item.y / item.z);
-        if (item.y < item.z - 1) win1 = (int)(C * (item.y + 1) / item.z);
-    }
-    const int64_t q0 = (int64_t)item.x * 64;
-    const int64_t q = q0 + lane;
-    const bool qv = q < I.n;
-    float qx = 0.0f, qy = 0.0f;
-    if (qv) {
-        const PtRec p = I.pts[q];
-        qx = p.x;
-        qy = p.y;
-    }
-    const float mnx = uni(wave_min(qv ? qx : FLT_MAX)), mxx = uni(wave_max(qv ? qx : -FLT_MAX));
-    const float mny = uni(wave_min(qv ? qy : FLT_MAX)), mxy = uni(wave_max(qv ? qy : -FLT_MAX));
-    const double reach = sqrt(fmax(A.thr_fixed, 0.0)) * 1.000001 + 1e-6;
-    int bxa, bxb, bya, byb;
-    bin_range(I.bg, mnx, mxx, mny, mxy, reach, bxa, bxb, bya, byb);
-    bxa = __builtin_amdgcn_readfirstlane(bxa);
-    bxb = __builtin_amdgcn_readfirstlane(bxb);
-    bya = __builtin_amdgcn_readfirstlane(bya);
-    byb = __builtin_amdgcn_readfirstlane(byb);
-
-    const float f_thr_lo = (float)(A.thr_fixed * (1.0 - PD_BAND));
-    const float f_thr_hi = fmaxf((float)(A.thr_fixed * (1.0 + PD_BAND)), FLT_MIN);
-    const float f_a = (float)A.a_fixed;
-    float acc = 0.0f, sum = 0.0f, comp = 0.0f;
-    int ord = 0;   // candidate ordinal at the start of the next candidate bin
-    for (int by = bya; by <= byb; ++by) {
-        for (int bx = bxa; bx <= bxb; ++bx) {
-            const int b = by * I.bg.nbx + bx;
-            const int bst = I.bin_start[b], ben = I.bin_start[b + 1];
-            if (bst == ben) continue;
-            const BinInfo bb = I.bin_box[b];
-            if (!__builtin_amdgcn_readfirstlane((int)(box_gap2(bb, mnx, mxx, mny, mxy) < A.thr_fixed))) continue;
-            // every pair of the bin and the wave is inside the screen when the
-            // largest fl32 offsets give d2f below it (fl32 of a difference,
-            // the product and the fma are monotone in |offset|, so no pair's
-            // d2f exceeds this one): such a bin's sources need no compare and
-            // no select, and add the same terms
-            const float gx = fmaxf(bb.x1 - mnx, mxx - bb.x0), gy = fmaxf(bb.y1 - mny, mxy - bb.y0);
-            const bool all_in = __builtin_amdgcn_readfirstlane((int)(__builtin_fmaf(gy, gy, gx * gx) < f_thr_lo));
-            // this part's share of the candidate sequence
-            const int o0 = ord, o1 = ord + (ben - bst);
-            ord = o1;
-            if (o1 <= win0 || o0 >= win1) continue;
-            const int st = bst + (win0 > o0 ? win0 - o0 : 0);
-            const int en = ben - (o1 > win1 ? o1 - win1 : 0);
-            for (int c0 = st; c0 < en; c0 += 32) {
-                const int c1 = c0 + 32 < en ? c0 + 32 : en;
-                // four records are loaded before their arithmetic, so the
-                // scalar loads overlap
-                if (all_in) {
-                    int si = c0;
-                    for (; si + 4 <= c1; si += 4) {
-                        const PtRec p0 = I.pts[si], p1 = I.pts[si + 1], p2 = I.pts[si + 2], p3 = I.pts[si + 3];
-                        for (const PtRec &p : {p0, p1, p2, p3}) {
-                            const float dx = p.x - qx, dy = p.y - qy;
-                            const float d2f = __builtin_fmaf(dy, dy, dx * dx);
-                            acc = __builtin_fmaf(fast_exp2(d2f * f_a), p.coef, acc);
-                        }
-                    }
-                    for (; si < c1; ++si) {
-                        const PtRec p = I.pts[si];
-                        const float dx = p.x - qx, dy = p.y - qy;
-                        const float d2f = __builtin_fmaf(dy, dy, dx * dx);
-                        acc = __builtin_fmaf(fast_exp2(d2f * f_a), p.coef, acc);
-                    }
-                } else {
-                    bool band = false;
-                    auto body = [&](const PtRec &p) {
-                        const float dx = p.x - qx, dy = p.y - qy;
-                        const float d2f = __builtin_fmaf(dy, dy, dx * dx);
-                        const bool in = d2f < f_thr_lo;
-                        band |= (d2f < f_thr_hi) != in;
-                        const float e = fast_exp2(d2f * f_a);
-                        acc = __builtin_fmaf(in ? e : 0.0f, p.coef, acc);
-                    };
-                    int si = c0;
-                    for (; si + 4 <= c1; si += 4) {
-                        const PtRec p0 = I.pts[si], p1 = I.pts[si + 1], p2 = I.pts[si + 2], p3 = I.pts[si + 3];
-                        body(p0);
-                        body(p1);
-                        body(p2);
-                        body(p3);
-                    }
-                    for (; si < c1; ++si) body(I.pts[si]);
-                    if (__any(band)) {   // rare: exact FP64 test for the chunk
-                        acc = 0.0f;
-                        for (int sj = c0; sj < c1; ++sj) {
-                            const PtRec p = I.pts[sj];
-                            const float dx = p.x - qx, dy = p.y - qy;
-                            const float d2f = __builtin_fmaf(dy, dy, dx * dx);
-                            const bool in = sq2(dx, dy) < A.thr_fixed;
-                            const float e = fast_exp2(d2f * f_a);
-                            acc = __builtin_fmaf(in ? e : 0.0f, p.coef, acc);
-                        }
-                    }
-                }
-                kahan_fold(acc, sum, comp);
-                acc = 0.0f;
-            }
-        }
-    }
-    if (item.z > 1) A.partials[(int64_t)item.w * 64 + lane] = (double)sum - (double)comp;
-    else if (qv) A.den[q] = sum;
 }
 
 // Whole groups of sources.  For a group of 64 sources whose every pair with the
@@ -1689,215 +1576,400 @@ __device__ __forceinline__ int block_exscan256(int v, int *s_w, int *total)
 
 
 
-// ============================================= batched LOO (fixed bandwidths) ==
+// =================================================== point sums in bin order ==
 //
-// Up to LM_K candidate bandwidths h_k (ascending) in one pass over point
-// pairs.  coef_k of a source depends on k through the candidate's
-// edge-correction weight; a pass of K candidates keeps candidate j in slot
-// LM_K - K + j of each source's LM_K coefficients (bin order).
+// Sums at the points that are more than an output: pilot densities, from which
+// the adaptive bandwidths and so the cut-offs follow, and the leave-one-out
+// densities whose logarithms are summed (bandwidth search).  With weights of very
+// different sizes a float sum of 32 terms depends on the order of the sources, and
+// alike for all queries around, so the order is part of the result: bins row by
+// row, the caller's order within a bin, 32 sources at a time in FP32 from the
+// bin's first one (or from where a wave of many candidates is cut), these sums in
+// Kahan pairs.  What is outside the cut-off adds nothing and is left out by bins.
+// A short list fills the device by candidates and by queries, fewer per wave, not
+// by cuts.
 
 #define LM_K MKDE_LM_K
 
-struct LooMultiArgs {
-    PointIndex idx;          // positions + bins (thr of the largest candidate)
-    const float *coefk;      // [n][MKDE_LM_K] bin order, candidate j of K in slot LM_K - K + j
-    const double *a_k;       // [LM_K] by slot (0 for unused slots)
-    const double *thr_k;     // [LM_K] by slot, ascending (-1 for unused slots)
-    int K;
+struct SumArgs {
+    PointIndex idx;          // bin order; thr of the largest candidate (K bandwidths)
+    const float *coefk;      // [K][n] bin order
+    const double *a_k;       // [K]
+    const double *thr_k;     // [K] ascending
+    int K, kw;               // candidates, and how many a wave takes (blockIdx.y picks them)
+    double thr_fixed, a_fixed;   // pilot
     float *den1;             // [K][n] bin order
-    const int *order;        // work items as for the point kernel
+    // work items (nullable order: one item per wave), as for the fine-order kernels
+    const int *order;
     const int4 *items;
     const unsigned *cost;
-    double *partials;        // 64 * MKDE_LM_K per slot
+    double *partials;        // 64 * LM_K per slot (64, one density)
     int n_items;
     const unsigned *n_items_dev;   // non-null: the item count on the device (n_items: grid bound)
 };
 
-// Slots K .. K-3 of a source's candidate walk (then the next four while a
-// lane is inside): `in` is slot K's lane mask; the block forms the masks of
-// slots K-1 .. K-3 and of K-4 (the next block's first) at its start, adds
-// the four terms, without selects when every lane is inside slot K-3 (then
-// inside all four), else each term selected by its mask.  A slot no lane is
-// inside adds exp2(..) * coef selected to +0 (acc + 0 = acc), so finishing a
-// block past the last slot with a lane inside changes no sum, and the walk
-// ends after the first block whose smallest slot is empty (the cut-off is
-// monotone in h).  Two scalar tests per block instead of two per slot.  The
-// four exponentials issue before their first use, so no wait state is
-// needed after a transcendental; a mask is at least two instructions old
-// when v_cndmask reads it.
-#define MKDE_LT(I) "v_mul_f32_e32 %[t" #I "], %[d2f], %[a" #I "]\n\t"
-#define MKDE_LE(I) "v_exp_f32_e32 %[t" #I "], %[t" #I "]\n\t"
-#define MKDE_LS(I) "v_cndmask_b32_e64 %[t" #I "], 0, %[t" #I "], %[m" #I "]\n\t"
-#define MKDE_LF(I) "v_fmac_f32_e32 %[c" #I "], %[f" #I "], %[t" #I "]\n\t"
-template <int K>
-__device__ __forceinline__ void loo_block(uint64_t in, double d2, float d2f, const double (&thr)[LM_K],
-                                          const float (&af)[LM_K], const float (&cf)[LM_K], float (&acc)[LM_K])
-{
-    static_assert(K % 4 == 3, "blocks of four slots");
-    if (in == 0) return;
-    uint64_t m2, m1, m0, next = 0;
-    asm("v_cmp_gt_f64_e64 %0, %3, %6\n\t"
-        "v_cmp_gt_f64_e64 %1, %4, %6\n\t"
-        "v_cmp_gt_f64_e64 %2, %5, %6"
-        : "=&s"(m2), "=&s"(m1), "=&s"(m0)
-        : "s"(thr[K - 1]), "s"(thr[K - 2]), "s"(thr[K - 3]), "v"(d2));
-    if constexpr (K > 3) asm("v_cmp_gt_f64_e64 %0, %1, %2" : "=s"(next) : "s"(thr[K - 4]), "v"(d2));
-    // one piece of assembly for both forms (a scalar branch inside it skips
-    // the selects when every lane is inside slot K-3), so the accumulators
-    // keep their registers whichever form runs
-    float t0, t1, t2, t3;
-    asm(MKDE_LT(0) MKDE_LT(1) MKDE_LT(2) MKDE_LT(3) MKDE_LE(0) MKDE_LE(1) MKDE_LE(2) MKDE_LE(3)
-        "s_cmp_eq_u64 %[m3], -1\n\t"
-        "s_cbranch_scc1 1f\n\t"
-        MKDE_LS(0) MKDE_LS(1) MKDE_LS(2) MKDE_LS(3)
-        "\n1:\n\t"
-        MKDE_LF(0) MKDE_LF(1) MKDE_LF(2) MKDE_LF(3)
-        : [t0] "=&v"(t0), [t1] "=&v"(t1), [t2] "=&v"(t2), [t3] "=&v"(t3), [c0] "+v"(acc[K]),
-          [c1] "+v"(acc[K - 1]), [c2] "+v"(acc[K - 2]), [c3] "+v"(acc[K - 3])
-        : [d2f] "v"(d2f), [a0] "v"(af[K]), [a1] "v"(af[K - 1]), [a2] "v"(af[K - 2]), [a3] "v"(af[K - 3]),
-          [f0] "s"(cf[K]), [f1] "s"(cf[K - 1]), [f2] "s"(cf[K - 2]), [f3] "s"(cf[K - 3]), [m0] "s"(in),
-          [m1] "s"(m2), [m2] "s"(m1), [m3] "s"(m0)
-        : "scc");
-    if constexpr (K > 3) loo_block<K - 4>(next, d2, d2f, thr, af, cf, acc);
-}
+// A work item: its candidate ordinals, and its 64 queries' box.
+struct SumItem {
+    int4 item;
+    int win0, win1;
+    int q;              // this lane's query of the 64
+    bool qv;
+    float qx, qy, mnx, mxx, mny, mxy;
+};
 
-// One source of the batched leave-one-out pass for the wave's 64 queries:
-// candidate slot k's term for a lane is exp2(d2f a_k) coef_k if the exact
-// cut-off fl64(dx^2 + dy^2) < thr_k holds, else 0, added to acc[k].  Slots are
-// visited from the largest bandwidth down and the walk ends at the first one
-// no lane is inside (the cut-off is monotone in h; unused slots sit below the
-// smallest candidate with thr = -1).  selfm has the bit of the lane whose
-// query is this source (or none): that lane gets d2f = +inf, so its terms are
-// exp2(-inf) * coef = 0 (leave-one-out).  Each slot's compare and term are
-// inline assembly so that its lane mask is consumed right after it is made
-// (left to itself the compiler forms all 16 masks up front and runs out of
-// scalar registers).
-__device__ __forceinline__ void loo_source(const PtRec *pts, const float *coefk, int si, uint64_t selfm, float qx,
-                                           float qy, float inf, const double (&thr)[LM_K], const float (&af)[LM_K],
-                                           float (&acc)[LM_K])
-{
-    const PtRec p = pts[si];
-    const float4 *cp = (const float4 *)(coefk + (int64_t)si * LM_K);
-    const float4 cf0 = cp[0], cf1 = cp[1], cf2 = cp[2], cf3 = cp[3];
-    const float cf[LM_K] = {cf0.x, cf0.y, cf0.z, cf0.w, cf1.x, cf1.y, cf1.z, cf1.w,
-                            cf2.x, cf2.y, cf2.z, cf2.w, cf3.x, cf3.y, cf3.z, cf3.w};
-    const float dx = p.x - qx, dy = p.y - qy;
-    float d2f = __builtin_fmaf(dy, dy, dx * dx);
-    const double d2 = sq2(dx, dy);
-    if (selfm) asm("v_cndmask_b32_e64 %0, %0, %1, %2" : "+v"(d2f) : "v"(inf), "s"(selfm));
-    // slot k's mask is made one step ahead of its use: candidate k-1's compare
-    // issues before candidate k's term, so the scalar test of a mask never
-    // waits on the compare that made it.  The first compare also takes the
-    // source's coefficients, so their scalar loads are issued together and
-    // complete before the chain.
-    uint64_t in;
-    asm("v_cmp_gt_f64_e64 %0, %1, %2"
-        : "=s"(in)
-        : "s"(thr[LM_K - 1]), "v"(d2), "s"(cf[0]), "s"(cf[1]), "s"(cf[2]), "s"(cf[3]), "s"(cf[4]), "s"(cf[5]),
-          "s"(cf[6]), "s"(cf[7]), "s"(cf[8]), "s"(cf[9]), "s"(cf[10]), "s"(cf[11]), "s"(cf[12]), "s"(cf[13]),
-          "s"(cf[14]), "s"(cf[15]));
-    loo_block<LM_K - 1>(in, d2, d2f, thr, af, cf, acc);
-}
-
-// Batched leave-one-out densities of up to 16 fixed bandwidths in one pass
-// over point pairs: each wave owns 64 queries in bin order (lane = query) and
-// walks the candidate bins of its own bounding box; a source's position and
-// coefficients are wave-uniform and come in by scalar loads.  Per (query,
-// source) pair the distance is computed twice: d2f = fl32(dx^2 + dy^2) for the
-// exponent and d2 = fl64(dx^2 + dy^2), exact, for the cut-off (FP64 compares
-// run at the FP32 rate on gfx950, so exactness costs one VALU instruction per
-// candidate and no re-check).  The K candidates (ascending) occupy slots
-// 16-K .. 15.  Thresholds live in SGPR pairs, the exponent factors in VGPRs
-// (wave-uniform values), each source's coefficients in SGPRs.  The sums fold
-// into Kahan pairs every 32 sources.
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6, 6))) void k_loo_multi_w(LooMultiArgs A)
+// Item g of the list; false: the grid is larger than the list (whole wave).
+__device__ __forceinline__ bool sum_item(const SumArgs &A, int64_t g, SumItem &T)
 {
     const PointIndex &I = A.idx;
+    const int64_t units = A.n_items_dev ? (int64_t)*A.n_items_dev : A.order ? (int64_t)A.n_items : (I.n + 63) / 64;
+    if (g >= units) return false;
+    T.item = uniform_item(A.order ? A.items[A.order[g]] : make_int4((int)g, 0, 1, -1));
+    T.win0 = 0;
+    T.win1 = INT_MAX;   // candidate counts are below 2^31
+    if (T.item.z > 1) {
+        const int64_t C = A.cost[T.item.x];
+        if (T.item.y > 0) T.win0 = (int)(C * T.item.y / T.item.z);
+        if (T.item.y < T.item.z - 1) T.win1 = (int)(C * (T.item.y + 1) / T.item.z);
+    }
+    T.q = T.item.x * 64 + (int)(threadIdx.x & 63);   // below 2^30
+    T.qv = T.q < I.n;
+    T.qx = T.qy = 0.0f;
+    if (T.qv) {
+        T.qx = I.pts[T.q].x;
+        T.qy = I.pts[T.q].y;
+    }
+    T.mnx = uni(wave_min(T.qv ? T.qx : FLT_MAX));
+    T.mxx = uni(wave_max(T.qv ? T.qx : -FLT_MAX));
+    T.mny = uni(wave_min(T.qv ? T.qy : FLT_MAX));
+    T.mxy = uni(wave_max(T.qv ? T.qy : -FLT_MAX));
+    return true;
+}
+
+// Walks an item's candidate bins, 64 of a row at a time (one per lane): the whole
+// wave calls fn(m, p0, p1, B, lm) with the mask m of the lanes whose bin, box B and
+// cut-off lm = lim(b), has sources p0 .. p1 - 1 of this part.
+template <class L, class F>
+__device__ __forceinline__ void sum_walk(const PointIndex &I, const SumItem &T, double reach, L lim, F fn)
+{
     const int lane = threadIdx.x & 63;
-    const int off = LM_K - A.K;
-    const int64_t n = I.n;
-    const int64_t g = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int64_t units = A.n_items_dev ? (int64_t)*A.n_items_dev : A.order ? (int64_t)A.n_items : (n + 63) / 64;
-    if (g >= units) return;
-    const int4 item = uniform_item(A.order ? A.items[A.order[g]] : make_int4((int)g, 0, 1, -1));
-    int win0 = 0, win1 = INT_MAX;   // candidate counts are below 2^31
-    if (item.z > 1) {
-        const int64_t C = A.cost[item.x];
-        if (item.y > 0) win0 = (int)(C * item.y / item.z);
-        if (item.y < item.z - 1) win1 = (int)(C * (item.y + 1) / item.z);
-    }
-    const int64_t q0 = (int64_t)item.x * 64;
-    const int64_t q = q0 + lane;
-    const bool qv = q < n;
-    float qx = 0.0f, qy = 0.0f;
-    if (qv) {
-        const PtRec p = I.pts[q];
-        qx = p.x;
-        qy = p.y;
-    }
-    double thr[LM_K];
-    float af[LM_K];
-#pragma unroll
-    for (int k = 0; k < LM_K; ++k) {
-        thr[k] = A.thr_k[k];
-        // a wave-uniform value copied into a VGPR: the scalar file holds the
-        // thresholds and the sources' coefficients
-        const float a = (float)A.a_k[k];
-        asm("v_mov_b32 %0, %1" : "=v"(af[k]) : "s"(a));
-    }
-    const double tmax = A.thr_k[LM_K - 1];
-    const float mnx = uni(wave_min(qv ? qx : FLT_MAX)), mxx = uni(wave_max(qv ? qx : -FLT_MAX));
-    const float mny = uni(wave_min(qv ? qy : FLT_MAX)), mxy = uni(wave_max(qv ? qy : -FLT_MAX));
     int bxa, bxb, bya, byb;
-    bin_range(I.bg, mnx, mxx, mny, mxy, sqrt(tmax) * 1.000001 + 1e-6, bxa, bxb, bya, byb);
+    bin_range(I.bg, T.mnx, T.mxx, T.mny, T.mxy, reach, bxa, bxb, bya, byb);
     bxa = __builtin_amdgcn_readfirstlane(bxa);
     bxb = __builtin_amdgcn_readfirstlane(bxb);
     bya = __builtin_amdgcn_readfirstlane(bya);
     byb = __builtin_amdgcn_readfirstlane(byb);
-    const int q0i = (int)q0;   // bin-order indexes are below 2^30
-    const float inf = INFINITY;
-
-    float acc[LM_K], sum[LM_K], comp[LM_K];
-#pragma unroll
-    for (int k = 0; k < LM_K; ++k) { acc[k] = 0.0f; sum[k] = 0.0f; comp[k] = 0.0f; }
-    int ord = 0;
+    int ord = 0;   // candidate ordinal of the next candidate bin
     for (int by = bya; by <= byb; ++by) {
-        for (int bx = bxa; bx <= bxb; ++bx) {
-            const int b = by * I.bg.nbx + bx;
-            const int bst = I.bin_start[b], ben = I.bin_start[b + 1];
-            if (bst == ben) continue;
-            if (!__builtin_amdgcn_readfirstlane((int)(box_gap2(I.bin_box[b], mnx, mxx, mny, mxy) < tmax))) continue;
-            const int o0 = ord, o1 = ord + (ben - bst);
-            ord = o1;
-            if (o1 <= win0 || o0 >= win1) continue;
-            const int st = bst + (win0 > o0 ? win0 - o0 : 0);
-            const int en = ben - (o1 > win1 ? o1 - win1 : 0);
-            for (int c0 = st; c0 < en; c0 += 32) {
-                const int c1 = c0 + 32 < en ? c0 + 32 : en;
-                for (int si = c0; si < c1; ++si) {
-                    // the lane whose query is this source, if any (scalar)
-                    const unsigned rel = (unsigned)(si - q0i);
-                    const uint64_t selfm = rel < 64u ? (uint64_t)1 << rel : (uint64_t)0;
-                    loo_source(I.pts, A.coefk, si, selfm, qx, qy, inf, thr, af, acc);
-                }
+        for (int bx = bxa; bx <= bxb; bx += 64) {
+            const bool on = bx + lane <= bxb;
+            const int b = by * I.bg.nbx + (on ? bx + lane : bxb);
+            int p0 = I.bin_start[b], p1 = I.bin_start[b + 1];
+            const BinInfo B = I.bin_box[b];
+            const double lm = lim(b);
+            bool mine = on && p0 < p1 && box_gap2(B, T.mnx, T.mxx, T.mny, T.mxy) < lm;
+            if (T.item.z > 1) {
+                const int cnt = mine ? p1 - p0 : 0;
+                const int o1 = ord + (int)wave_incl_scan((unsigned)cnt, lane), o0 = o1 - cnt;
+                ord = __builtin_amdgcn_readlane(o1, 63);
+                mine = mine && o1 > T.win0 && o0 < T.win1;
+                if (T.win1 < o1) p1 -= o1 - T.win1;
+                if (T.win0 > o0) p0 += T.win0 - o0;
+            }
+            const uint64_t m = __ballot(mine);
+            if (m) fn(m, p0, p1, B, lm);
+        }
+    }
+}
+
+// Bounds of the squared distances between a bin's box and the box x0 .. y1.
+__device__ __forceinline__ double box_far2(const BinInfo &B, float x0, float x1, float y0, float y1)
+{
+    return sq2(fmaxf(B.x1 - x0, x1 - B.x0), fmaxf(B.y1 - y0, y1 - B.y0));
+}
+
+// One bandwidth, or one per source.  A wave takes 64 / P of an item's queries and
+// P of the sums of 32 at a time, one per 64 / P lanes, which are then folded in
+// their order: as many waves more, each that much shorter, and the same sums.
+// The sources come in one per lane and are handed round through LDS.  The cut-off
+// is decided in FP32 where the distance is clear of the threshold (thr_bracket),
+// else by the exact FP64 test, and not at all for bins that are inside as a whole.
+// Bound by instruction issue: 8 a pair of an inside bin, 12 else.  (Scalar loads
+// of each source, one wave an item: two steps of the adaptive search on 100,000
+// clustered points 1.63 ms, now 0.81 ms; two candidates 0.84 -> 0.34 ms.)
+enum { SUM_PILOT, SUM_LOO, SUM_LOO_EACH };   // one bandwidth, one of K without the query, one per source without it
+template <int KIND, int P>
+__global__ __launch_bounds__(256) void k_point_sums(SumArgs A)
+{
+    constexpr int Q = 64 / P;
+    constexpr bool EACH = KIND == SUM_LOO_EACH, SELF = KIND == SUM_PILOT;
+    __shared__ float4 s_a[4][P][33];                // x, y, coef, af (33: the P records read together are in different banks)
+    __shared__ float2 s_b[EACH ? 4 : 1][P][33];     // lo, hi
+    const PointIndex &I = A.idx;
+    const int lane = threadIdx.x & 63, r = lane % Q, ph = lane / Q;
+    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t gw = (int64_t)blockIdx.x * 4 + wid;
+    const int u = (int)(gw % P), k = blockIdx.y;
+    SumItem T;
+    if (!sum_item(A, gw / P, T)) return;
+    const int q0 = T.item.x * 64, q = q0 + u * Q + r;
+    const bool qv = q < I.n;
+    const float qx = __shfl(T.qx, u * Q + r, WAVE), qy = __shfl(T.qy, u * Q + r, WAVE);
+    const float x0 = uni(wave_min(qv ? qx : FLT_MAX)), x1 = uni(wave_max(qv ? qx : -FLT_MAX));
+    const float y0 = uni(wave_min(qv ? qy : FLT_MAX)), y1 = uni(wave_max(qv ? qy : -FLT_MAX));
+    const double thr = EACH ? 0.0 : SELF ? A.thr_fixed : A.thr_k[k];
+    const double lim_all = EACH ? 0.0 : SELF ? A.thr_fixed : A.thr_k[A.K - 1];   // of the work list
+    const float f_a = EACH ? 0.0f : uni((float)(SELF ? A.a_fixed : A.a_k[k]));
+    float f_lo = 0.0f, f_hi = 0.0f;
+    if (!EACH) thr_bracket(thr, f_lo, f_hi);
+    float sum = 0.0f, comp = 0.0f;
+    int pos = 0, cnt = 0, np = 0;   // this lane's chunk, chunks taken up
+    bool all = true, own = false;
+
+    auto flush = [&]() __attribute__((always_inline)) {
+        wave_sync();
 #pragma unroll
-                for (int k = 0; k < LM_K; ++k) {
-                    kahan_fold(acc[k], sum[k], comp[k]);
-                    acc[k] = 0.0f;
+        for (int i = r; i < 32; i += Q) {
+            if (P == 1 && i >= 32) break;
+            // past the chunk's end: too far to count, without a weight
+            float4 v = make_float4(1e19f, 1e19f, 0.0f, -1.0f);
+            float2 t = make_float2(-1.0f, -1.0f);
+            if (i < cnt) {
+                const PtRec p = I.pts[pos + i];
+                v = make_float4(p.x, p.y, KIND == SUM_LOO ? A.coefk[(int64_t)k * I.n + pos + i] : p.coef, (float)p.a);
+                if (EACH) thr_bracket(p.thr, t.x, t.y);
+            }
+            s_a[wid][ph][i] = v;
+            if (EACH) s_b[EACH ? wid : 0][ph][i] = t;
+        }
+        wave_sync();
+        int jn = __builtin_amdgcn_readlane(cnt, 0);
+#pragma unroll
+        for (int i = 1; i < P; ++i) {
+            const int c = __builtin_amdgcn_readlane(cnt, i * Q);
+            jn = jn > c ? jn : c;
+        }
+        float acc = 0.0f;
+        bool band = !SELF && own;
+        if (!EACH && all && !band) {
+#pragma unroll 4
+            for (int j = 0; j < jn; ++j) {
+                const float4 p = s_a[wid][ph][j];
+                const float dx = p.x - qx, dy = p.y - qy;
+                const float d2f = __builtin_fmaf(dy, dy, dx * dx);
+                acc = __builtin_fmaf(fast_exp2(d2f * f_a), p.z, acc);
+            }
+        } else if (!band) {
+#pragma unroll 4
+            for (int j = 0; j < jn; ++j) {
+                const float4 p = s_a[wid][ph][j];
+                const float2 t = EACH ? s_b[EACH ? wid : 0][ph][j] : make_float2(f_lo, f_hi);
+                const float dx = p.x - qx, dy = p.y - qy;
+                const float d2f = __builtin_fmaf(dy, dy, dx * dx);
+                const bool in = d2f < t.x;
+                band |= !(d2f > t.y) != in;
+                const float e = fast_exp2(d2f * (EACH ? p.w : f_a));
+                acc = __builtin_fmaf(in ? e : 0.0f, p.z, acc);
+            }
+        }
+        if (__any(band)) {   // rare, and the bins of the queries themselves
+            acc = 0.0f;
+            for (int j = 0; j < jn; ++j) {
+                const float4 p = s_a[wid][ph][j];
+                const float dx = p.x - qx, dy = p.y - qy;
+                const float d2f = __builtin_fmaf(dy, dy, dx * dx);
+                bool in = sq2(dx, dy) < (EACH ? (j < cnt ? I.pts[pos + j].thr : -1.0) : thr);
+                if (!SELF && pos + j == q) in = false;
+                const float e = fast_exp2(d2f * (EACH ? p.w : f_a));
+                acc = __builtin_fmaf(in ? e : 0.0f, p.z, acc);
+            }
+        }
+        if (P == 1) {
+            kahan_fold(acc, sum, comp);
+        } else {
+            // the P sums in their order, in all of a query's lanes
+#pragma unroll
+            for (int i = 0; i < P; ++i) {
+                const float v = __shfl(acc, i * Q + r, WAVE);
+                if (i < np) kahan_fold(v, sum, comp);
+            }
+        }
+        np = 0;
+        cnt = 0;
+        all = true;
+        own = false;
+    };
+
+    const double reach = EACH ? *I.reach_p : sqrt(fmax(lim_all, 0.0)) * 1.000001 + 1e-6;
+    sum_walk(I, T, reach, [&](int b) { return EACH ? I.bin_thr[b] : lim_all; },
+             [&](uint64_t m, int p0, int p1, const BinInfo &B, double lm) __attribute__((always_inline)) {
+                 // of this wave's queries
+                 const int bin_all = !EACH && box_far2(B, x0, x1, y0, y1) < thr;
+                 m &= __ballot(box_gap2(B, x0, x1, y0, y1) < (EACH ? lm : thr));
+                 const uint64_t inside = __ballot(bin_all);
+                 while (m) {
+                     const int l = __builtin_ctzll(m);
+                     m &= m - 1ull;
+                     const int a = __builtin_amdgcn_readlane(p0, l), b = __builtin_amdgcn_readlane(p1, l);
+                     const bool is_own = b > q0 && a < q0 + 64, is_all = (inside >> l) & 1ull;
+                     for (int c = a; c < b; c += 32) {
+                         if (P == 1 || ph == np) {
+                             pos = c;
+                             cnt = b - c < 32 ? b - c : 32;
+                         }
+                         all = all && is_all;
+                         own = own || is_own;
+                         if (++np == P) flush();
+                     }
+                 }
+             });
+    if (P > 1 && np) flush();
+    if (ph != 0) return;
+    if (T.item.z > 1) {
+        const int64_t at = KIND == SUM_LOO ? (int64_t)T.item.w * LM_K + k : (int64_t)T.item.w;
+        A.partials[at * 64 + u * Q + r] = (double)sum - (double)comp;
+    } else if (qv) {
+        A.den1[(int64_t)k * I.n + q] = sum;
+    }
+}
+
+// Sources c0 .. c1 - 1 for candidates k .. k + N - 1: candidate k's term is
+// exp2(d2f a_k) coef_k if the exact cut-off fl64(dx^2 + dy^2) < thr_k holds (ALL:
+// every pair is inside), else 0, d2f = fl32(dx^2 + dy^2).  FP64 compares run at
+// the FP32 rate on gfx950, so exactness costs one instruction per candidate and
+// no re-check.  32 sources at a time: their positions and these N coefficients
+// come in one per lane and are handed round through LDS (s_src).  (With scalar
+// loads of each source the kernel waited for them two thirds of its time.)
+// s_sum: this lane's Kahan pairs from candidate k on, 64 apart.  The query itself is left out.
+#define LM_REC 12   // floats of a source's record for 8 candidates: x, y, coefficients
+template <int N, bool ALL>
+__device__ __forceinline__ void loo_run(const SumArgs &A, const SumItem &T, int k, int c0, int c1, float2 *s_sum,
+                                        float *s_src)
+{
+    constexpr int R = (N + 2 + 3) / 4 * 4;
+    const int lane = threadIdx.x & 63;
+    const int64_t n = A.idx.n;
+    double thr[N];
+    float af[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        thr[i] = A.thr_k[k + i];
+        af[i] = uni((float)A.a_k[k + i]);
+    }
+    const bool own = !ALL && c1 > T.item.x * 64 && c0 < T.item.x * 64 + 64;
+    for (int b0 = c0; b0 < c1; b0 += 32) {
+        const int cnt = c1 - b0 < 32 ? c1 - b0 : 32;
+        wave_sync();
+        if (lane < cnt) {
+            const int p = b0 + lane;
+            float rec[R] = {A.idx.pts[p].x, A.idx.pts[p].y};
+#pragma unroll
+            for (int i = 0; i < N; ++i) rec[2 + i] = A.coefk[(int64_t)(k + i) * n + p];
+#pragma unroll
+            for (int i = 0; i < R; i += 4)
+                *(float4 *)(s_src + lane * R + i) = make_float4(rec[i], rec[i + 1], rec[i + 2], rec[i + 3]);
+        }
+        wave_sync();
+        float acc[N];
+#pragma unroll
+        for (int i = 0; i < N; ++i) acc[i] = 0.0f;
+#pragma unroll 2
+        for (int j = 0; j < cnt; ++j) {
+            float rec[R];
+#pragma unroll
+            for (int i = 0; i < R; i += 4) {
+                const float4 v = *(const float4 *)(s_src + j * R + i);
+                rec[i] = v.x;
+                rec[i + 1] = v.y;
+                rec[i + 2] = v.z;
+                rec[i + 3] = v.w;
+            }
+            const float dx = rec[0] - T.qx, dy = rec[1] - T.qy;
+            const float d2f = __builtin_fmaf(dy, dy, dx * dx);
+            if (ALL) {
+#pragma unroll
+                for (int i = 0; i < N; ++i) acc[i] = __builtin_fmaf(fast_exp2(d2f * af[i]), rec[2 + i], acc[i]);
+            } else {
+                double d2 = sq2(dx, dy);
+                if (own) d2 = b0 + j == T.q ? (double)INFINITY : d2;
+#pragma unroll
+                for (int i = 0; i < N; ++i) {
+                    const float e = fast_exp2(d2f * af[i]);
+                    acc[i] = __builtin_fmaf(d2 < thr[i] ? e : 0.0f, rec[2 + i], acc[i]);
                 }
             }
         }
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            float2 v = s_sum[i * 64];
+            kahan_fold(acc[i], v.x, v.y);
+            s_sum[i * 64] = v;
+        }
     }
-    // outputs by candidate index k - off (rows of den1, rows of a part's partials)
-    if (item.z > 1) {
-        double *pp = A.partials + (int64_t)item.w * 64 * LM_K + lane;
-#pragma unroll
-        for (int k = 0; k < LM_K; ++k)
-            if (k >= off) pp[(k - off) * 64] = (double)sum[k] - (double)comp[k];
-    } else {
-#pragma unroll
-        for (int k = 0; k < LM_K; ++k)
-            if (qv && k >= off) A.den1[(int64_t)(k - off) * n + q] = sum[k];
+}
+
+// Candidates ka .. kb - 1, up to 8 at a time (s_sum: from candidate k0 on).
+template <bool ALL>
+__device__ __forceinline__ void loo_runs(const SumArgs &A, const SumItem &T, int k0, int ka, int kb, int c0, int c1,
+                                         float2 *s_sum, float *s_src)
+{
+    for (int k = ka; k < kb;) {
+        const int left = kb - k, m = left <= 8 ? left : left < 16 ? (left + 1) / 2 : 8;
+        switch (m) {
+#define MKDE_LR(N) case N: loo_run<N, ALL>(A, T, k, c0, c1, s_sum + (k - k0) * 64, s_src); break;
+            MKDE_LR(1) MKDE_LR(2) MKDE_LR(3) MKDE_LR(4) MKDE_LR(5) MKDE_LR(6) MKDE_LR(7) MKDE_LR(8)
+#undef MKDE_LR
+        }
+        k += m;
+    }
+}
+
+// Up to LM_K fixed bandwidths, ascending.  Each wave owns 64 queries (lane =
+// query).  A bin is summed only for the candidates that reach it, without tests
+// for those that hold every pair of it.  Bound by instruction issue: 9 a pair and
+// 6 a candidate's term, 4 and 4 where all pairs are inside.  The 16 largest of 64
+// candidates on 200,000 points: 42.7 ms with every source tested for the
+// candidates four at a time and scalar loads, 30.6 ms now.
+__global__ __launch_bounds__(256) void k_loo_multi(SumArgs A)
+{
+    extern __shared__ float2 s_loo[];   // [4][kw][64]
+    __shared__ float4 s_rec[4][32 * LM_REC / 4];
+    const int lane = threadIdx.x & 63;
+    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int ka = blockIdx.y * A.kw, kb = ka + A.kw < A.K ? ka + A.kw : A.K;
+    SumItem T;
+    if (!sum_item(A, (int64_t)blockIdx.x * 4 + wid, T)) return;
+    float2 *s_sum = s_loo + wid * A.kw * 64 + lane;
+    float *s_src = (float *)s_rec[wid];
+    for (int k = 0; k < kb - ka; ++k) s_sum[k * 64] = make_float2(0.0f, 0.0f);
+    const int q0 = T.item.x * 64;
+    // all candidates' ordinals: the work list counts them for the largest
+    const double tmax = A.thr_k[A.K - 1];
+    sum_walk(A.idx, T, sqrt(tmax) * 1.000001 + 1e-6, [&](int) { return tmax; },
+             [&](uint64_t m, int p0, int p1, const BinInfo &B, double) {
+                 const double near = box_gap2(B, T.mnx, T.mxx, T.mny, T.mxy);
+                 const double far = p1 > q0 && p0 < q0 + 64 ? (double)INFINITY
+                                                            : box_far2(B, T.mnx, T.mxx, T.mny, T.mxy);
+                 int k0 = ka, kf = ka;   // candidates below k0 reach no pair, those from kf on hold all
+                 for (int k = ka; k < kb; ++k) {
+                     const double t = A.thr_k[k];
+                     k0 += t <= near ? 1 : 0;
+                     kf += t <= far ? 1 : 0;
+                 }
+                 m &= __ballot(k0 < kb);
+                 while (m) {
+                     const int l = __builtin_ctzll(m);
+                     m &= m - 1ull;
+                     const int a = __builtin_amdgcn_readlane(p0, l), b = __builtin_amdgcn_readlane(p1, l);
+                     const int f = __builtin_amdgcn_readlane(kf, l);
+                     loo_runs<false>(A, T, ka, __builtin_amdgcn_readlane(k0, l), f, a, b, s_sum, s_src);
+                     loo_runs<true>(A, T, ka, f, kb, a, b, s_sum, s_src);
+                 }
+             });
+    if (T.item.z > 1) {
+        double *pp = A.partials + ((int64_t)T.item.w * LM_K + ka) * 64 + lane;
+        for (int k = 0; k < kb - ka; ++k) pp[k * 64] = (double)s_sum[k * 64].x - (double)s_sum[k * 64].y;
+    } else if (T.qv) {
+        for (int k = 0; k < kb - ka; ++k) A.den1[(int64_t)(ka + k) * A.idx.n + T.q] = s_sum[k * 64].x;
     }
 }
 
@@ -2271,14 +2343,6 @@ __global__ __launch_bounds__(256) void k_bt_up(BndTree T, int l, float4 *box)
 __device__ __forceinline__ double node_lb(float4 b, float px, float py)
 {
     return b.x > b.z ? DBL_MAX : sq2(gap1(px, b.x, b.z), gap1(py, b.y, b.w));
-}
-
-// Orders LDS accesses of the lanes of one wave (its LDS operations complete in
-// order, so only the compiler has to keep them).
-__device__ __forceinline__ void wave_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
 }
 
 // CalcDist2Boundary as a search of the hierarchy that prunes nodes whose lower
@@ -3095,26 +3159,26 @@ __global__ void k_sort_f32(int64_t n, const int *perm, const float *src, float *
 }
 
 // coefk[k*n + i] = w * ew_k / (2 pi h2_k), bin order
-// coef_out[i * stride]: one candidate's coefficient of every point (bin order)
+// coef_out[i]: one candidate's coefficient of every point (bin order)
 __global__ void k_coef_k(int64_t n, const int *perm, const float *w_orig, const float *ew_k_orig, double h2k,
-                         float *coef_out, int stride)
+                         float *coef_out)
 {
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const int o = perm[i];
-    coef_out[i * stride] = (float)((double)w_orig[o] * (double)ew_k_orig[o] / (h2k * (double)MKDE_TWO_PI_F));
+    coef_out[i] = (float)((double)w_orig[o] * (double)ew_k_orig[o] / (h2k * (double)MKDE_TWO_PI_F));
 }
 
 // k_coef_k with the bandwidth read from the device: h2k = fl32(h*h).
 __global__ void k_coef_k_dev(int64_t n, const int *perm, const float *w_orig, const float *ew_k_orig, const float *h_dev,
-                             float *coef_out, int stride)
+                             float *coef_out)
 {
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const float h = *h_dev;
     const double h2k = (double)(float)(h * h);
     const int o = perm[i];
-    coef_out[i * stride] = (float)((double)w_orig[o] * (double)ew_k_orig[o] / (h2k * (double)MKDE_TWO_PI_F));
+    coef_out[i] = (float)((double)w_orig[o] * (double)ew_k_orig[o] / (h2k * (double)MKDE_TWO_PI_F));
 }
 
 __global__ void k_fill_f32(int64_t n, float v, float *dst)
@@ -3249,11 +3313,13 @@ hipError_t density_merge(hipStream_t s, const GridDesc &g, const Tiling &tl, con
 }
 
 // Split rule of the point work lists.  kind 0: density at points, 1: the
-// leave-one-out sums (density at points without the query, or batched).
-SplitRule point_rule(int kind, const Tuning &T, bool batched)
+// leave-one-out sums (density at points without the query, or batched); binned:
+// in bin order, whose sums depend a little on where a wave is cut and keep to the
+// larger parts.
+SplitRule point_rule(int kind, const Tuning &T, bool batched, bool binned)
 {
     SplitRule r{MKDE_PTS_TMIN, batched ? T.loo_target : T.pts_target, 0u, 0ull};
-    if (kind == 1) {
+    if (kind == 1 && !binned) {
         r.few_tmin = MKDE_LOO_FEW_TMIN;
         r.few = MKDE_LOO_FEW;
     }
@@ -3277,6 +3343,18 @@ hipError_t point_plan(hipStream_t s, const PointIndex &idx, float h_fixed, const
     return hipGetLastError();
 }
 
+// Four waves an item while the list is short (1563 waves: two pilots 720 us with
+// one wave an item, 287 us with four; 15625 waves: 3.43 and 3.58 ms).
+template <int KIND>
+static void launch_sums(hipStream_t s, const SumArgs &A)
+{
+    const int64_t nw = (A.idx.n + 63) / 64, items = A.order ? A.n_items : nw;
+    const int P = nw * A.K <= MKDE_SUM_SHORT ? 4 : 1;
+    const dim3 grid((unsigned)((items * P + 3) / 4), (unsigned)A.K);
+    if (P == 4) hipLaunchKernelGGL(HIP_KERNEL_NAME(k_point_sums<KIND, 4>), grid, dim3(256), 0, s, A);
+    else hipLaunchKernelGGL(HIP_KERNEL_NAME(k_point_sums<KIND, 1>), grid, dim3(256), 0, s, A);
+}
+
 // n_items_dev non-null (here and in loo_multi): the item count is read on the
 // device and n_items is only the grid bound.
 // fine: the index is in fine order and res is scratch for n floats; else one
@@ -3285,7 +3363,7 @@ hipError_t point_density(hipStream_t s, const PointIndex &idx, bool fine, int lo
                          float h_fixed, const int *order, const int4 *items, const unsigned *cost,
                          double *partials, int n_items, const unsigned *n_items_dev)
 {
-    PtsArgs A{idx, den_sorted, res, 0.0, 0.0, order, items, cost, partials, n_items, n_items_dev};
+    PtsArgs A{idx, den_sorted, res, order, items, cost, partials, n_items, n_items_dev};
     if (idx.n <= 0) return hipSuccess;
     const int64_t units = order ? n_items : (idx.n + 63) / 64;
     const unsigned grid = (unsigned)((units + 3) / 4);
@@ -3300,22 +3378,53 @@ hipError_t point_density(hipStream_t s, const PointIndex &idx, bool fine, int lo
     } else {
         if (loo || !(h_fixed > 0.0f)) return hipErrorInvalidValue;
         const double h2 = (double)(float)(h_fixed * h_fixed);
-        A.thr_fixed = 9.0 * h2;
-        A.a_fixed = -MKDE_LOG2E / (2.0 * h2);
-        hipLaunchKernelGGL(k_pilot_density, dim3(grid), dim3(256), 0, s, A);
+        SumArgs S{};
+        S.idx = idx;
+        S.K = S.kw = 1;
+        S.thr_fixed = 9.0 * h2;
+        S.a_fixed = -MKDE_LOG2E / (2.0 * h2);
+        S.den1 = den_sorted;
+        S.order = order;
+        S.items = items;
+        S.cost = cost;
+        S.partials = partials;
+        S.n_items = n_items;
+        S.n_items_dev = n_items_dev;
+        launch_sums<SUM_PILOT>(s, S);
     }
     return hipGetLastError();
 }
 
 hipError_t loo_multi(hipStream_t s, const PointIndex &idx, const float *coefk, const double *a_k,
                      const double *thr_k, int K, float *den1, const int *order, const int4 *items,
-                     const unsigned *cost, double *partials, int n_items,
-                     const unsigned *n_items_dev)
+                     const unsigned *cost, double *partials, int n_items, const unsigned *n_items_dev)
 {
-    LooMultiArgs A{idx, coefk, a_k, thr_k, K, den1, order, items, cost, partials, n_items, n_items_dev};
     if (idx.n <= 0) return hipSuccess;
-    const int64_t units = order ? n_items : (idx.n + 63) / 64;
-    hipLaunchKernelGGL(k_loo_multi_w, dim3((unsigned)((units + 3) / 4)), dim3(256), 0, s, A);
+    if (idx.grp) return hipErrorInvalidValue;   // fine order
+    const int64_t nw = (idx.n + 63) / 64;
+    SumArgs A{idx, coefk, a_k, thr_k, K, 1, 0.0, 0.0, den1, order, items, cost, partials, n_items, n_items_dev};
+    // a distance shared by few candidates saves nothing, and a short list is
+    // better filled by a wave per candidate
+    if (K <= 2 || nw * K <= MKDE_LOO_WAVES) {
+        launch_sums<SUM_LOO>(s, A);
+        return hipGetLastError();
+    }
+    int ky = (int)((MKDE_LOO_WAVES + nw - 1) / nw);
+    ky = ky < K ? ky : K;
+    A.kw = (K + ky - 1) / ky;
+    hipLaunchKernelGGL(k_loo_multi, dim3((unsigned)((n_items + 3) / 4), (unsigned)((K + A.kw - 1) / A.kw)), dim3(256),
+                       4 * 64 * A.kw * sizeof(float2), s, A);
+    return hipGetLastError();
+}
+
+// Leave-one-out densities in bin order with the index's bandwidths.
+hipError_t loo_density(hipStream_t s, const PointIndex &idx, float *den, const int *order, const int4 *items,
+                       const unsigned *cost, double *partials, int n_items, const unsigned *n_items_dev)
+{
+    if (idx.n <= 0) return hipSuccess;
+    if (idx.grp) return hipErrorInvalidValue;   // fine order
+    SumArgs A{idx, nullptr, nullptr, nullptr, 1, 1, 0.0, 0.0, den, order, items, cost, partials, n_items, n_items_dev};
+    launch_sums<SUM_LOO_EACH>(s, A);
     return hipGetLastError();
 }
 
@@ -3626,18 +3735,18 @@ hipError_t sort_f32(hipStream_t s, int64_t n, const int *perm, const float *src,
 }
 
 hipError_t coef_k(hipStream_t s, int64_t n, const int *perm, const float *w, const float *ew_k, double h2k,
-                  float *coef_out, int stride)
+                  float *coef_out)
 {
     if (n > 0)
-        hipLaunchKernelGGL(k_coef_k, dim3(nblk(n, 256)), dim3(256), 0, s, n, perm, w, ew_k, h2k, coef_out, stride);
+        hipLaunchKernelGGL(k_coef_k, dim3(nblk(n, 256)), dim3(256), 0, s, n, perm, w, ew_k, h2k, coef_out);
     return hipGetLastError();
 }
 
 hipError_t coef_k_dev(hipStream_t s, int64_t n, const int *perm, const float *w, const float *ew_k, const float *h_dev,
-                      float *coef_out, int stride)
+                      float *coef_out)
 {
     if (n > 0)
-        hipLaunchKernelGGL(k_coef_k_dev, dim3(nblk(n, 256)), dim3(256), 0, s, n, perm, w, ew_k, h_dev, coef_out, stride);
+        hipLaunchKernelGGL(k_coef_k_dev, dim3(nblk(n, 256)), dim3(256), 0, s, n, perm, w, ew_k, h_dev, coef_out);
     return hipGetLastError();
 }
 

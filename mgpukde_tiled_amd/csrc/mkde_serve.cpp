@@ -43,7 +43,7 @@ extern "C" int mkde_internal_fail(int code, const char *msg);
 extern "C" void mkde_internal_share_device(mkde_ctx *c);
 namespace mkde_dev {
 Tuning default_tuning();
-SplitRule point_rule(int, const Tuning &, bool);
+SplitRule point_rule(int, const Tuning &, bool, bool);
 }
 
 namespace {
@@ -141,10 +141,10 @@ extern "C" int64_t mkde_job_footprint(int64_t n, int64_t ncols, int64_t nrows, i
     // part for densities at points and 8 KB per part for a 16-candidate pass
     // (a bandwidth search sizes them so for its captured graph)
     int64_t items = 0, slots = 0;
-    point_work_bounds(n, mkde_dev::point_rule(loo ? 1 : 0, tune, false), &items, &slots);
+    point_work_bounds(n, mkde_dev::point_rule(loo ? 1 : 0, tune, false, true), &items, &slots);
     b += items * 20 + slots * 512;
     if (loo) {
-        point_work_bounds(n, mkde_dev::point_rule(1, tune, true), &items, &slots);
+        point_work_bounds(n, mkde_dev::point_rule(1, tune, true, true), &items, &slots);
         b += items * 20 + slots * 8192;
     }
     return b;
