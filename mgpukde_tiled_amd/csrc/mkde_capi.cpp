@@ -41,7 +41,7 @@ hipError_t density_plan(hipStream_t, const GridDesc &, const float *, const Poin
 hipError_t work_items(hipStream_t, int, const WorkList &, int4 *, int4 *, int *);
 hipError_t density_tile(hipStream_t, const GridDesc &, const float *, float *, const PointIndex &,
                         unsigned long long *, const int *, const int4 *, const unsigned *, double *, int,
-                        const Tiling &);
+                        const Tiling &, double *, int *);
 hipError_t density_merge(hipStream_t, const GridDesc &, const Tiling &, const float *, int, const int4 *,
                          const double *, float *);
 SplitRule point_rule(int, const Tuning &, bool, bool);
@@ -286,7 +286,8 @@ struct mkde_ctx {
     DevBuf<unsigned> blk_cost, blk_item0, blk_slot0, blk_sidx, blk_counts, blk_hist;
     DevBuf<int4> dt_items, dt_splits;
     DevBuf<int> dt_order;
-    DevBuf<double> dt_partials;
+    DevBuf<double> dt_partials, dt_nodes;
+    DevBuf<int> dt_node_on;
 };
 
 extern "C" const char *mkde_last_error(void) { return g_err.c_str(); }
@@ -1754,6 +1755,7 @@ extern "C" int mkde_density_tile_resident(mkde_ctx *c)
     const float *tm = c->tile_is_ec_mask ? c->mask.p : c->tile_has_mask ? c->tmask.p : nullptr;
     const int *order = nullptr;
     int n_items = 0, n_split = 0;
+    bool nodes = false;
     if (c->dt_order_on) {
         const int64_t nblk = mkde_dev::raster_blocks(c->tg, c->tl);
         CHK(c->blk_cost.ensure(nblk));
@@ -1772,12 +1774,18 @@ extern "C" int mkde_density_tile_resident(mkde_ctx *c)
         CHK(c->dt_order.ensure(n_items));
         CHK(c->dt_splits.ensure(n_split));
         CHK(c->dt_partials.ensure((size_t)c->host_words[1] * MKDE_DT_CELLS));
+        nodes = c->host_words[3] >= MKDE_DN_SPLIT;
+        if (nodes) {
+            CHK(c->dt_nodes.ensure((size_t)n_items * MKDE_DN_CELLS));
+            CHK(c->dt_node_on.ensure(n_items));
+        }
         HIPCHK(mkde_dev::work_items(c->stream, (int)nblk, W, c->dt_items.p, c->dt_splits.p, c->dt_order.p));
         order = c->dt_order.p;
     }
     HIPCHK(hipEventRecord(c->ev0, c->stream));
     HIPCHK(mkde_dev::density_tile(c->stream, c->tg, tm, c->tout.p, I, c->dt_stats_on ? c->dt_stats.p : nullptr,
-                                  order, c->dt_items.p, c->blk_cost.p, c->dt_partials.p, n_items, c->tl));
+                                  order, c->dt_items.p, c->blk_cost.p, c->dt_partials.p, n_items, c->tl,
+                                  nodes ? c->dt_nodes.p : nullptr, c->dt_node_on.p));
     HIPCHK(mkde_dev::density_merge(c->stream, c->tg, c->tl, tm, n_split, c->dt_splits.p, c->dt_partials.p,
                                    c->tout.p));
     HIPCHK(hipEventRecord(c->ev1, c->stream));

@@ -134,6 +134,10 @@ struct PointIndex {
 // each, one 32 x 32 quadrant per wave (MKDE_DT_BW / 16 waves).
 #define MKDE_DT_BW 64
 #define MKDE_DT_CELLS (64 * MKDE_DT_BW)
+// Sums of an item at the nodes of its block, for rasters whose split threshold
+// (candidates of an item) is at least this.
+#define MKDE_DN_CELLS 256
+#define MKDE_DN_SPLIT 4096
 
 // A raster processed as tiles of tw x th cells, each tile with its own origin
 // from the raster geotransform (GDAL order gt0, gt1, gt3, gt5).  Density

@@ -130,6 +130,15 @@ __device__ __forceinline__ int block_compact256(bool flag, int *s_wcnt, int *tot
     return block_compact<4>(flag, s_wcnt, total);
 }
 
+__device__ __forceinline__ unsigned wave_incl_scan(unsigned v, int lane)
+{
+    for (int d = 1; d < WAVE; d <<= 1) {
+        const unsigned o = __shfl_up(v, d, WAVE);
+        if (lane >= d) v += o;
+    }
+    return v;
+}
+
 __device__ __forceinline__ int clampi(int64_t v, int64_t lo, int64_t hi)
 {
     return (int)(v < lo ? lo : (v > hi ? hi : v));
@@ -415,6 +424,8 @@ struct TileArgs {
     double *partials;            // MKDE_DT_CELLS per slot
     int nbx;                     // density blocks per raster row
     Tiling tl;
+    double *nodes;               // per item DN_N x DN_N sums of wide kernels
+    int *node_on;                // per item: whether it has them
 };
 
 // Geometry of one 64x64 block: global cell range [c0,c1]x[r0,r1], and the
@@ -457,13 +468,215 @@ __device__ __forceinline__ BlockGeom block_geom(const GridDesc &g, const Tiling 
     return b;
 }
 
+// Wide kernels at nodes.  A block-FULL point whose bandwidth is not small against
+// the block is smooth over it: the sum of all such points is formed at 16 x 16
+// Chebyshev nodes of the block instead of its 64 x 64 cells, one 16 x 16 x 4 MFMA
+// for four points, and interpolated to the cells once at the end (FP64).  For h >=
+// half extent / (2 DN_KAPPA) (24 cells) the interpolant of a point is within
+// 4.4e-9 of its value anywhere in the block, and the weights of a cell have a root
+// sum of squares of 1, so rounding at the nodes is not amplified.  Per point and
+// block: 0.25 MFMA of 8 passes, 10 VALU instructions and 1.3 lane permutations,
+// where the cells take 2 MFMA of 16 passes and 30 instructions.  Every wave walks
+// the candidate bins by itself, without barriers, and takes every fourth 64 points.
+// Bound by instruction issue.  A kernel of its own: inside k_density_tile, whose
+// registers and scalars it then shares, everything else took 10% longer.
+// 1M points, adaptive bandwidths, 8192^2 cells: 23.6 ms with all points at the
+// cells, 1.6 + 15.7 ms now.  Rasters of few candidates an item (MKDE_DN_SPLIT)
+// keep to the cells: 50,000 points on 2048^2 took 405 us there and 464 us here.
+#define DN_N 16
+#define DN_KAPPA 0.65
+// Candidates of an item from which on its bins are searched for such points, and
+// points from which on the interpolation (about 1200 instructions a wave) pays.
+#define DN_CAND 2048
+#define DN_MIN 192
+// Smallest cut-off threshold 9 h^2 of a point that goes to the nodes.
+__device__ __forceinline__ double dn_thr_min(double L) { return L * L * (9.0 / (4.0 * DN_KAPPA * DN_KAPPA)) * 0.999999; }
+
+__device__ __forceinline__ double dn_node(int j)
+{
+    const int i = j < 8 ? j : 15 - j;
+    const double c = i == 0   ? 0.99518472667219692873
+                     : i == 1 ? 0.95694033573220882438
+                     : i == 2 ? 0.88192126434835504956
+                     : i == 3 ? 0.77301045336273699338
+                     : i == 4 ? 0.63439328416364548779
+                     : i == 5 ? 0.47139673682599780857
+                     : i == 6 ? 0.29028467725446233105
+                              : 0.09801714032956077016;   // cos((2i + 1) pi / 32)
+    return j < 8 ? c : -c;
+}
+
+// Centre and half extent of a block's node grid.
+struct BlockNodes {
+    double mx, my, L;
+};
+__device__ __forceinline__ BlockNodes block_nodes(float bx0, float bx1, float by0, float by1, double cs)
+{
+    return BlockNodes{0.5 * ((double)bx0 + (double)bx1), 0.5 * ((double)by0 + (double)by1),
+                      0.5 * fmax(fmax((double)bx1 - (double)bx0, (double)by1 - (double)by0), 0.5 * cs)};
+}
+
+// Whether a point that is FULL for a block of half extent L goes to the nodes:
+// L <= 2 DN_KAPPA h, a = -log2(e) / (2 h^2).
+__device__ __forceinline__ bool dn_wide(double a, double L)
+{
+    return L * L * -a <= 2.0 * DN_KAPPA * DN_KAPPA * MKDE_LOG2E;
+}
+
+// Interpolation weights of a cell at v (centre mid, half extent L) to w[64 j],
+// barycentric: w_j = b_j / (x - x_j) / sum, b_j = (-1)^j sin((2j + 1) pi / 32).
+__device__ __forceinline__ void dn_weights(double v, double mid, double L, double *w)
+{
+    const double x = (v - mid) / L;
+    double t[DN_N], sum = 0.0;
+    int hit = -1;
+#pragma unroll
+    for (int j = 0; j < DN_N; ++j) {
+        const double d = x - dn_node(j);
+        if (d == 0.0) hit = j;
+        const double b = dn_node(j < 8 ? 7 - j : j - 8);   // the sine
+        t[j] = ((j & 1) ? -b : b) / d;
+        sum += t[j];
+    }
+    const double r = 1.0 / sum;
+#pragma unroll
+    for (int j = 0; j < DN_N; ++j) w[64 * j] = hit < 0 ? t[j] * r : hit == j ? 1.0 : 0.0;
+}
+
+// This wave's share of the node sums of an item: lane l, entry v of s is row node
+// 4 (l >> 4) + v, column node l & 15 (the accumulator layout of
+// v_mfma_f32_16x16x4_f32).  Returns the points summed.  win0 .. win1 - 1: the
+// item's candidate ordinals (split: there are others).
+__device__ __forceinline__ int dn_sums(const PointIndex &I, int bxa, int bxb, int bya, int byb, bool split, int64_t win0,
+                                       int64_t win1, float bx0, float bx1, float by0, float by1, double mx, double my,
+                                       double L, double (&s)[4])
+{
+    typedef float f32x4 __attribute__((ext_vector_type(4)));
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const double nx = mx + L * dn_node(lane & 15), ny = my + L * dn_node(lane & 15);
+    const int nbx_r = bxb - bxa + 1, nb_total = nbx_r * (byb - bya + 1);
+    // no point of a bin is wide enough when its largest threshold is not
+    const double thr_min = dn_thr_min(L);
+#pragma unroll
+    for (int v = 0; v < 4; ++v) s[v] = 0.0;
+    f32x4 c = {0.0f, 0.0f, 0.0f, 0.0f};
+    int terms = 0, total = 0, turn = 0;   // turn: 64s of points seen, of all waves
+    int64_t ord = 0;
+    for (int base = 0; base < nb_total; base += 64) {
+        const int k = base + lane;
+        const int kc = k < nb_total ? k : nb_total - 1;
+        const int b = (bya + kc / nbx_r) * I.bg.nbx + (bxa + kc % nbx_r);
+        int p0 = I.bin_start[b], p1 = I.bin_start[b + 1];
+        const double lim = I.bin_thr[b];
+        bool on = k < nb_total && p1 > p0 && box_gap2(I.bin_box[b], bx0, bx1, by0, by1) < lim;
+        if (split) {
+            const int cnt = on ? p1 - p0 : 0;
+            const unsigned incl = wave_incl_scan((unsigned)cnt, lane);
+            const int64_t o1 = ord + incl, o0 = o1 - cnt;
+            ord += (unsigned)__builtin_amdgcn_readlane((int)incl, 63);
+            on = on && o1 > win0 && o0 < win1;
+            if (win1 < o1) p1 -= (int)(o1 - win1);
+            if (win0 > o0) p0 += (int)(win0 - o0);
+        }
+        uint64_t m = __ballot(on && lim >= thr_min);
+        while (m) {
+            const int l = __builtin_ctzll(m);
+            m &= m - 1ull;
+            const int a = __builtin_amdgcn_readlane(p0, l), e = __builtin_amdgcn_readlane(p1, l);
+            for (int st = a; st < e; st += 64) {
+                if ((turn++ & 3) != wave) continue;
+                const int i = st + lane;
+                PtRec p{};
+                bool take = false;
+                if (i < e) {
+                    p = I.pts[i];
+                    take = p.thr > 0.0 && dn_wide(p.a, L) && sq2(far1(p.x, bx0, bx1), far1(p.y, by0, by1)) < p.thr;
+                }
+                const uint64_t tm = __ballot(take);
+                if (!tm) continue;
+                const int cnt = __popcll(tm);
+                total += cnt;
+                // taken points to the front lanes, the others behind them
+                const uint64_t below = ((uint64_t)1 << lane) - 1;
+                const int to = 4 * (take ? __popcll(tm & below) : cnt + __popcll(~tm & below));
+                const double pa = p.a;
+                const int alo = __builtin_amdgcn_ds_permute(to, __double2loint(pa));
+                const int ahi = __builtin_amdgcn_ds_permute(to, __double2hiint(pa));
+                const int px = __builtin_amdgcn_ds_permute(to, __builtin_bit_cast(int, p.x));
+                const int py = __builtin_amdgcn_ds_permute(to, __builtin_bit_cast(int, p.y));
+                const int pc = __builtin_amdgcn_ds_permute(to, __builtin_bit_cast(int, take ? p.coef : 0.0f));
+                for (int g = 0; g < cnt; g += 4) {
+                    // lane l: point g + l / 16 (past the end: one without a weight)
+                    const int from = 4 * (g + (lane >> 4));
+                    const double qa = __hiloint2double(__builtin_amdgcn_ds_bpermute(from, ahi),
+                                                       __builtin_amdgcn_ds_bpermute(from, alo));
+                    const float qx = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(from, px));
+                    const float qy = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(from, py));
+                    const float qc = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(from, pc));
+                    const bool in = g + (lane >> 4) < cnt;
+                    const double dx = nx - (double)qx, dy = ny - (double)qy;
+                    const float ex = fast_exp2((float)(dx * dx * qa)), ey = fast_exp2((float)(dy * dy * qa)) * qc;
+                    c = __builtin_amdgcn_mfma_f32_16x16x4f32(in ? ey : 0.0f, in ? ex : 0.0f, c, 0, 0, 0);
+                    if (++terms == 4) {   // 16 terms in FP32
+#pragma unroll
+                        for (int v = 0; v < 4; ++v) {
+                            s[v] += (double)c[v];
+                            c[v] = 0.0f;
+                        }
+                        terms = 0;
+                    }
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int v = 0; v < 4; ++v) s[v] += (double)c[v];
+    return total;
+}
+
+// Node sums of every item that has enough candidates and such points.
+__global__ __launch_bounds__(DT_NT) void k_density_nodes(TileArgs A)
+{
+    static_assert(DT_NW == 4 && DN_N * DN_N == DT_NT, "a node per thread");
+    __shared__ double s_part[DT_NW * DN_N * DN_N];
+    __shared__ int s_cnt[DT_NW];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int at = A.order[blockIdx.x];
+    const int4 item = A.items[at];
+    const int64_t C = A.cost[item.x];
+    const BlockGeom B = block_geom(A.g, A.tl, A.nbx, item.x);
+    const int64_t lc0 = B.c0 - B.xoff, lr0 = B.r0 - B.yoff, lc1 = B.c1 - B.xoff, lr1 = B.r1 - B.yoff;
+    const float bx0 = cell_x(B.xll, B.cs, lc0), bx1 = cell_x(B.xll, B.cs, lc1);
+    const float by1 = cell_y(B.yll, B.cs, B.nrm05, lr0), by0 = cell_y(B.yll, B.cs, B.nrm05, lr1);
+    const BlockNodes bn = block_nodes(bx0, bx1, by0, by1, B.cs);
+    const double reach = *A.idx.reach_p;
+    if (C / item.z < DN_CAND || reach * reach < dn_thr_min(bn.L)) {
+        if (tid == 0) A.node_on[at] = 0;
+        return;
+    }
+    int64_t win0 = 0, win1 = INT64_MAX;
+    if (item.y > 0) win0 = C * item.y / item.z;
+    if (item.y < item.z - 1) win1 = C * (item.y + 1) / item.z;
+    int bxa, bxb, bya, byb;
+    bin_range(A.idx.bg, bx0, bx1, by0, by1, reach, bxa, bxb, bya, byb);
+    double s[4];
+    const int got = dn_sums(A.idx, bxa, bxb, bya, byb, item.z > 1, win0, win1, bx0, bx1, by0, by1, bn.mx, bn.my, bn.L, s);
+#pragma unroll
+    for (int v = 0; v < 4; ++v) s_part[wave * 256 + (4 * (lane >> 4) + v) * DN_N + (lane & 15)] = s[v];
+    if (lane == 0) s_cnt[wave] = got;
+    __syncthreads();
+    const bool on = s_cnt[0] + s_cnt[1] + s_cnt[2] + s_cnt[3] >= DN_MIN;
+    if (tid == 0) A.node_on[at] = on;
+    if (on) A.nodes[(int64_t)at * (DN_N * DN_N) + tid] = ((s_part[tid] + s_part[256 + tid]) + s_part[512 + tid]) + s_part[768 + tid];
+}
+
 // 4 waves per SIMD: at most 128 VGPRs (no spills).  64 x 64 blocks: 37.7 KB
 // of LDS per workgroup, 4 workgroups per CU, so each SIMD's 4 waves belong to
 // 4 workgroups and a barrier wait in one leaves 3 to issue.  (64 x 128
 // blocks share Ey and the reach over twice the columns, but at 55 KB and 8
 // waves only 2 workgroups fit per CU: measured 31.6 ms against 24.3 ms on
 // the adaptive 1M job.)
-template <bool STATS>
+template <bool STATS, bool NODES>
 __global__ __launch_bounds__(DT_NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_density_tile(TileArgs A)
 {
     __shared__ int s_bins[DT_NT];
@@ -571,6 +784,10 @@ __global__ __launch_bounds__(DT_NT) __attribute__((amdgpu_waves_per_eu(4, 4))) v
     bin_range(I.bg, bx0, bx1, by0, by1, *I.reach_p, bxa, bxb, bya, byb);
     const int nbx_r = bxb - bxa + 1;
     const int nb_total = nbx_r * (byb - bya + 1);
+
+    // wide kernels at the nodes (k_density_nodes)
+    const BlockNodes bn = block_nodes(bx0, bx1, by0, by1, cs);
+    const bool nodes = NODES && A.node_on[A.order[blockIdx.x]] != 0;
 
     int qn = 0;       // queue length (uniform)
     int npend = 0;    // sub-batches in acc since the last fold (uniform)
@@ -731,7 +948,8 @@ __global__ __launch_bounds__(DT_NT) __attribute__((amdgpu_waves_per_eu(4, 4))) v
             part4_8(acc[8], acc[9], acc[10], acc[11], xr[4], ex, eyv, dx);
             part4_12(acc[12], acc[13], acc[14], acc[15], xr[6], ex, eyv, dx);
         }
-        if (++npend == DT_FOLD) fold();
+        // (with node sums: every sub-batch, so that no raster loses precision)
+        if (NODES || ++npend == DT_FOLD) fold();
         __syncthreads();
     };
 
@@ -776,6 +994,10 @@ __global__ __launch_bounds__(DT_NT) __attribute__((amdgpu_waves_per_eu(4, 4))) v
                     }
                     if (STATS && cls == 1) ++st_full;
                     if (STATS && cls == 2) ++st_part;
+                    if (NODES && cls == 1 && nodes && dn_wide(p.a, bn.L)) {   // summed at the nodes
+                        cls = 0;
+                        if (STATS) st_wf += DT_NW;
+                    }
                 }
                 int na;
                 int pos = block_compact<DT_NW>(cls != 0, s_wcnt, &na);
@@ -828,6 +1050,25 @@ __global__ __launch_bounds__(DT_NT) __attribute__((amdgpu_waves_per_eu(4, 4))) v
     }
     if (qn > 0) process(qn, 0);
     if (npend > 0) fold();
+    if (NODES && nodes) {
+        // cell (row, column) += sum_i Wy[i][row] sum_j N[i][j] Wx[j][column]
+        static_assert(sizeof(s_ex) >= 64 * DN_N * sizeof(double) && sizeof(s_ey) >= 64 * DN_N * sizeof(double) &&
+                          MKDE_DT_BW == 64, "weights of the cells");
+        double *wx = (double *)s_ex, *wy = (double *)s_ey;
+        const double *N = A.nodes + (int64_t)__builtin_amdgcn_readfirstlane(A.order[blockIdx.x]) * (DN_N * DN_N);
+        __syncthreads();
+        if (tid < 64) dn_weights((double)s_ccx[tid], bn.mx, bn.L, wx + tid);
+        else if (tid < 128) dn_weights((double)s_ccy[tid - 64], bn.my, bn.L, wy + (tid - 64));
+        __syncthreads();
+#pragma unroll 1
+        for (int i = 0; i < DN_N; ++i) {
+            double t = 0.0;
+#pragma unroll
+            for (int j = 0; j < DN_N; ++j) t = __builtin_fma(N[i * DN_N + j], wx[64 * j + wc], t);
+#pragma unroll
+            for (int j = 0; j < 16; ++j) sum[j] = __builtin_fma(wy[64 * i + DT_ROW(wave, lane, j)], t, sum[j]);
+        }
+    }
 
     // write back: nodata cells keep the mask value; parts of a split block
     // leave FP64 partial sums for k_density_merge
@@ -957,15 +1198,6 @@ __device__ __forceinline__ unsigned split_threshold(unsigned long long total, co
 __device__ __forceinline__ unsigned split_parts(unsigned c, unsigned T)
 {
     return c > T ? (unsigned)(((unsigned long long)c + T - 1) / T) : 1u;
-}
-
-__device__ __forceinline__ unsigned wave_incl_scan(unsigned v, int lane)
-{
-    for (int d = 1; d < WAVE; d <<= 1) {
-        const unsigned o = __shfl_up(v, d, WAVE);
-        if (lane >= d) v += o;
-    }
-    return v;
 }
 
 // One workgroup of 1024 threads, four units per thread and step.  host
@@ -3290,15 +3522,23 @@ hipError_t work_items(hipStream_t s, int n, const WorkList &W, int4 *items, int4
 }
 
 // order == nullptr: one item per block in raster order; else n_items items.
+// nodes, node_on: non-null where wide kernels are summed at nodes (with order).
 hipError_t density_tile(hipStream_t s, const GridDesc &g, const float *mask, float *out, const PointIndex &idx,
                         unsigned long long *stats, const int *order, const int4 *items, const unsigned *cost,
-                        double *partials, int n_items, const Tiling &tl)
+                        double *partials, int n_items, const Tiling &tl, double *nodes, int *node_on)
 {
     const int nbx = (int)((g.ncols + MKDE_DT_BW - 1) / MKDE_DT_BW);
-    TileArgs A{g, mask, out, idx, stats, order, items, cost, partials, nbx, tl};
+    TileArgs A{g, mask, out, idx, stats, order, items, cost, partials, nbx, tl, nodes, node_on};
     dim3 grid((unsigned)(order ? n_items : raster_blocks(g, tl)));
-    if (stats) hipLaunchKernelGGL(k_density_tile<true>, grid, dim3(DT_NT), 0, s, A);
-    else hipLaunchKernelGGL(k_density_tile<false>, grid, dim3(DT_NT), 0, s, A);
+    if (order && nodes) {
+        hipLaunchKernelGGL(k_density_nodes, grid, dim3(DT_NT), 0, s, A);
+        if (stats) hipLaunchKernelGGL(HIP_KERNEL_NAME(k_density_tile<true, true>), grid, dim3(DT_NT), 0, s, A);
+        else hipLaunchKernelGGL(HIP_KERNEL_NAME(k_density_tile<false, true>), grid, dim3(DT_NT), 0, s, A);
+    } else if (stats) {
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_density_tile<true, false>), grid, dim3(DT_NT), 0, s, A);
+    } else {
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_density_tile<false, false>), grid, dim3(DT_NT), 0, s, A);
+    }
     return hipGetLastError();
 }
 

@@ -136,6 +136,9 @@ extern "C" int64_t mkde_job_footprint(int64_t n, int64_t ncols, int64_t nrows, i
     const double nblk = (double)((ncols + MKDE_DT_BW - 1) / MKDE_DT_BW) * (double)((nrows + 63) / 64);
     b += (int64_t)std::min(2.0 * (double)tune.dt_target, 2.0 * (double)n * nblk / 2048.0 + nblk) *
          (8 * MKDE_DT_CELLS);
+    // node sums of its items, from the split threshold MKDE_DN_SPLIT on
+    if ((double)n * nblk >= (double)MKDE_DN_SPLIT * (double)tune.dt_target)
+        b += (int64_t)(nblk + 2.0 * (double)tune.dt_target) * (8 * MKDE_DN_CELLS + 4);
     // work lists of the point kernels at their largest (point_work_bounds):
     // items (20 B each) and FP64 partials of split 64-query waves, 512 B per
     // part for densities at points and 8 KB per part for a 16-candidate pass
