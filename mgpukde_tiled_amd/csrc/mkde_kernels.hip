@@ -1705,81 +1705,73 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
     }
 }
 
-typedef float f32x8 __attribute__((ext_vector_type(8)));
-
-// The other sources, pair by pair, and the total.
+// The other sources, pair by pair, and the total.  A group's records come in one
+// per lane and are handed round through LDS.  Bound by instruction issue, 8 or 12
+// a pair.  (Scalar loads, four records at a time: 3.66 ms on 1M clustered points, 2.71 ms now.)
 template <bool LOO>
 __global__ __launch_bounds__(256) void k_point_density_f(PtsArgs A)
 {
+    __shared__ float4 s_a[4][64];   // x, y, coef, af
+    __shared__ float2 s_b[4][64];   // lo, hi
     const PointIndex &I = A.idx;
     const SrcRec *src = (const SrcRec *)I.pts;
     const int lane = threadIdx.x & 63;
     FineItem T;
     if (!fine_item(A, T)) return;
+    float4 *pa = s_a[threadIdx.x >> 6];
+    float2 *pb = s_b[threadIdx.x >> 6];
     const int q = T.q;
     const bool qv = q < I.n;
     const float qx = qv ? src[q].x : T.W.x0, qy = qv ? src[q].y : T.W.y0;
-    float acc = 0.0f, sum = 0.0f, comp = 0.0f;
+    float sum = 0.0f, comp = 0.0f;
     fine_walk<LOO, false>(I, T, [&](int c0, int c1, bool all) {
         // the query itself is left out of its own group's sums
         const bool self = LOO && (c0 >> 6) == T.item.x;
-        for (int s0 = c0; s0 < c1; s0 += 32) {
-            const int s1 = s0 + 32 < c1 ? s0 + 32 : c1;
-            // four records are loaded before their arithmetic, so the scalar
-            // loads overlap
+        wave_sync();
+        if (c0 + lane < c1) {
+            const SrcRec p = src[c0 + lane];
+            pa[lane] = make_float4(p.x, p.y, p.coef, p.af);
+            pb[lane] = make_float2(p.lo, p.hi);
+        }
+        wave_sync();
+        for (int s0 = 0; s0 < c1 - c0; s0 += 32) {
+            const int s1 = s0 + 32 < c1 - c0 ? s0 + 32 : c1 - c0;
+            float acc = 0.0f;
+            bool band = self;
             if (all) {
-                auto body = [&](const SrcRec &p) {
+#pragma unroll 4
+                for (int j = s0; j < s1; ++j) {
+                    const float4 p = pa[j];
                     const float dx = p.x - qx, dy = p.y - qy;
                     const float d2f = __builtin_fmaf(dy, dy, dx * dx);
-                    acc = __builtin_fmaf(fast_exp2(d2f * p.af), p.coef, acc);
-                };
-                int si = s0;
-                for (; si + 4 <= s1; si += 4) {
-                    const SrcRec p0 = src[si], p1 = src[si + 1], p2 = src[si + 2], p3 = src[si + 3];
-                    body(p0);
-                    body(p1);
-                    body(p2);
-                    body(p3);
+                    acc = __builtin_fmaf(fast_exp2(d2f * p.w), p.z, acc);
                 }
-                for (; si < s1; ++si) body(src[si]);
-            } else {
-                bool band = self;
-                auto body = [&](const f32x8 &p) {
-                    const float dx = p[0] - qx, dy = p[1] - qy;
+            } else if (!self) {
+#pragma unroll 4
+                for (int j = s0; j < s1; ++j) {
+                    const float4 p = pa[j];
+                    const float2 t = pb[j];
+                    const float dx = p.x - qx, dy = p.y - qy;
                     const float d2f = __builtin_fmaf(dy, dy, dx * dx);
-                    const bool in = d2f < p[4];
-                    band |= !(d2f > p[5]) != in;
-                    const float e = fast_exp2(d2f * p[3]);
-                    acc = __builtin_fmaf(in ? e : 0.0f, p[2], acc);
-                };
-                // whole records, one scalar load each
-                const f32x8 *rec = (const f32x8 *)src;
-                int si = s0;
-                if (!self) {
-                    for (; si + 4 <= s1; si += 4) {
-                        const f32x8 p0 = rec[si], p1 = rec[si + 1], p2 = rec[si + 2], p3 = rec[si + 3];
-                        body(p0);
-                        body(p1);
-                        body(p2);
-                        body(p3);
-                    }
-                    for (; si < s1; ++si) body(rec[si]);
+                    const bool in = d2f < t.x;
+                    band |= !(d2f > t.y) != in;
+                    const float e = fast_exp2(d2f * p.w);
+                    acc = __builtin_fmaf(in ? e : 0.0f, p.z, acc);
                 }
-                if (__any(band)) {   // rare, and the wave's own group: exact FP64 test
-                    acc = 0.0f;
-                    for (int sj = s0; sj < s1; ++sj) {
-                        const SrcRec p = src[sj];
-                        const float dx = p.x - qx, dy = p.y - qy;
-                        const float d2f = __builtin_fmaf(dy, dy, dx * dx);
-                        bool in = sq2(dx, dy) < p.thr;
-                        if (LOO && sj == q) in = false;
-                        const float e = fast_exp2(d2f * p.af);
-                        acc = __builtin_fmaf(in ? e : 0.0f, p.coef, acc);
-                    }
+            }
+            if (__any(band)) {   // rare, and the wave's own group: exact FP64 test
+                acc = 0.0f;
+                for (int j = s0; j < s1; ++j) {
+                    const float4 p = pa[j];
+                    const float dx = p.x - qx, dy = p.y - qy;
+                    const float d2f = __builtin_fmaf(dy, dy, dx * dx);
+                    bool in = sq2(dx, dy) < src[c0 + j].thr;
+                    if (LOO && c0 + j == q) in = false;
+                    const float e = fast_exp2(d2f * p.w);
+                    acc = __builtin_fmaf(in ? e : 0.0f, p.z, acc);
                 }
             }
             kahan_fold(acc, sum, comp);
-            acc = 0.0f;
         }
     });
     const double den = (double)sum - (double)comp;
