@@ -1774,7 +1774,8 @@ extern "C" int mkde_density_tile_resident(mkde_ctx *c)
         CHK(c->dt_order.ensure(n_items));
         CHK(c->dt_splits.ensure(n_split));
         CHK(c->dt_partials.ensure((size_t)c->host_words[1] * MKDE_DT_CELLS));
-        nodes = c->host_words[3] >= MKDE_DN_SPLIT;
+        nodes = c->host_words[3] >= MKDE_DN_SPLIT &&
+                *(const double *)(c->host_words + 4) >= MKDE_DN_REACH * (double)c->tg.cs;
         if (nodes) {
             CHK(c->dt_nodes.ensure((size_t)n_items * MKDE_DN_CELLS));
             CHK(c->dt_node_on.ensure(n_items));

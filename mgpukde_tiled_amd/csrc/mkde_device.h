@@ -138,6 +138,8 @@ struct PointIndex {
 // (candidates of an item) is at least this.
 #define MKDE_DN_CELLS 256
 #define MKDE_DN_SPLIT 4096
+// Cells that some point's cut-off radius must reach: 3 * 31.5 / (2 * 0.65).
+#define MKDE_DN_REACH 72.7
 
 // A raster processed as tiles of tw x th cells, each tile with its own origin
 // from the raster geotransform (GDAL order gt0, gt1, gt3, gt5).  Density
