@@ -1201,7 +1201,7 @@ __global__ __launch_bounds__(256) void k_density_merge(GridDesc g, Tiling tl, in
 // then every unit writes its items and takes their places in the order
 // (k_work_items).  With each of those in a launch of its own a list took 16
 // launches, ~70 us of a small job; one workgroup needs 4 us at 1,000 units and
-// 25 us at 16,384.
+// 31 us at 16,384 (66 us with the buckets counted by ballots).
 #define DT_TMIN 2048u
 #define DT_TARGET 4096ull
 
@@ -1227,13 +1227,13 @@ __global__ __launch_bounds__(1024) void k_work_scan(int n, SplitRule rule, WorkL
 {
     __shared__ unsigned long long s_t[16];
     __shared__ unsigned s_w[16][3];
-    __shared__ unsigned s_h[32];
+    __shared__ unsigned s_h[16][32];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     unsigned long long acc = 0;
     for (int i = tid; i < n; i += 1024) acc += W.cost[i];
     for (int d = 32; d >= 1; d >>= 1) acc += __shfl_xor(acc, d, WAVE);
     if (lane == 0) s_t[wave] = acc;
-    if (tid < 32) s_h[tid] = 0;
+    if (tid < 512) s_h[tid >> 5][tid & 31] = 0;
     __syncthreads();
     unsigned long long total = 0;
     for (int w = 0; w < 16; ++w) total += s_t[w];
@@ -1285,21 +1285,10 @@ __global__ __launch_bounds__(1024) void k_work_scan(int n, SplitRule rule, WorkL
                 op += k[j];
             }
         }
-        // bucket sizes: the lanes of a wave share few buckets, so each is added
-        // once per wave
+        // bucket sizes, a copy per wave
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int bk = k[j] ? cost_bucket(c[j] / k[j]) : -1;
-            uint64_t todo = __ballot(bk >= 0);
-            while (todo) {
-                const int b = __builtin_amdgcn_readlane(bk, __builtin_ctzll(todo));
-                const uint64_t same = __ballot(bk == b);
-                unsigned v = bk == b ? k[j] : 0u;
-                for (int d = 32; d >= 1; d >>= 1) v += __shfl_xor(v, d, WAVE);
-                if (lane == 0) atomicAdd(&s_h[b], v);
-                todo &= ~same;
-            }
-        }
+        for (int j = 0; j < 4; ++j)
+            if (k[j]) atomicAdd(&s_h[wave][cost_bucket(c[j] / k[j])], k[j]);
         __syncthreads();
     }
     if (tid == 0) {
@@ -1312,7 +1301,7 @@ __global__ __launch_bounds__(1024) void k_work_scan(int n, SplitRule rule, WorkL
         unsigned run = 0;
         for (int b = 0; b < 32; ++b) {
             W.hist[b] = run;
-            run += s_h[b];
+            for (int w = 0; w < 16; ++w) run += s_h[w][b];
         }
     }
 }
