@@ -10,9 +10,9 @@ namespace mkde_copy {
 // runtime reads the caller's pages in place and needs no staging: lanes win only
 // where several threads' worth of copying is to be had (repeated copies of
 // 8 / 16 / 64 MB: 326 / 617 / 2400 us without, 260 / 455 / 1440 us with lanes, but a
-// single 16 MB mask on a new context 790 against 960 us; a 21 MB tile mask a call, warm, 300 us less with lanes).  From the
-// device: 2 / 4 / 16 / 64 MB 131 / 252 / 1030 / 6750 us without, 127 / 190 / 446 /
-// 1890 us with lanes.
+// single 16 MB mask on a new context 790 against 960 us; a 21 MB tile mask a call,
+// warm, 300 us less with lanes).  From the device: 2 / 4 / 16 / 64 MB 131 / 252 /
+// 1030 / 6750 us without, 127 / 190 / 446 / 1890 us with lanes.
 constexpr size_t MIN_TO_DEVICE = (size_t)20 << 20;
 constexpr size_t MIN_TO_HOST = (size_t)1 << 20;
 // Contexts that share the device with others (the job server's), either way.
