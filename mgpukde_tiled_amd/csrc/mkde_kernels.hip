@@ -193,6 +193,11 @@ __global__ void k_prep_points(int64_t n, const int *perm, const float *xs, const
     out[i] = r;
 }
 
+// Whether a source may enter a sum whose weights have both signs (moments of a
+// group, nodes of a block): an infinite coefficient, or one whose float sums may
+// overflow, would cancel to NaN there, while its kernels add up to +inf.
+__device__ __forceinline__ bool coef_signed_ok(float coef) { return fabsf(coef) < 1e30f; }
+
 // A float squared distance below lo is inside the cut-off thr, one above hi is
 // not.  fl32(dx^2 + dy^2) is within 2^-22 relative where it neither overflows nor
 // becomes subnormal; elsewhere nothing is taken as decided (lo = -1, a hi that
@@ -205,7 +210,8 @@ __device__ __forceinline__ void thr_bracket(double thr, float &lo, float &hi)
 }
 
 // The same in fine order (SrcRec, one wave per group of 64), with each group's
-// box and thresholds.
+// box and thresholds.  A group with a coefficient that must not enter the moments
+// gets a smallest threshold that no pair is inside.
 __global__ __launch_bounds__(256) void k_prep_fine(int64_t n, const int *perm, const float *xs, const float *ys,
                                                    const float *w_orig, const float *h_orig, const float *ew_orig,
                                                    float h_fixed, SrcRec *out, GroupInfo *grp)
@@ -231,7 +237,7 @@ __global__ __launch_bounds__(256) void k_prep_fine(int64_t n, const int *perm, c
         out[i] = r;
     }
     float x0 = on ? r.x : FLT_MAX, y0 = on ? r.y : FLT_MAX, x1 = on ? r.x : -FLT_MAX, y1 = on ? r.y : -FLT_MAX;
-    double lo = on ? r.thr : DBL_MAX, hi = on ? r.thr : -DBL_MAX;
+    double lo = on ? (coef_signed_ok(r.coef) ? r.thr : -1.0) : DBL_MAX, hi = on ? r.thr : -DBL_MAX;
     for (int d = 32; d >= 1; d >>= 1) {
         x0 = fminf(x0, __shfl_xor(x0, d, WAVE));
         x1 = fmaxf(x1, __shfl_xor(x1, d, WAVE));
@@ -519,9 +525,9 @@ __device__ __forceinline__ BlockNodes block_nodes(float bx0, float bx1, float by
 
 // Whether a point that is FULL for a block of half extent L goes to the nodes:
 // L <= 2 DN_KAPPA h, a = -log2(e) / (2 h^2).
-__device__ __forceinline__ bool dn_wide(double a, double L)
+__device__ __forceinline__ bool dn_wide(const PtRec &p, double L)
 {
-    return L * L * -a <= 2.0 * DN_KAPPA * DN_KAPPA * MKDE_LOG2E;
+    return L * L * -p.a <= 2.0 * DN_KAPPA * DN_KAPPA * MKDE_LOG2E && coef_signed_ok(p.coef);
 }
 
 // Interpolation weights of a cell at v (centre mid, half extent L) to w[64 j],
@@ -591,7 +597,7 @@ __device__ __forceinline__ int dn_sums(const PointIndex &I, int bxa, int bxb, in
                 bool take = false;
                 if (i < e) {
                     p = I.pts[i];
-                    take = p.thr > 0.0 && dn_wide(p.a, L) && sq2(far1(p.x, bx0, bx1), far1(p.y, by0, by1)) < p.thr;
+                    take = p.thr > 0.0 && dn_wide(p, L) && sq2(far1(p.x, bx0, bx1), far1(p.y, by0, by1)) < p.thr;
                 }
                 const uint64_t tm = __ballot(take);
                 if (!tm) continue;
@@ -997,7 +1003,7 @@ __global__ __launch_bounds__(DT_NT) __attribute__((amdgpu_waves_per_eu(4, 4))) v
                     }
                     if (STATS && cls == 1) ++st_full;
                     if (STATS && cls == 2) ++st_part;
-                    if (NODES && cls == 1 && dn_wide(p.a, bn.L)) {   // summed at the nodes
+                    if (NODES && cls == 1 && dn_wide(p, bn.L)) {   // summed at the nodes
                         cls = 0;
                         if (STATS) st_wf += DT_NW;
                     }
@@ -1716,7 +1722,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
     }
 }
 
-// The other sources, pair by pair, and the total.  A group's records come in one
+// The other sources, pair by pair, and the total.  (The select is on the
+// coefficient: an infinite one adds nothing outside its cut-off.)  A group's records come in one
 // per lane and are handed round through LDS.  Bound by instruction issue, 8 or 12
 // a pair.  (Scalar loads, four records at a time: 3.66 ms on 1M clustered points, 2.71 ms now.)
 template <bool LOO>
@@ -1767,7 +1774,7 @@ __global__ __launch_bounds__(256) void k_point_density_f(PtsArgs A)
                     const bool in = d2f < t.x;
                     band |= !(d2f > t.y) != in;
                     const float e = fast_exp2(d2f * p.w);
-                    acc = __builtin_fmaf(in ? e : 0.0f, p.z, acc);
+                    acc = __builtin_fmaf(e, in ? p.z : 0.0f, acc);
                 }
             }
             if (__any(band)) {   // rare, and the wave's own group: exact FP64 test
@@ -1779,10 +1786,11 @@ __global__ __launch_bounds__(256) void k_point_density_f(PtsArgs A)
                     bool in = sq2(dx, dy) < src[c0 + j].thr;
                     if (LOO && c0 + j == q) in = false;
                     const float e = fast_exp2(d2f * p.w);
-                    acc = __builtin_fmaf(in ? e : 0.0f, p.z, acc);
+                    acc = __builtin_fmaf(e, in ? p.z : 0.0f, acc);
                 }
             }
             kahan_fold(acc, sum, comp);
+            if (!(fabsf(sum) < INFINITY)) comp = 0.0f;   // an infinite sum stays one
         }
     });
     const double den = (double)sum - (double)comp;
