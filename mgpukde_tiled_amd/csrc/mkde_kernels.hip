@@ -2592,25 +2592,98 @@ __device__ __forceinline__ double node_lb(float4 b, float px, float py)
 // bound is not below the best squared distance so far: the result is the
 // brute-force minimum over all boundary cells, exactly.  One wave searches for
 // 64 neighbouring points (bin order).
-//   1. Each lane walks down to one leaf, nearest child first, and takes its
-//      cells: a good first distance of its own.
-//   2. The wave keeps one stack of nodes (LDS).  Up to 64 nodes are popped at a
-//      time, one per lane, with their loads in flight together; children within
-//      the largest distance of the wave's bounding box are pushed.  Leaves are
-//      then taken one by one for all 64 points, where any point needs them: the
-//      leaf's cells are listed in LDS, four at a time are taken without waiting
-//      on each other.
-// What bounds it is the longest search: points near the centre of a round study
-// area find hundreds of leaves nearly equidistant.  Node by node a search costs
-// a memory latency each, so nodes are taken 64 at a time; with a search per
-// lane, lanes popped nodes and scanned leaves in turn (50,000
-// points in a disk of radius 570 cells 303 -> 58 us, 1M points in one of radius
-// 3,900 1080 -> 338 us; one node at a time for the whole wave: 218 and 1173 us).
+//   1. Every lane searches by itself, nearest child first, down to a leaf.
+//   2. The points that are still open go on together where they lie close
+//      together compared with their distances (BT_WAVE_AREA): the wave keeps one
+//      stack of nodes (LDS).  Up to 64 nodes are popped at a time, one per lane,
+//      with their loads in flight together; children within the largest distance
+//      of the open points' box are pushed.  Leaves are then taken one by one for
+//      all of them, where any needs them: the leaf's cells are listed in LDS, four
+//      at a time are taken without waiting on each other.
+//   3. What is left, where the wave did not search or gave up, every lane finishes
+//      by itself.  The wave gives up when too few points need the leaves it
+//      visits: a leaf costs it BT_COST and pays back one a point.
+// What bounds a search is its longest one: points near the centre of a round study
+// area find hundreds of leaves nearly equidistant, and node by node each costs a
+// memory latency, so there the wave takes nodes 64 at a time.  Near a ragged
+// boundary every point needs a few leaves of its own and the wave would look at
+// all leaves around: 64 points on 8192^2 cells with 2% nodata cells 120 us with a
+// stack per lane, 33.8 ms by the wave alone, 77 us now; half the raster like that
+// and half without, 200,000 points 301 / 1863 / 261 us; a coast, 1M points 868 /
+// 1655 / 312 us; a disk with 20 holes, 1M points 1258 / 331 / 380 us; a plain disk
+// on 4096^2, 200,000 points 6.2 / 0.76 / 0.78 ms (times with the flags and the
+// hierarchy, 70 to 150 us).
 
 #define BT_STACK 1024
 // Nodes popped at a time are limited so that their children fit below this; at
 // the limit nodes go one by one, which needs at most 3 more per level.
 #define BT_STACK_SOFT (BT_STACK - 64)
+// The wave looks at the leaves within far of the open points' box, a lane at those
+// within far of its point.  Area of the first in far^2 up to which the wave starts,
+// its cost of a leaf, and what it may lose before it gives up.  (Areas of 10 and 25:
+// 64 points on 2048^2 cells without holes 102 and 184 us.  Cost 8 / 2 / 1: the disk's
+// 200,000 points 3.4 / 0.78 / 0.78 ms, the half ragged raster's 200 / 261 / 400 us.)
+#define BT_WAVE_AREA 10.0
+#define BT_COST 2
+#define BT_CREDIT 512
+
+// A lane's search, depth first: at node (ix, iy) of level lev, with the children
+// that are left at the nodes above in 4 bits a level (level l in bits 4 l - 4 ..
+// 4 l - 1; none below lev), so it needs no stack.
+struct LaneSearch {
+    int lev, ix, iy;
+    uint64_t todo;
+};
+
+__device__ __forceinline__ void leaf_best(const GridDesc &g, const BndTree &T, int ix, int iy, double nrm05, float px,
+                                          float py, double &best)
+{
+    const int64_t at = bt_node(ix, iy, T.nx[1]);
+    const uint4 m0 = T.bits[2 * at], m1 = T.bits[2 * at + 1];
+    const unsigned m[8] = {m0.x, m0.y, m0.z, m0.w, m1.x, m1.y, m1.z, m1.w};
+#pragma unroll
+    for (int w = 0; w < 8; ++w) {
+        unsigned v = m[w];
+        while (v) {
+            const int k = w * 32 + __builtin_ctz(v);
+            v &= v - 1u;
+            const float cx = cell_x(g.xll, g.cs, (int64_t)ix * MKDE_BT_S + (k & (MKDE_BT_S - 1)));
+            const float cy = cell_y(g.yll, g.cs, nrm05, (int64_t)iy * MKDE_BT_S + (k >> 4));
+            best = fmin(best, sq2(cx - px, cy - py));
+        }
+    }
+}
+
+// One step (todo != 0): back to the lowest node with children left, and to the
+// nearest of them; a leaf's cells are taken.
+__device__ __forceinline__ void lane_step(const GridDesc &g, const BndTree &T, double nrm05, float px, float py,
+                                          LaneSearch &L, double &best)
+{
+    const int at = __builtin_ctzll(L.todo) & ~3, up = (at >> 2) + 1 - L.lev;
+    L.lev += up;
+    L.ix >>= up;
+    L.iy >>= up;
+    const float4 *ch = T.box + T.off[L.lev - 1] + (((int64_t)L.iy * T.nx[L.lev] + L.ix) << 2);
+    const unsigned left = (unsigned)(L.todo >> at) & 15u;
+    unsigned rest = 0;
+    double lb = best;
+    int k = -1;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const double l = (left >> j) & 1u ? node_lb(ch[j], px, py) : DBL_MAX;
+        rest |= l < best ? 1u << j : 0u;
+        k = l < lb ? j : k;
+        lb = l < lb ? l : lb;
+    }
+    L.todo &= ~((uint64_t)15 << at);
+    if (k < 0) return;
+    L.todo |= (uint64_t)(rest & ~(1u << k)) << at;
+    L.ix = 2 * L.ix + (k & 1);
+    L.iy = 2 * L.iy + (k >> 1);
+    --L.lev;
+    if (L.lev > 0) L.todo |= (uint64_t)15 << (at - 4);
+    else leaf_best(g, T, L.ix, L.iy, nrm05, px, py, best);
+}
 
 __global__ __launch_bounds__(64) void k_dist_tree(int64_t n, const float *xs, const float *ys, const int *perm,
                                                   GridDesc g, BndTree T, double *dist)
@@ -2620,55 +2693,40 @@ __global__ __launch_bounds__(64) void k_dist_tree(int64_t n, const float *xs, co
     const int lane = threadIdx.x;
     const int64_t i = (int64_t)blockIdx.x * 64 + lane;
     const bool on = i < n;
-    // lanes without a point repeat the last one
-    const int64_t is = on ? i : n - 1;
-    const float px = xs[is], py = ys[is];
-    const float wx0 = uni(wave_min(px)), wx1 = uni(wave_max(px)), wy0 = uni(wave_min(py)), wy1 = uni(wave_max(py));
+    const float px = xs[on ? i : n - 1], py = ys[on ? i : n - 1];
     const double nrm05 = (double)g.nrows - 0.5;
+    const int top = T.nlev - 1;
     double best = DBL_MAX;
 
-    // 1. a first distance per lane
-    int lx = 0, ly = 0;
-    for (int lev = T.nlev - 1; lev > 0; --lev) {
-        const float4 *ch = T.box + T.off[lev - 1] + (((int64_t)ly * T.nx[lev] + lx) << 2);
-        double lb = DBL_MAX;
-        int k = 0;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const double l = node_lb(ch[j], px, py);
-            k = l < lb ? j : k;
-            lb = l < lb ? l : lb;
-        }
-        lx = 2 * lx + (k & 1);
-        ly = 2 * ly + (k >> 1);
-    }
-    {
-        const int64_t at = bt_node(lx, ly, T.nx[1]);
-        const uint4 m0 = T.bits[2 * at], m1 = T.bits[2 * at + 1];
-        const unsigned m[8] = {m0.x, m0.y, m0.z, m0.w, m1.x, m1.y, m1.z, m1.w};
-#pragma unroll
-        for (int w = 0; w < 8; ++w) {
-            unsigned v = m[w];
-            while (v) {
-                const int k = w * 32 + __builtin_ctz(v);
-                v &= v - 1u;
-                const float cx = cell_x(g.xll, g.cs, (int64_t)lx * MKDE_BT_S + (k & (MKDE_BT_S - 1)));
-                const float cy = cell_y(g.yll, g.cs, nrm05, (int64_t)ly * MKDE_BT_S + (k >> 4));
-                best = fmin(best, sq2(cx - px, cy - py));
-            }
-        }
-    }
-    auto wave_best = [&]() {
-        double v = best;
+    // 1. (and 3., where the points lie far apart)
+    LaneSearch L{top, 0, 0, on && top > 0 ? (uint64_t)15 << (4 * top - 4) : 0ull};
+    if (top == 0 && on) leaf_best(g, T, 0, 0, nrm05, px, py, best);
+    int steps = top;
+    float wx0 = 0.0f, wx1 = 0.0f, wy0 = 0.0f, wy1 = 0.0f;   // box of the open points
+    double far = 0.0;   // no node beyond this is needed
+    auto wave_far = [&]() {
+        double v = L.todo ? best : 0.0;
         for (int d = 32; d >= 1; d >>= 1) v = fmax(v, __shfl_xor(v, d, WAVE));
         return v;
     };
-    double far = wave_best();   // no node beyond this is needed
+    while (__ballot(L.todo != 0)) {
+        if (steps-- == 0) {
+            wx0 = uni(wave_min(L.todo ? px : FLT_MAX));
+            wx1 = uni(wave_max(L.todo ? px : -FLT_MAX));
+            wy0 = uni(wave_min(L.todo ? py : FLT_MAX));
+            wy1 = uni(wave_max(L.todo ? py : -FLT_MAX));
+            far = wave_far();
+            const double f = sqrt(far), w = (double)wx1 - (double)wx0 + 2.0 * f, h = (double)wy1 - (double)wy0 + 2.0 * f;
+            if (w * h <= BT_WAVE_AREA * far) break;
+        }
+        if (L.todo) lane_step(g, T, nrm05, px, py, L, best);
+    }
 
-    // 2. the rest
-    if (lane == 0) s_node[0] = (unsigned)(T.nlev - 1) << 28;
-    int sp = 1;
-    while (sp > 0) {
+    // 2. the open ones together
+    const bool open = L.todo != 0;
+    if (lane == 0) s_node[0] = (unsigned)top << 28;
+    int sp = __ballot(open) ? 1 : 0, credit = BT_CREDIT;
+    while (sp > 0 && credit >= 0) {
         wave_sync();
         const int room = (BT_STACK_SOFT - sp) / 3;
         int take = sp < 64 ? sp : 64;
@@ -2701,7 +2759,9 @@ __global__ __launch_bounds__(64) void k_dist_tree(int64_t n, const float *xs, co
                 auto get = [&](unsigned v) { return (unsigned)__builtin_amdgcn_readlane((int)v, l); };
                 auto getf = [&](float v) { return __uint_as_float(get(__float_as_uint(v))); };
                 const float4 lb = make_float4(getf(own.x), getf(own.y), getf(own.z), getf(own.w));
-                if (!__ballot(node_lb(lb, px, py) < best)) continue;
+                const uint64_t who = __ballot(open && node_lb(lb, px, py) < best);
+                credit += __popcll(who) - BT_COST;
+                if (!who) continue;
                 const uint64_t m[4] = {get(m0.x) | (uint64_t)get(m0.y) << 32, get(m0.z) | (uint64_t)get(m0.w) << 32,
                                        get(m1.x) | (uint64_t)get(m1.y) << 32, get(m1.z) | (uint64_t)get(m1.w) << 32};
                 const int64_t c0 = (int64_t)get((unsigned)ix) * MKDE_BT_S, r0 = (int64_t)get((unsigned)iy) * MKDE_BT_S;
@@ -2729,7 +2789,7 @@ __global__ __launch_bounds__(64) void k_dist_tree(int64_t n, const float *xs, co
                 }
                 wave_sync();
             } while (leaves);
-            far = wave_best();
+            far = wave_far();
         }
         // children of the other nodes
         if (__ballot(need && lev > 0)) {
@@ -2747,6 +2807,10 @@ __global__ __launch_bounds__(64) void k_dist_tree(int64_t n, const float *xs, co
             }
         }
     }
+    // 3. all has been seen, or each lane goes on where it was
+    if (sp == 0) L.todo = 0;
+    while (__ballot(L.todo != 0))
+        if (L.todo) lane_step(g, T, nrm05, px, py, L, best);
     if (on) dist[perm[i]] = best;
 }
 
