@@ -273,6 +273,7 @@ struct mkde_ctx {
     std::vector<uint64_t> s_key;
     // work list of the point kernels (64-query waves, heavy ones split)
     DevBuf<unsigned> pw_cost, pw_item0, pw_slot0, pw_sidx, pw_counts, pw_hist;
+    DevBuf<WorkChunk> pw_chunks;
     DevBuf<int4> pw_items, pw_splits;
     DevBuf<int> pw_order;
     DevBuf<double> pw_partials;
@@ -284,6 +285,7 @@ struct mkde_ctx {
     bool dt_order_on = true;
     int pts_per_bin = 64;   // target points per bin of the point index
     DevBuf<unsigned> blk_cost, blk_item0, blk_slot0, blk_sidx, blk_counts, blk_hist;
+    DevBuf<WorkChunk> blk_chunks;
     DevBuf<int4> dt_items, dt_splits;
     DevBuf<int> dt_order;
     DevBuf<double> dt_partials, dt_nodes;
@@ -1089,7 +1091,9 @@ static int point_list(mkde_ctx *c, int64_t nw, WorkList &W)
     CHK(c->pw_sidx.ensure(nw));
     CHK(c->pw_counts.ensure(4));
     CHK(c->pw_hist.ensure(32));
-    W = WorkList{c->pw_cost.p, c->pw_item0.p, c->pw_slot0.p, c->pw_sidx.p, c->pw_counts.p, c->pw_hist.p};
+    if (work_chunks(nw)) CHK(c->pw_chunks.ensure(work_chunks(nw)));
+    W = WorkList{c->pw_cost.p,   c->pw_item0.p, c->pw_slot0.p,  c->pw_sidx.p,
+                 c->pw_counts.p, c->pw_hist.p,  c->pw_chunks.p};
     return MKDE_OK;
 }
 
@@ -1219,21 +1223,16 @@ extern "C" int mkde_density_at_points_noalloc(mkde_ctx *c, int loo, float *den_d
     float *den_s = cv.take<float>((size_t)n);
     unsigned *cost = cv.take<unsigned>(nw), *item0 = cv.take<unsigned>(nw), *slot0 = cv.take<unsigned>(nw);
     unsigned *sidx = cv.take<unsigned>(nw);
-    // two words a wave and one per 1024 waves in reserve: the sizes that fit do
-    // not depend on how many scans the work list takes
-    (void)cv.take<unsigned>(nw);
-    (void)cv.take<unsigned>(nw);
-    (void)cv.take<unsigned>((nw + 1023) / 1024);
+    WorkChunk *chunks = work_chunks(nw) ? cv.take<WorkChunk>((size_t)work_chunks(nw)) : nullptr;
     unsigned *counts = cv.take<unsigned>(4);
     unsigned *hist = cv.take<unsigned>(32);
-    (void)cv.take<unsigned long long>(1);
     if (!cv.ok)
         return fail(MKDE_E_RANGE, "%lld points need %zu bytes of scratch, more than the %u available", (long long)n,
                     cv.used, MKDE_SCRATCH_BYTES);
     const bool fine = density_fine(c, loo);
     CHK(prep(c, fine));
     PointIndex I = index_of(c);
-    const WorkList W{cost, item0, slot0, sidx, counts, hist};
+    const WorkList W{cost, item0, slot0, sidx, counts, hist, chunks};
     HIPCHK(mkde_dev::point_plan(c->stream, I, c->h_fixed, nullptr, 0, mkde_dev::point_rule(loo ? 1 : 0, c->tune, false, !I.grp),
                                 W, c->host_words));
     HIPCHK(hipStreamSynchronize(c->stream));
@@ -1418,6 +1417,7 @@ static int loo_loglik_graph(mkde_ctx *c, int K, const std::vector<int> &ord, con
                               (uint64_t)(uintptr_t)c->pw_item0.p,
                               (uint64_t)(uintptr_t)c->pw_slot0.p, (uint64_t)(uintptr_t)c->pw_sidx.p,
                               (uint64_t)(uintptr_t)c->pw_counts.p, (uint64_t)(uintptr_t)c->pw_hist.p,
+                              (uint64_t)(uintptr_t)c->pw_chunks.p,
                               (uint64_t)(uintptr_t)c->pw_items.p,
                               (uint64_t)(uintptr_t)c->pw_order.p, (uint64_t)(uintptr_t)c->pw_splits.p,
                               (uint64_t)(uintptr_t)c->pw_partials.p, (uint64_t)(uintptr_t)c->partial.p,
@@ -1764,8 +1764,9 @@ extern "C" int mkde_density_tile_resident(mkde_ctx *c)
         CHK(c->blk_sidx.ensure(nblk));
         CHK(c->blk_counts.ensure(4));
         CHK(c->blk_hist.ensure(32));
-        const WorkList W{c->blk_cost.p, c->blk_item0.p,  c->blk_slot0.p,
-                         c->blk_sidx.p, c->blk_counts.p, c->blk_hist.p};
+        if (work_chunks(nblk)) CHK(c->blk_chunks.ensure(work_chunks(nblk)));
+        const WorkList W{c->blk_cost.p,   c->blk_item0.p, c->blk_slot0.p, c->blk_sidx.p,
+                         c->blk_counts.p, c->blk_hist.p,  c->blk_chunks.p};
         HIPCHK(mkde_dev::density_plan(c->stream, c->tg, tm, I, c->tl, W, c->tune, c->host_words));
         HIPCHK(hipStreamSynchronize(c->stream));
         n_items = (int)c->host_words[0];

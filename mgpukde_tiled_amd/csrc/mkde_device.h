@@ -152,6 +152,21 @@ struct Tiling {
     double gt0, gt1, gt3, gt5;
 };
 
+// Lists of more units than MKDE_WS_ONE are scanned by several workgroups, in chunks
+// of MKDE_WS_UNITS: a chunk's cost, {items, slots, split units} and items of each
+// cost bucket.
+#define MKDE_WS_ONE 16384
+#define MKDE_WS_UNITS 4096
+struct WorkChunk {
+    unsigned long long cost;
+    unsigned n[3];
+    unsigned hist[32];
+};
+inline int64_t work_chunks(int64_t units)
+{
+    return units > MKDE_WS_ONE ? (units + MKDE_WS_UNITS - 1) / MKDE_WS_UNITS : 0;
+}
+
 // Device buffers of a work list (per unit unless noted): costs, the exclusive
 // scan of the parts, and for split units the first partial slot and the place
 // in the split list; the counts {items, slots, splits, T} and the places of the
@@ -160,6 +175,7 @@ struct WorkList {
     unsigned *cost, *item0, *slot0, *sidx;
     unsigned *counts;              // 4
     unsigned *hist;                // 32
+    WorkChunk *chunks;             // work_chunks(units); unused when that is 0
 };
 
 // Boundary-cell hierarchy for exact nearest-boundary distances: leaves of

@@ -1207,7 +1207,12 @@ __global__ __launch_bounds__(256) void k_density_merge(GridDesc g, Tiling tl, in
 // then every unit writes its items and takes their places in the order
 // (k_work_items).  With each of those in a launch of its own a list took 16
 // launches, ~70 us of a small job; one workgroup needs 4 us at 1,000 units and
-// 31 us at 16,384 (66 us with the buckets counted by ballots).
+// 31 us at 16,384 (66 us with the buckets counted by ballots).  Longer lists than
+// MKDE_WS_ONE are scanned by a workgroup per 4096 units, in three launches (totals,
+// counts, scan): rasters of few points, 16,384 / 65,536 / 262,144 / 1,048,576 blocks,
+// 225 / 744 / 2813 / 11080 us by one workgroup, 220 / 667 / 2430 / 9446 us by many
+// (16 launches: 259 / 708 / 2480 / 9496 us); 4,096 blocks 97 and 108 us,
+// and between 6,000 and 16,000 units both are within 13 us.
 #define DT_TMIN 2048u
 #define DT_TARGET 4096ull
 
@@ -1227,48 +1232,132 @@ __device__ __forceinline__ unsigned split_parts(unsigned c, unsigned T)
     return c > T ? (unsigned)(((unsigned long long)c + T - 1) / T) : 1u;
 }
 
-// One workgroup of 1024 threads, four units per thread and step.  host
-// (nullable, pinned): also receives the counts.
+#define WS_UNITS MKDE_WS_UNITS   // units of a step: four per thread
+
+// Sum over the 1024 threads of a workgroup, in all of them (s_t: 16 words).
+__device__ __forceinline__ unsigned long long sum1024(unsigned long long v, unsigned long long *s_t)
+{
+    for (int d = 32; d >= 1; d >>= 1) v += __shfl_xor(v, d, WAVE);
+    __syncthreads();   // s_t of the sum before has been read
+    if ((threadIdx.x & 63) == 0) s_t[threadIdx.x >> 6] = v;
+    __syncthreads();
+    unsigned long long total = 0;
+    for (int w = 0; w < 16; ++w) total += s_t[w];
+    return total;
+}
+
+// Costs and parts of this thread's four units, and the number of items, slots and
+// split units among them.
+struct StepUnits {
+    unsigned c[4], k[4], ni, np, ns;
+};
+__device__ __forceinline__ StepUnits step_units(const unsigned *cost, int b0, int n, unsigned T)
+{
+    StepUnits u;
+    u.ni = u.np = u.ns = 0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        u.c[j] = b0 + j < n ? cost[b0 + j] : 0u;
+        u.k[j] = b0 + j < n ? split_parts(u.c[j], T) : 0u;
+        u.ni += u.k[j];
+        u.np += u.k[j] > 1 ? u.k[j] : 0u;
+        u.ns += u.k[j] > 1 ? 1u : 0u;
+    }
+    return u;
+}
+
+// Total of the chunks' costs -> split threshold.
+__device__ __forceinline__ unsigned chunks_threshold(const WorkList &W, int nchunks, const SplitRule &rule,
+                                                     unsigned long long *s_t)
+{
+    unsigned long long acc = 0;
+    for (int i = threadIdx.x; i < nchunks; i += 1024) acc += W.chunks[i].cost;
+    return split_threshold(sum1024(acc, s_t), rule);
+}
+
+// Long lists, first launch: each chunk's total cost.
+__global__ __launch_bounds__(1024) void k_work_totals(int n, WorkList W)
+{
+    __shared__ unsigned long long s_t[16];
+    const int b0 = (int)blockIdx.x * WS_UNITS + 4 * (int)threadIdx.x;
+    unsigned long long acc = 0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc += b0 + j < n ? W.cost[b0 + j] : 0u;
+    acc = sum1024(acc, s_t);
+    if (threadIdx.x == 0) W.chunks[blockIdx.x].cost = acc;
+}
+
+// Second launch: each chunk's items, slots, split units and bucket sizes.
+__global__ __launch_bounds__(1024) void k_work_counts(int n, SplitRule rule, WorkList W)
+{
+    __shared__ unsigned long long s_t[16];
+    __shared__ unsigned s_h[16][32];
+    const int tid = threadIdx.x, wave = tid >> 6;
+    if (tid < 512) s_h[tid >> 5][tid & 31] = 0;
+    const unsigned T = chunks_threshold(W, (int)gridDim.x, rule, s_t);
+    const StepUnits u = step_units(W.cost, (int)blockIdx.x * WS_UNITS + 4 * tid, n, T);
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+        if (u.k[j]) atomicAdd(&s_h[wave][cost_bucket(u.c[j] / u.k[j])], u.k[j]);
+    const unsigned long long ni = sum1024(u.ni, s_t), np = sum1024(u.np, s_t), ns = sum1024(u.ns, s_t);
+    WorkChunk &ch = W.chunks[blockIdx.x];
+    if (tid == 0) {
+        ch.n[0] = (unsigned)ni;
+        ch.n[1] = (unsigned)np;
+        ch.n[2] = (unsigned)ns;
+    }
+    if (tid < 32) {
+        unsigned h = 0;
+        for (int w = 0; w < 16; ++w) h += s_h[w][tid];
+        ch.hist[tid] = h;
+    }
+}
+
+// One workgroup of 1024 threads, four units per thread and step; MANY: the last
+// launch of a long list, a workgroup per step.  host (nullable, pinned): also
+// receives the counts.
+template <bool MANY>
 __global__ __launch_bounds__(1024) void k_work_scan(int n, SplitRule rule, WorkList W, unsigned *host, const double *extra)
 {
     __shared__ unsigned long long s_t[16];
     __shared__ unsigned s_w[16][3];
     __shared__ unsigned s_h[16][32];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    unsigned long long acc = 0;
-    for (int i = tid; i < n; i += 1024) acc += W.cost[i];
-    for (int d = 32; d >= 1; d >>= 1) acc += __shfl_xor(acc, d, WAVE);
-    if (lane == 0) s_t[wave] = acc;
     if (tid < 512) s_h[tid >> 5][tid & 31] = 0;
-    __syncthreads();
-    unsigned long long total = 0;
-    for (int w = 0; w < 16; ++w) total += s_t[w];
-    const unsigned T = split_threshold(total, rule);
-
+    unsigned T;
     unsigned run_i = 0, run_p = 0, run_s = 0;   // items, slots, splits before this step
-    for (int base = 0; base < n; base += 4096) {
+    unsigned all[3] = {0, 0, 0};                // MANY, first workgroup: of the list
+    if (MANY) {
+        T = chunks_threshold(W, (int)gridDim.x, rule, s_t);
+        const int lim = blockIdx.x ? (int)blockIdx.x : (int)gridDim.x;
+        unsigned long long a[3] = {0, 0, 0};
+        for (int i = tid; i < lim; i += 1024)
+            for (int q = 0; q < 3; ++q) a[q] += W.chunks[i].n[q];
+        for (int q = 0; q < 3; ++q) all[q] = (unsigned)sum1024(a[q], s_t);
+        if (blockIdx.x) {
+            run_i = all[0];
+            run_p = all[1];
+            run_s = all[2];
+        } else {
+            for (int i = tid >> 5; i < (int)gridDim.x; i += 32) atomicAdd(&s_h[wave][tid & 31], W.chunks[i].hist[tid & 31]);
+        }
+    } else {
+        unsigned long long acc = 0;
+        for (int i = tid; i < n; i += 1024) acc += W.cost[i];
+        T = split_threshold(sum1024(acc, s_t), rule);
+    }
+    const int first = MANY ? (int)blockIdx.x * WS_UNITS : 0, end = MANY ? first + 1 : n;
+    for (int base = first; base < end; base += WS_UNITS) {
         const int b0 = base + 4 * tid;
-        unsigned k[4], c[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            c[j] = b0 + j < n ? W.cost[b0 + j] : 0u;
-            k[j] = b0 + j < n ? split_parts(c[j], T) : 0u;
-        }
-        unsigned ni = 0, np = 0, ns = 0;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            ni += k[j];
-            np += k[j] > 1 ? k[j] : 0u;
-            ns += k[j] > 1 ? 1u : 0u;
-        }
-        const unsigned ii = wave_incl_scan(ni, lane), ip = wave_incl_scan(np, lane), is = wave_incl_scan(ns, lane);
+        const StepUnits u = step_units(W.cost, b0, n, T);
+        const unsigned ii = wave_incl_scan(u.ni, lane), ip = wave_incl_scan(u.np, lane), is = wave_incl_scan(u.ns, lane);
         if (lane == WAVE - 1) {
             s_w[wave][0] = ii;
             s_w[wave][1] = ip;
             s_w[wave][2] = is;
         }
         __syncthreads();
-        unsigned oi = run_i + ii - ni, op = run_p + ip - np, os = run_s + is - ns;
+        unsigned oi = run_i + ii - u.ni, op = run_p + ip - u.np, os = run_s + is - u.ns;
         for (int w = 0; w < 16; ++w) {
             const unsigned a0 = s_w[w][0], a1 = s_w[w][1], a2 = s_w[w][2];
             if (w < wave) {
@@ -1284,21 +1373,22 @@ __global__ __launch_bounds__(1024) void k_work_scan(int n, SplitRule rule, WorkL
         for (int j = 0; j < 4; ++j) {
             if (b0 + j >= n) break;
             W.item0[b0 + j] = oi;
-            oi += k[j];
-            if (k[j] > 1) {
+            oi += u.k[j];
+            if (u.k[j] > 1) {
                 W.slot0[b0 + j] = op;
                 W.sidx[b0 + j] = os++;
-                op += k[j];
+                op += u.k[j];
             }
         }
         // bucket sizes, a copy per wave
+        if (!MANY)
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-            if (k[j]) atomicAdd(&s_h[wave][cost_bucket(c[j] / k[j])], k[j]);
+            for (int j = 0; j < 4; ++j)
+                if (u.k[j]) atomicAdd(&s_h[wave][cost_bucket(u.c[j] / u.k[j])], u.k[j]);
         __syncthreads();
     }
-    if (tid == 0) {
-        const unsigned out[4] = {run_i, run_p, run_s, T};
+    if (tid == 0 && (!MANY || blockIdx.x == 0)) {
+        const unsigned out[4] = {MANY ? all[0] : run_i, MANY ? all[1] : run_p, MANY ? all[2] : run_s, T};
         for (int j = 0; j < 4; ++j) {
             W.counts[j] = out[j];
             if (host) host[j] = out[j];
@@ -3575,6 +3665,19 @@ static void scan_u32(hipStream_t s, int n, const unsigned *in, unsigned *out, un
     hipLaunchKernelGGL(k_scan_add, dim3(nblk_(n)), dim3(256), 0, s, n, out, chunks);
 }
 
+// Scans of n units' costs.
+static void work_scan(hipStream_t s, int n, const SplitRule &rule, const WorkList &W, unsigned *host, const double *extra)
+{
+    const unsigned nchunks = (unsigned)work_chunks(n);
+    if (nchunks == 0) {
+        hipLaunchKernelGGL(k_work_scan<false>, dim3(1), dim3(1024), 0, s, n, rule, W, host, extra);
+        return;
+    }
+    hipLaunchKernelGGL(k_work_totals, dim3(nchunks), dim3(1024), 0, s, n, W);
+    hipLaunchKernelGGL(k_work_counts, dim3(nchunks), dim3(1024), 0, s, n, rule, W);
+    hipLaunchKernelGGL(k_work_scan<true>, dim3(nchunks), dim3(1024), 0, s, n, rule, W, host, extra);
+}
+
 // Costs and scans of the density work list; W.counts and, when given, the
 // pinned host words receive {items, slots, splits, T} and, in the next two, the
 // points' reach.
@@ -3585,7 +3688,7 @@ hipError_t density_plan(hipStream_t s, const GridDesc &g, const float *mask, con
     const int nblk = (int)raster_blocks(g, tl);
     hipLaunchKernelGGL(k_block_cost, dim3((unsigned)nblk), dim3(256), 0, s, g, mask, idx, nbx, tl, W.cost);
     const SplitRule rule{DT_TMIN, T.dt_target, 0u, 0ull};
-    hipLaunchKernelGGL(k_work_scan, dim3(1), dim3(1024), 0, s, nblk, rule, W, host, idx.reach_p);
+    work_scan(s, nblk, rule, W, host, idx.reach_p);
     return hipGetLastError();
 }
 
@@ -3655,7 +3758,7 @@ hipError_t point_plan(hipStream_t s, const PointIndex &idx, float h_fixed, const
     const double lim_fixed = !thr_k && h_fixed > 0.0f ? 9.0 * (double)(float)(h_fixed * h_fixed) : 0.0;
     if (idx.grp) hipLaunchKernelGGL(k_fine_cost, dim3((unsigned)((nw + 3) / 4)), dim3(256), 0, s, idx, W.cost);
     else hipLaunchKernelGGL(k_wave_cost, dim3((unsigned)((nw + 3) / 4)), dim3(256), 0, s, idx, lim_fixed, lim_dev, W.cost);
-    hipLaunchKernelGGL(k_work_scan, dim3(1), dim3(1024), 0, s, nw, rule, W, host, (const double *)nullptr);
+    work_scan(s, nw, rule, W, host, nullptr);
     return hipGetLastError();
 }
 
