@@ -145,7 +145,8 @@ int mkde_density_at_points(mkde_ctx *ctx, int loo, float *den);
  * (caller's point order).  The work list, the split partial sums and the
  * bin-order densities live in a static 32 MiB array per device (held until the
  * process ends) instead of context buffers; no hipMalloc / hipFree is called.
- * About 5 million points fit; more return MKDE_E_RANGE before any kernel runs.
+ * About 7 million points fit (where the partial sums of the usual parts do not,
+ * waves are cut into larger parts); more return MKDE_E_RANGE.
  * Every call on one device shares that array: calls that overlap on one GPU
  * (two contexts, two threads) race and must be serialised by the caller. */
 int mkde_density_at_points_noalloc(mkde_ctx *ctx, int loo, float *den_dev);

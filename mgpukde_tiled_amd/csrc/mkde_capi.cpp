@@ -1233,14 +1233,27 @@ extern "C" int mkde_density_at_points_noalloc(mkde_ctx *c, int loo, float *den_d
     CHK(prep(c, fine));
     PointIndex I = index_of(c);
     const WorkList W{cost, item0, slot0, sidx, counts, hist, chunks};
-    HIPCHK(mkde_dev::point_plan(c->stream, I, c->h_fixed, nullptr, 0, mkde_dev::point_rule(loo ? 1 : 0, c->tune, false, !I.grp),
-                                W, c->host_words));
-    HIPCHK(hipStreamSynchronize(c->stream));
-    const unsigned cnt[3] = {c->host_words[0], c->host_words[1], c->host_words[2]};   // items, slots, split waves
-    int4 *items = cv.take<int4>(cnt[0]);
-    int *order = cv.take<int>(cnt[0]);
-    int4 *splits = cv.take<int4>(cnt[2]);
-    double *partials = cv.take<double>((size_t)cnt[1] * 64);
+    // the list at the splits of the allocating call; while that does not fit, at
+    // larger parts, down to one per wave
+    SplitRule rule = mkde_dev::point_rule(loo ? 1 : 0, c->tune, false, !I.grp);
+    const Carve before = cv;
+    unsigned cnt[3];   // items, slots, split waves
+    int4 *items, *splits;
+    int *order;
+    double *partials;
+    for (;;) {
+        HIPCHK(mkde_dev::point_plan(c->stream, I, c->h_fixed, nullptr, 0, rule, W, c->host_words));
+        HIPCHK(hipStreamSynchronize(c->stream));
+        for (int k = 0; k < 3; ++k) cnt[k] = c->host_words[k];
+        cv = before;
+        items = cv.take<int4>(cnt[0]);
+        order = cv.take<int>(cnt[0]);
+        splits = cv.take<int4>(cnt[2]);
+        partials = cv.take<double>((size_t)cnt[1] * 64);
+        const unsigned T = c->host_words[3];
+        if (cv.ok || cnt[1] == 0) break;
+        rule = SplitRule{T < 1u << 30 ? 2 * T : ~0u, rule.target, 0u, 0ull};
+    }
     if (!cv.ok)
         return fail(MKDE_E_RANGE,
                     "the work list of %lld points (%u items, %u split parts) needs %zu bytes of scratch, more than "
