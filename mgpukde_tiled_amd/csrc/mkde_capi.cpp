@@ -487,6 +487,36 @@ static void forget_points(mkde_ctx *c)
     c->pts_dirty = true;
 }
 
+// Bounds of n coordinates, widened from lo and hi; false: one is not finite.
+// Eight at a time and no branch: as one chain with an early exit the loop took 0.40
+// or 0.80 ms for 1M points, depending on the address it was linked at (0.2 ms now).
+static bool finite_bounds(int64_t n, const float *v, float &lo, float &hi)
+{
+    typedef float f8 __attribute__((ext_vector_type(8)));
+    typedef int i8 __attribute__((ext_vector_type(8)));
+    f8 a = lo, b = hi;
+    i8 bad = 0;
+    auto take = [&](f8 t) {
+        a = t < a ? t : a;
+        b = b < t ? t : b;
+        bad |= (__builtin_bit_cast(i8, t) & 0x7f800000) == 0x7f800000;
+    };
+    int64_t i = 0;
+    for (; i + 8 <= n; i += 8) {
+        f8 t;
+        memcpy(&t, v + i, sizeof t);
+        take(t);
+    }
+    for (; i < n; ++i) take(v[i]);
+    int any = 0;
+    for (int j = 0; j < 8; ++j) {
+        lo = std::min(lo, a[j]);
+        hi = std::max(hi, b[j]);
+        any |= bad[j];
+    }
+    return any == 0;
+}
+
 extern "C" int mkde_points_upload(mkde_ctx *c, int64_t n, const float *x, const float *y, const float *w)
 {
     if (!c) return fail(MKDE_E_ARG, "null context");
@@ -495,14 +525,10 @@ extern "C" int mkde_points_upload(mkde_ctx *c, int64_t n, const float *x, const 
     // validate (and take the bounding box) before anything of the context
     // changes: on this error the previous points stay usable
     float x0 = FLT_MAX, x1 = -FLT_MAX, y0 = FLT_MAX, y1 = -FLT_MAX;
-    for (int64_t i = 0; i < n; ++i) {
-        if (!std::isfinite(x[i]) || !std::isfinite(y[i]))
-            return fail(MKDE_E_ARG, "point %lld has a non-finite coordinate", (long long)i);
-        x0 = std::min(x0, x[i]);
-        x1 = std::max(x1, x[i]);
-        y0 = std::min(y0, y[i]);
-        y1 = std::max(y1, y[i]);
-    }
+    if (!(finite_bounds(n, x, x0, x1) & finite_bounds(n, y, y0, y1)))
+        for (int64_t i = 0; i < n; ++i)
+            if (!std::isfinite(x[i]) || !std::isfinite(y[i]))
+                return fail(MKDE_E_ARG, "point %lld has a non-finite coordinate", (long long)i);
     CHK(set_device(c));
     const BinGrid bg = bin_grid(n, x0, x1, y0, y1, c->pts_per_bin);
     const int nbins = bg.nbx * bg.nby;
