@@ -2744,6 +2744,23 @@ __device__ __forceinline__ void leaf_best(const GridDesc &g, const BndTree &T, i
     }
 }
 
+// Of the four children ch of a node, those of `left` that may hold a cell nearer than
+// best: all of them in rest, the nearest in k (-1: none).
+__device__ __forceinline__ void nearest_child(const float4 *ch, unsigned left, float px, float py, double best,
+                                              unsigned &rest, int &k)
+{
+    double lb = best;
+    rest = 0;
+    k = -1;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const double l = (left >> j) & 1u ? node_lb(ch[j], px, py) : DBL_MAX;
+        rest |= l < best ? 1u << j : 0u;
+        k = l < lb ? j : k;
+        lb = l < lb ? l : lb;
+    }
+}
+
 // One step (todo != 0): back to the lowest node with children left, and to the
 // nearest of them; a leaf's cells are taken.
 __device__ __forceinline__ void lane_step(const GridDesc &g, const BndTree &T, double nrm05, float px, float py,
@@ -2754,17 +2771,9 @@ __device__ __forceinline__ void lane_step(const GridDesc &g, const BndTree &T, d
     L.ix >>= up;
     L.iy >>= up;
     const float4 *ch = T.box + T.off[L.lev - 1] + (((int64_t)L.iy * T.nx[L.lev] + L.ix) << 2);
-    const unsigned left = (unsigned)(L.todo >> at) & 15u;
-    unsigned rest = 0;
-    double lb = best;
-    int k = -1;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const double l = (left >> j) & 1u ? node_lb(ch[j], px, py) : DBL_MAX;
-        rest |= l < best ? 1u << j : 0u;
-        k = l < lb ? j : k;
-        lb = l < lb ? l : lb;
-    }
+    unsigned rest;
+    int k;
+    nearest_child(ch, (unsigned)(L.todo >> at) & 15u, px, py, best, rest, k);
     L.todo &= ~((uint64_t)15 << at);
     if (k < 0) return;
     L.todo |= (uint64_t)(rest & ~(1u << k)) << at;
@@ -2788,10 +2797,20 @@ __global__ __launch_bounds__(64) void k_dist_tree(int64_t n, const float *xs, co
     const int top = T.nlev - 1;
     double best = DBL_MAX;
 
-    // 1. (and 3., where the points lie far apart)
-    LaneSearch L{top, 0, 0, on && top > 0 ? (uint64_t)15 << (4 * top - 4) : 0ull};
-    if (top == 0 && on) leaf_best(g, T, 0, 0, nrm05, px, py, best);
-    int steps = top;
+    // 1. down to a leaf, all lanes level by level
+    LaneSearch L{0, 0, 0, 0};
+    bool down = on;
+    for (int lev = top; lev > 0; --lev) {
+        unsigned rest;
+        int k;
+        nearest_child(T.box + T.off[lev - 1] + (((int64_t)L.iy * T.nx[lev] + L.ix) << 2), 15u, px, py, best, rest, k);
+        down = down && k >= 0;
+        if (!down) continue;
+        L.todo |= (uint64_t)(rest & ~(1u << k)) << (4 * lev - 4);
+        L.ix = 2 * L.ix + (k & 1);
+        L.iy = 2 * L.iy + (k >> 1);
+    }
+    if (down) leaf_best(g, T, L.ix, L.iy, nrm05, px, py, best);
     float wx0 = 0.0f, wx1 = 0.0f, wy0 = 0.0f, wy1 = 0.0f;   // box of the open points
     double far = 0.0;   // no node beyond this is needed
     auto wave_far = [&]() {
@@ -2799,23 +2818,21 @@ __global__ __launch_bounds__(64) void k_dist_tree(int64_t n, const float *xs, co
         for (int d = 32; d >= 1; d >>= 1) v = fmax(v, __shfl_xor(v, d, WAVE));
         return v;
     };
-    while (__ballot(L.todo != 0)) {
-        if (steps-- == 0) {
-            wx0 = uni(wave_min(L.todo ? px : FLT_MAX));
-            wx1 = uni(wave_max(L.todo ? px : -FLT_MAX));
-            wy0 = uni(wave_min(L.todo ? py : FLT_MAX));
-            wy1 = uni(wave_max(L.todo ? py : -FLT_MAX));
-            far = wave_far();
-            const double f = sqrt(far), w = (double)wx1 - (double)wx0 + 2.0 * f, h = (double)wy1 - (double)wy0 + 2.0 * f;
-            if (w * h <= BT_WAVE_AREA * far) break;
-        }
-        if (L.todo) lane_step(g, T, nrm05, px, py, L, best);
-    }
 
     // 2. the open ones together
     const bool open = L.todo != 0;
-    if (lane == 0) s_node[0] = (unsigned)top << 28;
-    int sp = __ballot(open) ? 1 : 0, credit = BT_CREDIT;
+    int sp = 0, credit = BT_CREDIT;
+    if (__ballot(open)) {
+        wx0 = uni(wave_min(open ? px : FLT_MAX));
+        wx1 = uni(wave_max(open ? px : -FLT_MAX));
+        wy0 = uni(wave_min(open ? py : FLT_MAX));
+        wy1 = uni(wave_max(open ? py : -FLT_MAX));
+        far = wave_far();
+        const double f = sqrt(far), w = (double)wx1 - (double)wx0 + 2.0 * f, h = (double)wy1 - (double)wy0 + 2.0 * f;
+        if (w * h <= BT_WAVE_AREA * far) sp = 1;
+        if (lane == 0) s_node[0] = (unsigned)top << 28;
+    }
+    const bool together = sp > 0;
     while (sp > 0 && credit >= 0) {
         wave_sync();
         const int room = (BT_STACK_SOFT - sp) / 3;
@@ -2898,7 +2915,7 @@ __global__ __launch_bounds__(64) void k_dist_tree(int64_t n, const float *xs, co
         }
     }
     // 3. all has been seen, or each lane goes on where it was
-    if (sp == 0) L.todo = 0;
+    if (together && sp == 0) L.todo = 0;
     while (__ballot(L.todo != 0))
         if (L.todo) lane_step(g, T, nrm05, px, py, L, best);
     if (on) dist[perm[i]] = best;
