@@ -2692,17 +2692,17 @@ __device__ __forceinline__ double node_lb(float4 b, float px, float py)
 //      at a time are taken without waiting on each other.
 //   3. What is left, where the wave did not search or gave up, every lane finishes
 //      by itself.  The wave gives up when too few points need the leaves it
-//      visits: a leaf costs it BT_COST and pays back one a point.
+//      visits: one that none needs costs it BT_COST, the others pay one a point.
 // What bounds a search is its longest one: points near the centre of a round study
 // area find hundreds of leaves nearly equidistant, and node by node each costs a
 // memory latency, so there the wave takes nodes 64 at a time.  Near a ragged
 // boundary every point needs a few leaves of its own and the wave would look at
-// all leaves around: 64 points on 8192^2 cells with 2% nodata cells 120 us with a
-// stack per lane, 33.8 ms by the wave alone, 77 us now; half the raster like that
-// and half without, 200,000 points 301 / 1863 / 261 us; a coast, 1M points 868 /
-// 1655 / 312 us; a disk with 20 holes, 1M points 1258 / 331 / 380 us; a plain disk
-// on 4096^2, 200,000 points 6.2 / 0.76 / 0.78 ms (times with the flags and the
-// hierarchy, 70 to 150 us).
+// all leaves around: 64 points on 8192^2 cells with 2% nodata cells 119 us with a
+// stack per lane, 33.9 ms by the wave alone, 73 us now; half the raster like that
+// and half without, 200,000 points 305 / 1878 / 250 us; a coast, 1M points 889 /
+// 1662 / 291 us; a disk with 20 holes, 1M points 1270 / 333 / 356 us; a plain disk
+// on 4096^2, 200,000 points 6.2 / 0.77 / 0.77 ms (times with the flags and the
+// hierarchy, 60 to 150 us).
 
 #define BT_STACK 1024
 // Nodes popped at a time are limited so that their children fit below this; at
@@ -2710,9 +2710,10 @@ __device__ __forceinline__ double node_lb(float4 b, float px, float py)
 #define BT_STACK_SOFT (BT_STACK - 64)
 // The wave looks at the leaves within far of the open points' box, a lane at those
 // within far of its point.  Area of the first in far^2 up to which the wave starts,
-// its cost of a leaf, and what it may lose before it gives up.  (Areas of 10 and 25:
-// 64 points on 2048^2 cells without holes 102 and 184 us.  Cost 8 / 2 / 1: the disk's
-// 200,000 points 3.4 / 0.78 / 0.78 ms, the half ragged raster's 200 / 261 / 400 us.)
+// its cost of a leaf that no point needs, and what it may lose before it gives up.
+// (Areas of 10 and 25: 64 points on 2048^2 cells without holes 102 and 184 us.  A cost
+// of 1 instead of 2: the half ragged raster's 200,000 points 434 us, a coast's 1M 381;
+// 2 for every leaf: 307 and 341; twice the credit: 346 and 370 us.)
 #define BT_WAVE_AREA 10.0
 #define BT_COST 2
 #define BT_CREDIT 512
@@ -2814,13 +2815,15 @@ __global__ __launch_bounds__(64) void k_dist_tree(int64_t n, const float *xs, co
     float wx0 = 0.0f, wx1 = 0.0f, wy0 = 0.0f, wy1 = 0.0f;   // box of the open points
     double far = 0.0;   // no node beyond this is needed
     auto wave_far = [&]() {
-        double v = L.todo ? best : 0.0;
+        double v = best;
         for (int d = 32; d >= 1; d >>= 1) v = fmax(v, __shfl_xor(v, d, WAVE));
         return v;
     };
 
     // 2. the open ones together
     const bool open = L.todo != 0;
+    const double closed = best;
+    if (!open) best = -1.0;   // nothing is nearer
     int sp = 0, credit = BT_CREDIT;
     if (__ballot(open)) {
         wx0 = uni(wave_min(open ? px : FLT_MAX));
@@ -2866,8 +2869,8 @@ __global__ __launch_bounds__(64) void k_dist_tree(int64_t n, const float *xs, co
                 auto get = [&](unsigned v) { return (unsigned)__builtin_amdgcn_readlane((int)v, l); };
                 auto getf = [&](float v) { return __uint_as_float(get(__float_as_uint(v))); };
                 const float4 lb = make_float4(getf(own.x), getf(own.y), getf(own.z), getf(own.w));
-                const uint64_t who = __ballot(open && node_lb(lb, px, py) < best);
-                credit += __popcll(who) - BT_COST;
+                const uint64_t who = __ballot(node_lb(lb, px, py) < best);
+                credit += who ? __popcll(who) : -BT_COST;
                 if (!who) continue;
                 const uint64_t m[4] = {get(m0.x) | (uint64_t)get(m0.y) << 32, get(m0.z) | (uint64_t)get(m0.w) << 32,
                                        get(m1.x) | (uint64_t)get(m1.y) << 32, get(m1.z) | (uint64_t)get(m1.w) << 32};
@@ -2915,6 +2918,7 @@ __global__ __launch_bounds__(64) void k_dist_tree(int64_t n, const float *xs, co
         }
     }
     // 3. all has been seen, or each lane goes on where it was
+    if (!open) best = closed;
     if (together && sp == 0) L.todo = 0;
     while (__ballot(L.todo != 0))
         if (L.todo) lane_step(g, T, nrm05, px, py, L, best);
