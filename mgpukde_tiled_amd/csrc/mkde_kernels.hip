@@ -2698,9 +2698,9 @@ __device__ __forceinline__ double node_lb(float4 b, float px, float py)
 // memory latency, so there the wave takes nodes 64 at a time.  Near a ragged
 // boundary every point needs a few leaves of its own and the wave would look at
 // all leaves around: 64 points on 8192^2 cells with 2% nodata cells 119 us with a
-// stack per lane, 33.9 ms by the wave alone, 73 us now; half the raster like that
-// and half without, 200,000 points 305 / 1878 / 250 us; a coast, 1M points 889 /
-// 1662 / 291 us; a disk with 20 holes, 1M points 1270 / 333 / 356 us; a plain disk
+// stack per lane, 33.9 ms by the wave alone, 72 us now; half the raster like that
+// and half without, 200,000 points 305 / 1878 / 292 us; a coast, 1M points 889 /
+// 1662 / 337 us; a disk with 20 holes, 1M points 1270 / 333 / 355 us; a plain disk
 // on 4096^2, 200,000 points 6.2 / 0.77 / 0.77 ms (times with the flags and the
 // hierarchy, 60 to 150 us).
 
@@ -2711,12 +2711,12 @@ __device__ __forceinline__ double node_lb(float4 b, float px, float py)
 // The wave looks at the leaves within far of the open points' box, a lane at those
 // within far of its point.  Area of the first in far^2 up to which the wave starts,
 // its cost of a leaf that no point needs, and what it may lose before it gives up.
-// (Areas of 10 and 25: 64 points on 2048^2 cells without holes 102 and 184 us.  A cost
-// of 1 instead of 2: the half ragged raster's 200,000 points 434 us, a coast's 1M 381;
-// 2 for every leaf: 307 and 341; twice the credit: 346 and 370 us.)
-#define BT_WAVE_AREA 10.0
+// (Area 10: 50,000 points in a disk with 5 holes 89 instead of 68 us, 64 points on 2048^2
+// cells without holes 97 instead of 172.  Credit 512 / 1024 / 2048 at that cost: a disk
+// with 20 holes, 1M points 491 / 355 / 355 us, a coast 294 / 337 / 420.)
+#define BT_WAVE_AREA 20.0
 #define BT_COST 2
-#define BT_CREDIT 512
+#define BT_CREDIT 1024
 
 // A lane's search, depth first: at node (ix, iy) of level lev, with the children
 // that are left at the nodes above in 4 bits a level (level l in bits 4 l - 4 ..
