@@ -74,6 +74,8 @@ int mkde_synchronize(mkde_ctx *ctx);
 /* Device memory held by a context's buffers (bytes; buffers grow to the
  * largest job seen and are reused), and a release of all of them (the
  * context keeps its stream and forgets points, mask, tile and bandwidths).
+ * The release also frees the device's staging memory for large copies (at most
+ * 24 MB pinned and 12 streams, shared by its contexts and kept between them).
  * No reference counterpart: used by the job server's HBM admission. */
 int mkde_ctx_memory(mkde_ctx *ctx, int64_t *bytes);
 int mkde_ctx_release(mkde_ctx *ctx);

@@ -341,7 +341,6 @@ extern "C" int mkde_ctx_create(int device, mkde_ctx **out)
         delete c;
         return fail(MKDE_E_HIP, "context set-up failed: %s", hipGetErrorString(e));
     }
-    mkde_copy::retain();
     *out = c;
     return MKDE_OK;
 }
@@ -365,7 +364,6 @@ extern "C" int mkde_ctx_destroy(mkde_ctx *c)
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
     t_acct = nullptr;
-    mkde_copy::release();
     return MKDE_OK;
 }
 
@@ -410,6 +408,7 @@ extern "C" int mkde_ctx_release(mkde_ctx *c)
     c->tune = tune;
     c->pts_per_bin = ppb;
     t_acct = &c->dev_bytes;
+    mkde_copy::give_back(dev);
     return MKDE_OK;
 }
 
@@ -426,10 +425,7 @@ static int copy_host(mkde_ctx *c, void *dst, const void *src, size_t bytes, bool
 {
     if (bytes == 0) return MKDE_OK;
     bool done = false;
-    const size_t least = c->shared_device ? mkde_copy::MIN_SHARED
-                         : to_host        ? mkde_copy::MIN_TO_HOST
-                                          : mkde_copy::MIN_TO_DEVICE;
-    if (bytes >= least) {
+    if (bytes >= mkde_copy::least(c->shared_device, to_host)) {
         HIPCHK(hipStreamSynchronize(c->stream));
         HIPCHK(mkde_copy::run(c->device, c->shared_device ? c->stream : nullptr, dst, src, bytes, to_host, &done));
     }

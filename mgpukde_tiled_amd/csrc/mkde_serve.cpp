@@ -37,6 +37,7 @@
 #include <vector>
 
 #include "mkde.h"
+#include "mkde_copy.h"
 #include "mkde_device.h"
 
 extern "C" int mkde_internal_fail(int code, const char *msg);
@@ -339,6 +340,7 @@ extern "C" int mkde_server_create(int device, int slots, int64_t hbm_budget, mkd
     if (!s) return sfail(MKDE_E_NOMEM, "out of host memory");
     s->device = device;
     s->budget = hbm_budget;
+    mkde_copy::give_back(device);   // their streams would share the slots' hardware queues
     s->slots.resize(slots);
     for (int i = 0; i < slots; ++i) s->slots[i].th = std::thread(worker, s, i);
     int st;
