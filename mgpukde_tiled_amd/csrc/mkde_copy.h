@@ -6,16 +6,19 @@
 
 namespace mkde_copy {
 
-// Copies below this many bytes go through one hipMemcpyAsync.  To the device the
-// runtime reads the caller's pages in place and needs no staging: lanes win only
-// where several threads' worth of copying is to be had (repeated copies of
-// 8 / 16 / 64 MB: 326 / 617 / 2400 us without, 260 / 455 / 1440 us with lanes, but a
-// single 16 MB mask on a new context 790 against 960 us; a 21 MB tile mask a call,
-// warm, 300 us less with lanes).  From the device: 2 / 4 / 16 / 64 MB 131 / 252 /
-// 1030 / 6750 us without, 127 / 190 / 446 / 1890 us with lanes.
-constexpr size_t MIN_TO_DEVICE = (size_t)20 << 20;
-constexpr size_t MIN_TO_HOST = (size_t)1 << 20;
-// Contexts that share the device with others (the job server's), either way.
+// Copies below this many bytes go through one hipMemcpyAsync.  From the device 1 /
+// 1.5 / 2 / 4 / 16 MB take 73 / 92 / 120 / 244 / 950 us that way into warm pages and
+// 237 / 340 / 475 / 980 / 3900 us into fresh ones, 68 / 82 / 104 / 185 / 545 and 240 /
+// 325 / 450 / 690 / 1230 us with lanes.  To the device the runtime pins the caller's
+// pages in place and keeps them so for a while: 4 / 6 / 8 / 16 / 32 MB out of buffers
+// in turn take 169 / 240 / 315 / 594 / 1164 us, with lanes 168 / 223 / 258 / 463 / 740 us;
+// the same buffer again and again 132 / 189 / 243 / 460 / 1010 us, with lanes 150 / 200 /
+// 250 / 500 / 895 us.
+constexpr size_t MIN_TO_HOST = (size_t)3 << 19;
+constexpr size_t MIN_TO_DEVICE = (size_t)8 << 20;
+// Contexts that share the device with others (the job server's), either way: a burst
+// of 12 jobs on rasters of 4 / 8.6 / 16 / 32 / 64 MB takes 5.4 / 7.6 / 11.5 / 23.9 / 43.4 ms
+// without lanes and 5.8 / 7.6 / 12.0 / 21.7 / 42.0 ms with them.
 constexpr size_t MIN_SHARED = (size_t)32 << 20;
 inline size_t least(bool shared, bool to_host) { return shared ? MIN_SHARED : to_host ? MIN_TO_HOST : MIN_TO_DEVICE; }
 // Lanes are made once such copies on the device have come to this many bytes.
