@@ -134,7 +134,7 @@ int main()
         CHECK(live_streams[dev] == 8);
         for (size_t n : {MIN_TO_HOST, 2 * MB - 1, 2 * MB, 2 * MB + 1, 9 * MB + 77, 17 * MB + 5})
             CHECK(copy(dev, nullptr, n, true, (unsigned)n) == 1);
-        for (size_t n : {MIN_TO_DEVICE, MIN_TO_DEVICE + 1, 20 * MB - 3}) CHECK(copy(dev, nullptr, n, false, (unsigned)n) == 1);
+        for (size_t n : {MIN_TO_DEVICE, MIN_TO_DEVICE + 1, MIN_TO_DEVICE + 3 * MB - 3}) CHECK(copy(dev, nullptr, n, false, (unsigned)n) == 1);
     }
     // on the caller's stream; below its own limit not at all
     Stream *own = new Stream{1};
@@ -159,10 +159,10 @@ int main()
     for (int at = 0; at < 150; ++at) {
         calls = 0;
         fail_at = at;
-        const int r = copy(2, nullptr, 12 * MB + 3, at % 2, at);
+        const int r = copy(2, nullptr, MIN_TO_DEVICE + 3, at % 2, at);
         fail_at = -1;
         (r < 0 ? failed : r ? right : none)++;
-        CHECK(copy(2, nullptr, 12 * MB + 3, at % 2, at) == 1);
+        CHECK(copy(2, nullptr, MIN_TO_DEVICE + 3, at % 2, at) == 1);
         if (at % 7 == 0) give_back(2);
     }
     CHECK(failed > 20 && right > 10);
