@@ -479,8 +479,10 @@ __device__ __forceinline__ BlockGeom block_geom(const GridDesc &g, const Tiling 
 // Chebyshev nodes of the block instead of its 64 x 64 cells, one 16 x 16 x 4 MFMA
 // for four points, and interpolated to the cells once at the end (FP64).  For h >=
 // half extent / (2 DN_KAPPA) (24 cells) the interpolant of a point is within
-// 4.4e-9 of its value anywhere in the block, and the weights of a cell have a root
-// sum of squares of 1, so rounding at the nodes is not amplified.  Per point and
+// 4.4e-9 of its value anywhere in the block.  A cell's weights have a root sum of
+// squares of 1 on average, 1.39 at most in each direction (1.94 in a corner), by
+// which rounding at the nodes can grow; the nodes fold into FP64 every 16 points,
+// and the error against 64 bits came out no larger than at the cells.  Per point and
 // block: 0.25 MFMA of 8 passes, 10 VALU instructions and 1.3 lane permutations,
 // where the cells take 2 MFMA of 16 passes and 30 instructions.  Every wave walks
 // the candidate bins by itself, without barriers, and takes every fourth 64 points.
@@ -1645,8 +1647,8 @@ struct FineItem {
 __device__ __forceinline__ bool fine_item(const PtsArgs &A, FineItem &F)
 {
     const PointIndex &I = A.idx;
-    // the wave index and the work item are wave-uniform: made explicit so the
-    // source records are read with scalar loads
+    // the wave index and the work item are wave-uniform: made explicit so that
+    // item and box are read with scalar loads and the walk's limits are scalars
     const int64_t g = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int64_t units = A.n_items_dev ? (int64_t)*A.n_items_dev : A.order ? (int64_t)A.n_items : (I.n + 63) / 64;
     if (g >= units) return false;
@@ -1753,10 +1755,10 @@ __global__ __launch_bounds__(256) void k_fine_cost(PointIndex I, unsigned *cost)
 
 // The sources taken in whole groups.  Runs before k_point_density_f and
 // leaves an unsplit wave's sum as a pair of floats in den and res, a part's in
-// its slot of the partials.  A kernel of its own: with its moments it takes 4
-// waves per SIMD, while the other sources' scalar loads want 8 to hide behind.
+// its slot of the partials.  A kernel of its own: its moments take 128 registers
+// (4 waves per SIMD), in one kernel they took 164 or spilled.
 // 1M clustered points, adaptive bandwidths, leave-one-out: 8.8 ms pair by pair
-// with an FP64 test each, 0.63 + 3.63 ms now (12.0 ms with both in one kernel).
+// with an FP64 test each, 0.64 + 2.71 ms now (12.0 ms with both in one kernel).
 template <bool LOO>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_group_density_f(PtsArgs A)
 {
